@@ -129,6 +129,52 @@ static const KernelId kP2R2c[5] = {K_hmd_fft_r2c_16, K_hmd_fft_r2c_32, K_hmd_fft
 static const KernelId kP2C2r[5] = {K_hmd_fft_c2r_16, K_hmd_fft_c2r_32, K_hmd_fft_c2r_64,
                                    K_hmd_fft_c2r_128, K_hmd_fft_c2r_256};
 
+// n = n1 n2 with both factors lengths that the mixed two-stage kernels hold in
+// registers, as near the square root as there is (false: no such pair; the
+// Stockham pass takes the line).
+static bool mix_factors(uint32_t n, uint32_t f[2]) {
+  static const uint32_t kLen[] = {16, 15, 12, 10, 9, 8, 6, 5, 4, 3, 2};
+  uint32_t best = 0;
+  for (uint32_t a : kLen)
+    for (uint32_t b : kLen)
+      if (a <= b && a * b == n && a > best) {
+        best = a;
+        f[0] = a;
+        f[1] = b;
+      }
+  return best != 0;
+}
+
+// Launch shapes of the mixed two-stage passes.  Columns: 8 adjacent lines a
+// workgroup (whole 64-byte segments of the mesh) while that gives every CU a
+// workgroup, else 4; the energy partials follow the grid.  Rows: 8 lines or
+// more, up to 32 once every CU has two workgroups.
+static ForceField::FftPass plan_mix_axis(uint32_t n, uint32_t n_outer, uint32_t cols,
+                                         uint32_t num_cus) {
+  ForceField::FftPass ps;
+  if (!mix_factors(n, ps.f)) return ps;
+  ps.mix = true;
+  ps.k = K_hmd_fft_axis_mix;
+  ps.W = (uint64_t)n_outer * ceil_div(cols, 8) >= num_cus ? 8u : 4u;
+  ps.grid = n_outer * ceil_div(cols, ps.W);
+  ps.shmem = 8 * ((size_t)n + (size_t)n * ps.W + (size_t)ps.f[1] * (ps.f[0] | 1u) * ps.W);
+  return ps;
+}
+
+static ForceField::FftPass plan_mix_lines(uint32_t n, uint32_t n_lines, uint32_t num_cus,
+                                          bool r2c) {
+  ForceField::FftPass ps;
+  if (!mix_factors(n, ps.f)) return ps;
+  ps.mix = true;
+  ps.k = r2c ? K_hmd_fft_r2c_mix : K_hmd_fft_c2r_mix;
+  const size_t per_line = 8 * ((n | 1u) + (size_t)ps.f[0] * (ps.f[1] | 1u));
+  const uint32_t fit = (uint32_t)(49152 / per_line);   // 12 lines at n = 240
+  ps.W = std::min(fit, std::max(8u, std::min(32u, n_lines / (2 * num_cus))));
+  ps.grid = ceil_div(n_lines, ps.W);
+  ps.shmem = 8 * (2 * (size_t)n + 1) + ps.W * per_line;
+  return ps;
+}
+
 // Strided axis of length n over n_outer slabs of `cols` adjacent lines:
 // column tiles of width W (stage-1 capacity 2 x 256 / N2, 64 KiB of LDS),
 // at least `target` blocks in all (a few per compute unit).
@@ -538,6 +584,11 @@ void ForceField::plan_fft() {
   pass_c2r = plan_lines(n2 / 2, n0 * n1, target, false);
   pass_b = plan_axis(n1, n0, nch, target);
   pass_a = plan_axis(n0, n1, nch, target, 2);
+  const uint32_t cus = (uint32_t)c.num_cus;
+  if (!pass_r2c.p2) pass_r2c = plan_mix_lines(n2 / 2, n0 * n1, cus, true);
+  if (!pass_c2r.p2) pass_c2r = plan_mix_lines(n2 / 2, n0 * n1, cus, false);
+  if (!pass_b.p2) pass_b = plan_mix_axis(n1, n0, nch, cus);
+  if (!pass_a.p2) pass_a = plan_mix_axis(n0, n1, nch, cus);
   slab = FftSlab{};
   if (n0 == n1 && n1 == n2 && (n0 == 128 || n0 == 64)) {
     const size_t nc = n2 / 2;
@@ -553,7 +604,7 @@ void ForceField::plan_fft() {
   }
   if (slab.on) {
     partial_blocks = n1;
-  } else if (pass_a.p2) {
+  } else if (pass_a.p2 || pass_a.mix) {
     partial_blocks = pass_a.grid;
   } else {
     const uint32_t La = lines_per_block(n0);
@@ -561,13 +612,14 @@ void ForceField::plan_fft() {
   }
   partials.alloc(2 * (size_t)partial_blocks);
   if (pass_a.p2 || slab.on) gv.alloc(2 * (size_t)n0 * n1 * nch, false);
+  if (pass_a.mix && !slab.on) gv64.alloc(2 * (size_t)n0 * n1 * nch, false);
   compute_gv_table();
 }
 
-// (G, vf) influence table of the power-of-two a-axis pass for the current
-// box (rebuilt when the box changes).
+// (G, vf) influence table of the power-of-two and mixed a-axis passes for the
+// current box (rebuilt when the box changes).
 void ForceField::compute_gv_table() {
-  if (pass_a.p2 || slab.on) {
+  if (pass_a.p2 || pass_a.mix || slab.on) {
     const uint32_t n0 = grid[0], n1 = grid[1], n2 = grid[2], nch = n2 / 2 + 1;
     const size_t m_c = (size_t)n0 * n1 * nch;
     FftParams g{};
@@ -577,6 +629,7 @@ void ForceField::compute_gv_table() {
     g.n0 = n0; g.n1 = n1; g.n2 = n2; g.nch = nch;
     g.bfac0 = bfac[0].ptr; g.bfac1 = bfac[1].ptr; g.bfac2 = bfac[2].ptr;
     g.gv = gv.ptr;
+    g.gv64 = pass_a.mix && !slab.on ? gv64.ptr : nullptr;
     launch(c, K_hmd_spme_gv_table, (uint32_t)ceil_div(m_c, (size_t)256), 256, 0, g);
   }
 }
@@ -855,6 +908,7 @@ void ForceField::spme_forces(bool fev) {
   f.n0 = n0; f.n1 = n1; f.n2 = n2; f.nch = nch;
   f.bfac0 = bfac[0].ptr; f.bfac1 = bfac[1].ptr; f.bfac2 = bfac[2].ptr;
   f.gv = gv.ptr;
+  f.gv64 = gv64.ptr;
   auto set_radix = [&](const std::vector<uint32_t>& r) {
     f.n_stages = (uint32_t)r.size();
     for (size_t k = 0; k < r.size(); ++k) f.radix[k] = r[k];
@@ -892,8 +946,8 @@ void ForceField::spme_forces(bool fev) {
     FftParams& r = q;
     r.n_stages = (uint32_t)rad_c.size();
     for (size_t k = 0; k < rad_c.size(); ++k) r.radix[k] = rad_c[k];
-    if (pass_r2c.p2) {
-      q.lines_per_block = pass_r2c.W;
+    if (pass_r2c.p2 || pass_r2c.mix) {
+      pass_r2c.set(q);
       launch(c, pass_r2c.k, pass_r2c.grid, 256, pass_r2c.shmem, q);
     } else {
       launch(c, K_hmd_fft_r2c_c, ceil_div(q.n_lines, q.lines_per_block), 256,
@@ -916,9 +970,9 @@ void ForceField::spme_forces(bool fev) {
   for (size_t k = 0; k < rad_b.size(); ++k) fb.radix[k] = rad_b[k];
   const size_t sh_b = 2 * (size_t)fb.lines_per_block * (n1 + 1) * 8;
   auto launch_b = [&]() {
-    if (pass_b.p2) {
+    if (pass_b.p2 || pass_b.mix) {
       FftParams q = fb;
-      q.lines_per_block = pass_b.W;
+      pass_b.set(q);
       launch(c, pass_b.k, pass_b.grid, 256, pass_b.shmem, q);
     } else {
       launch(c, K_hmd_fft_axis, ceil_div(fb.n_lines, fb.lines_per_block), 256, sh_b, fb);
@@ -941,8 +995,8 @@ void ForceField::spme_forces(bool fev) {
   set_radix(rad_a);
   fa.n_stages = f.n_stages;
   for (int k = 0; k < 8; ++k) fa.radix[k] = f.radix[k];
-  if (pass_a.p2) {
-    fa.lines_per_block = pass_a.W;
+  if (pass_a.p2 || pass_a.mix) {
+    pass_a.set(fa);
     launch(c, pass_a.k, pass_a.grid, 256, pass_a.shmem, fa);   // data + (G, vf) tiles
   } else {
     launch(c, K_hmd_fft_axis, ceil_div(fa.n_lines, fa.lines_per_block), 256,
@@ -963,8 +1017,8 @@ void ForceField::spme_forces(bool fev) {
     q.sign = +1;
     q.n_stages = (uint32_t)rad_c.size();
     for (size_t k = 0; k < rad_c.size(); ++k) q.radix[k] = rad_c[k];
-    if (pass_c2r.p2) {
-      q.lines_per_block = pass_c2r.W;
+    if (pass_c2r.p2 || pass_c2r.mix) {
+      pass_c2r.set(q);
       launch(c, pass_c2r.k, pass_c2r.grid, 256, pass_c2r.shmem, q);
     } else {
       launch(c, K_hmd_fft_c2r_c, ceil_div(q.n_lines, q.lines_per_block), 256,

@@ -123,16 +123,26 @@ struct ForceField {
   DevBuf<float> rho, V, mesh_c, tw_a, tw_b, tw_c, tw_r2c, u_self;
   DevBuf<double> bfac[3];
   DevBuf<float> gv;            // float2 (G, vf) per complex mesh point (p2 a-axis pass)
+  DevBuf<double> gv64;         // double2 (G, vf), mixed a-axis pass
   DevBuf<float> slow_f, slow_e, slow_w;
   DevBuf<double> partials, spme_out;
   std::vector<uint32_t> rad_a, rad_b, rad_c;
-  // Launch shape of one FFT pass: compile-time power-of-two kernel (p2) or
-  // the generic mixed-radix one.
+  // Launch shape of one FFT pass: compile-time power-of-two kernel (p2), the
+  // two-stage kernel of factors f (mix) or, where neither takes the length,
+  // the mixed-radix Stockham one.
   struct FftPass {
-    bool p2 = false;
+    bool p2 = false, mix = false;
     KernelId k = K_COUNT;
     uint32_t W = 0, grid = 0;
+    uint32_t f[2] = {0, 0};
     size_t shmem = 0;
+    void set(FftParams& q) const {
+      q.lines_per_block = W;
+      if (mix) {
+        q.radix[0] = f[0];
+        q.radix[1] = f[1];
+      }
+    }
   };
   FftPass pass_r2c, pass_c2r, pass_b, pass_a;
   // Slab path (128^3 and 64^3 meshes): three kernels in place of the five

@@ -212,7 +212,8 @@ __device__ inline void hmd_influence(const FftParams& p, uint32_t ka, uint32_t k
 }
 
 // Influence table: (G, vf) of every complex mesh point, evaluated in FP64 and
-// rounded once to f32, in the layout of the complex mesh.  The box is fixed
+// (power-of-two a axes) rounded once to f32, in the layout of the complex
+// mesh.  The box is fixed
 // for the life of a force field, so the a-axis pass reads this table instead
 // of evaluating exp per point every step.
 __device__ __forceinline__ void hmd_spme_gv_table_body(const FftParams& p, const uint32_t hmd_bx,
@@ -225,7 +226,10 @@ __device__ __forceinline__ void hmd_spme_gv_table_body(const FftParams& p, const
   const uint32_t ka = (uint32_t)(i / ((size_t)p.nch * p.n1));
   double G, vf;
   hmd_influence(p, ka, kb, kc, p.bfac0[ka] * p.bfac1[kb] * p.bfac2[kc], G, vf);
-  reinterpret_cast<float2*>(const_cast<float*>(p.gv))[i] = make_float2((float)G, (float)vf);
+  if (p.gv64)
+    reinterpret_cast<double2*>(const_cast<double*>(p.gv64))[i] = make_double2(G, vf);
+  else
+    reinterpret_cast<float2*>(const_cast<float*>(p.gv))[i] = make_float2((float)G, (float)vf);
 }
 HMD_KERNEL(hmd_spme_gv_table, FftParams, 256)
 
@@ -921,3 +925,395 @@ __device__ inline void hmd_fft_slab_inv(const FftParams& p, const uint32_t hmd_b
   HMD_KERNEL(hmd_fft_slab_inv_##TAG, FftParams, 1024)
 HMD_FFT_SLAB(128, 16, 8, 16, 8, 8, 8)
 HMD_FFT_SLAB(64, 8, 8, 8, 8, 8, 4)
+
+// ---------------------------------------------------------------------------
+// Line lengths n = n1 n2 with both factors among 2, 3, 4, 5, 6, 8, 9, 10, 12,
+// 15, 16 (every 2-3-5-smooth mesh length in use that is not a power of two:
+// 18 ... 150 and their halves): the two-stage transform above with the factors
+// chosen at run time.  Each stage is a switch over register DFTs of fixed
+// length, so a line is two LDS round trips and one twiddle per point, where
+// the Stockham pass below takes one round trip, a twiddle from memory and two
+// integer divisions per radix (4, 2, 3, 5) and evaluates the influence
+// function (an FP64 exp) at every point of every step; here it is a table.
+// Bound by latency: a workgroup of a small mesh runs a handful of butterflies
+// a thread, so what counts is the number of dependent LDS and L2 round trips.
+// A step of the 648-atom box (24^3) went from 200 to 157 us, of 4,503 atoms
+// (40^3) from 315 to 242 us, of 39,993 atoms (80^3) from 314 to 230 us.
+// One direction is compiled: the inverse conjugates on the way in and out.
+// cos and sin of 2 pi k / R.
+template <int R> struct HmdRoots;
+template <> struct HmdRoots<6> {
+  static __device__ float C(int k) {
+    const float t[6] = {
+        1.0f, 0.5f, -0.5f, -1.0f, -0.5f, 0.5f};
+    return t[k];
+  }
+  static __device__ float S(int k) {
+    const float t[6] = {
+        0.0f, 0.866025403784439f, 0.866025403784439f, 0.0f, -0.866025403784438f,
+        -0.866025403784439f};
+    return t[k];
+  }
+};
+template <> struct HmdRoots<9> {
+  static __device__ float C(int k) {
+    const float t[9] = {
+        1.0f, 0.766044443118978f, 0.173648177666930f, -0.5f, -0.939692620785908f,
+        -0.939692620785908f, -0.5f, 0.173648177666930f, 0.766044443118978f};
+    return t[k];
+  }
+  static __device__ float S(int k) {
+    const float t[9] = {
+        0.0f, 0.642787609686539f, 0.984807753012208f, 0.866025403784439f, 0.342020143325669f,
+        -0.342020143325669f, -0.866025403784438f, -0.984807753012208f, -0.642787609686540f};
+    return t[k];
+  }
+};
+template <> struct HmdRoots<10> {
+  static __device__ float C(int k) {
+    const float t[10] = {
+        1.0f, 0.809016994374947f, 0.309016994374947f, -0.309016994374947f, -0.809016994374947f,
+        -1.0f, -0.809016994374948f, -0.309016994374948f, 0.309016994374947f, 0.809016994374947f};
+    return t[k];
+  }
+  static __device__ float S(int k) {
+    const float t[10] = {
+        0.0f, 0.587785252292473f, 0.951056516295154f, 0.951056516295154f, 0.587785252292473f,
+        0.0f, -0.587785252292473f, -0.951056516295154f, -0.951056516295154f, -0.587785252292473f};
+    return t[k];
+  }
+};
+template <> struct HmdRoots<12> {
+  static __device__ float C(int k) {
+    const float t[12] = {
+        1.0f, 0.866025403784439f, 0.5f, 0.0f, -0.5f, -0.866025403784439f, -1.0f,
+        -0.866025403784439f, -0.5f, 0.0f, 0.5f, 0.866025403784438f};
+    return t[k];
+  }
+  static __device__ float S(int k) {
+    const float t[12] = {
+        0.0f, 0.5f, 0.866025403784439f, 1.0f, 0.866025403784439f, 0.5f, 0.0f, -0.5f,
+        -0.866025403784438f, -1.0f, -0.866025403784439f, -0.5f};
+    return t[k];
+  }
+};
+template <> struct HmdRoots<15> {
+  static __device__ float C(int k) {
+    const float t[15] = {
+        1.0f, 0.913545457642601f, 0.669130606358858f, 0.309016994374947f, -0.104528463267653f,
+        -0.5f, -0.809016994374947f, -0.978147600733806f, -0.978147600733806f,
+        -0.809016994374948f, -0.5f, -0.104528463267654f, 0.309016994374947f, 0.669130606358858f,
+        0.913545457642601f};
+    return t[k];
+  }
+  static __device__ float S(int k) {
+    const float t[15] = {
+        0.0f, 0.406736643075800f, 0.743144825477394f, 0.951056516295154f, 0.994521895368273f,
+        0.866025403784439f, 0.587785252292473f, 0.207911690817759f, -0.207911690817759f,
+        -0.587785252292473f, -0.866025403784438f, -0.994521895368273f, -0.951056516295154f,
+        -0.743144825477394f, -0.406736643075800f};
+    return t[k];
+  }
+};
+
+__device__ inline void hmd_dft2(float2* v) {
+  const float2 a = v[0], b = v[1];
+  v[0] = cadd(a, b);
+  v[1] = csub(a, b);
+}
+
+// Forward DFT of A B points in registers: B DFTs of length A, the twiddles,
+// A DFTs of length B.
+template <int R>
+__device__ inline void hmd_dft_fwd(float2* v);
+
+template <int A, int B>
+__device__ inline void hmd_dft_ab(float2* v) {
+  constexpr int R = A * B;
+  float2 t[B][A];
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+#pragma unroll
+    for (int a = 0; a < A; ++a) t[b][a] = v[B * a + b];
+    hmd_dft_fwd<A>(t[b]);
+#pragma unroll
+    for (int k = 1; k < A; ++k)
+      if (b > 0)
+        t[b][k] = cmul(t[b][k], make_float2(HmdRoots<R>::C((b * k) % R),
+                                            -HmdRoots<R>::S((b * k) % R)));
+  }
+#pragma unroll
+  for (int k = 0; k < A; ++k) {
+    float2 u[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) u[b] = t[b][k];
+    hmd_dft_fwd<B>(u);
+#pragma unroll
+    for (int q = 0; q < B; ++q) v[k + A * q] = u[q];
+  }
+}
+
+template <int R>
+__device__ inline void hmd_dft_fwd(float2* v) {
+  if constexpr (R == 2) hmd_dft2(v);
+  else if constexpr (R == 3 || R == 5) hmd_dft(v, (uint32_t)R, -1);
+  else if constexpr (R == 4) hmd_dft4<-1>(v);
+  else if constexpr (R == 8) hmd_dft8<-1>(v);
+  else if constexpr (R == 16) hmd_dft16<-1>(v);
+  else if constexpr (R == 6) hmd_dft_ab<2, 3>(v);
+  else if constexpr (R == 9) hmd_dft_ab<3, 3>(v);
+  else if constexpr (R == 10) hmd_dft_ab<2, 5>(v);
+  else if constexpr (R == 12) hmd_dft_ab<4, 3>(v);
+  else hmd_dft_ab<3, 5>(v);
+}
+
+// t / d and t % d for t = t0, t0 + step, ...: one division, then carries.
+struct HmdSplit {
+  uint32_t q, r, d, dq, dr;
+  __device__ inline HmdSplit(uint32_t t0, uint32_t step, uint32_t div)
+      : q(t0 / div), r(t0 % div), d(div), dq(step / div), dr(step % div) {}
+  __device__ inline void next() {
+    q += dq;
+    r += dr;
+    if (r >= d) { r -= d; ++q; }
+  }
+};
+
+// Layout of W lines in LDS.  Rows (c axis): line w holds its points in a row
+// of A (stride n | 1) and of B (n1 rows of n2 | 1); columns (a and b axes):
+// point k of line w at k W + w, B with n1 | 1 rows of W per stage-1 task, so
+// that the strided side of each stage falls on different banks.
+struct HmdMixTile {
+  uint32_t n1, n2, W;
+  uint32_t ea, la;         // A: point and line strides
+  uint32_t bm, bk, lb;     // B: strides of the stage-1 task, its output and the line
+  bool rows;
+};
+
+__device__ inline HmdMixTile hmd_mix_rows(uint32_t n1, uint32_t n2, uint32_t W) {
+  return HmdMixTile{n1, n2, W, 1u, (n1 * n2) | 1u, 1u, n2 | 1u, n1 * (n2 | 1u), true};
+}
+__device__ inline HmdMixTile hmd_mix_cols(uint32_t n1, uint32_t n2, uint32_t W) {
+  return HmdMixTile{n1, n2, W, W, 1u, (n1 | 1u) * W, W, 1u, false};
+}
+
+// Stage 1: for every line and m < n2, the n1-point DFT over points
+// n2 j + m, times e^{-2 pi i m k / n}.
+template <int R>
+__device__ inline void hmd_mix_stage1(const HmdMixTile& L, const float2* A, float2* B,
+                                      const float2* tw, float conj) {
+  HmdSplit s(threadIdx.x, blockDim.x, L.rows ? L.n2 : L.W);
+  for (uint32_t t = threadIdx.x; t < L.W * L.n2; t += blockDim.x, s.next()) {
+    const uint32_t w = L.rows ? s.q : s.r, m = L.rows ? s.r : s.q;
+    float2 v[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      v[j] = A[(L.n2 * (uint32_t)j + m) * L.ea + w * L.la];
+      v[j].y *= conj;
+    }
+    hmd_dft_fwd<R>(v);
+    float2* out = B + m * L.bm + w * L.lb;
+    out[0] = v[0];
+#pragma unroll
+    for (int k = 1; k < R; ++k) out[(uint32_t)k * L.bk] = cmul(v[k], tw[m * (uint32_t)k]);
+  }
+}
+
+// Stage 2: for every line and k1 < n1, the n2-point DFT over m, to points
+// k1 + n1 k2.
+template <int R>
+__device__ inline void hmd_mix_stage2(const HmdMixTile& L, const float2* B, float2* A,
+                                      float conj) {
+  HmdSplit s(threadIdx.x, blockDim.x, L.rows ? L.n1 : L.W);
+  for (uint32_t t = threadIdx.x; t < L.W * L.n1; t += blockDim.x, s.next()) {
+    const uint32_t w = L.rows ? s.q : s.r, k1 = L.rows ? s.r : s.q;
+    float2 u[R];
+    const float2* in = B + k1 * L.bk + w * L.lb;
+#pragma unroll
+    for (int m = 0; m < R; ++m) u[m] = in[(uint32_t)m * L.bm];
+    hmd_dft_fwd<R>(u);
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      u[k].y *= conj;
+      A[(k1 + L.n1 * (uint32_t)k) * L.ea + w * L.la] = u[k];
+    }
+  }
+}
+
+#define HMD_MIX_SWITCH(R, CALL)     \
+  switch (R) {                      \
+    case 2: CALL(2); break;         \
+    case 3: CALL(3); break;         \
+    case 4: CALL(4); break;         \
+    case 5: CALL(5); break;         \
+    case 6: CALL(6); break;         \
+    case 8: CALL(8); break;         \
+    case 9: CALL(9); break;         \
+    case 10: CALL(10); break;       \
+    case 12: CALL(12); break;       \
+    case 15: CALL(15); break;       \
+    default: CALL(16); break;       \
+  }
+
+// The W lines of A transformed in place through B; starts after a barrier
+// and ends with one.
+__device__ inline void hmd_mix_fft(const HmdMixTile& L, float2* A, float2* B, const float2* tw,
+                                   int sign) {
+  const float conj = sign < 0 ? 1.0f : -1.0f;
+#define HMD_MIX_CALL(R) hmd_mix_stage1<R>(L, A, B, tw, conj)
+  HMD_MIX_SWITCH(L.n1, HMD_MIX_CALL)
+#undef HMD_MIX_CALL
+  __syncthreads();
+#define HMD_MIX_CALL(R) hmd_mix_stage2<R>(L, B, A, conj)
+  HMD_MIX_SWITCH(L.n2, HMD_MIX_CALL)
+#undef HMD_MIX_CALL
+  __syncthreads();
+}
+
+// Passes 2-4.  One workgroup takes W adjacent columns (W a power of two) of
+// one slab.  The influence table (FP64, as the factors were evaluated in the
+// pass before) is fetched ahead of the forward transform, HMD_MIX_GV points a
+// thread, the rest at their use.
+#define HMD_MIX_GV 4
+__device__ __forceinline__ void hmd_fft_axis_mix_body(const FftParams& p, const uint32_t hmd_bx,
+    const uint32_t hmd_gx) {
+  extern __shared__ float2 s_buf[];
+  __shared__ double s_w[2][HMD_FFT_THREADS / HMD_WAVE];
+  const uint32_t n = p.n, W = p.lines_per_block, sh = (uint32_t)__builtin_ctz(W);
+  const HmdMixTile L = hmd_mix_cols(p.radix[0], p.radix[1], W);
+  float2* tw = s_buf;
+  float2* A = tw + n;
+  float2* B = A + n * W;
+  for (uint32_t k = threadIdx.x; k < n; k += blockDim.x)
+    tw[k] = reinterpret_cast<const float2*>(p.twiddle)[k];
+  const uint32_t n_tiles = (p.line_minor + W - 1) >> sh;
+  const uint32_t outer = hmd_bx / n_tiles;
+  const uint32_t c0 = (hmd_bx - outer * n_tiles) << sh;
+  const uint32_t Wc = min(W, p.line_minor - c0);
+  float2* data = reinterpret_cast<float2*>(p.data);
+  const size_t base = (size_t)outer * p.major_stride + c0;
+  const uint32_t total = n << sh;
+  const auto at = [&](uint32_t t) {
+    return base + (size_t)(t >> sh) * p.elem_stride + (t & (W - 1u));
+  };
+  hmd_fill_tile(
+      A, total,
+      [&](uint32_t t) { return ((t & (W - 1u)) < Wc) ? data[at(t)] : make_float2(0.0f, 0.0f); },
+      [](uint32_t t) { return t; });
+  const double2* gv = reinterpret_cast<const double2*>(p.gv64);
+  double2 g[HMD_MIX_GV];
+  if (p.apply_influence) {
+#pragma unroll
+    for (int u = 0; u < HMD_MIX_GV; ++u) {
+      const uint32_t t = threadIdx.x + (uint32_t)u * blockDim.x;
+      g[u] = (t < total && (t & (W - 1u)) < Wc) ? gv[at(t)] : make_double2(0.0, 0.0);
+    }
+  }
+  __syncthreads();
+  hmd_mix_fft(L, A, B, tw, p.sign);
+  if (p.apply_influence) {
+    double vir = 0.0, ene = 0.0;
+    const auto solve = [&](uint32_t t, double2 G) {
+      const uint32_t kc = c0 + (t & (W - 1u));
+      const float2 x = A[t];
+      const double hw = (kc == 0u || (p.n2 % 2u == 0u && 2u * kc == p.n2)) ? 1.0 : 2.0;
+      const double r2 = (double)x.x * x.x + (double)x.y * x.y;
+      vir += hw * G.y * r2;
+      ene += hw * G.x * r2;
+      const float Gf = (float)G.x;
+      A[t] = make_float2(Gf * x.x, Gf * x.y);
+    };
+#pragma unroll
+    for (int u = 0; u < HMD_MIX_GV; ++u) {
+      const uint32_t t = threadIdx.x + (uint32_t)u * blockDim.x;
+      if (t < total && (t & (W - 1u)) < Wc) solve(t, g[u]);
+    }
+    for (uint32_t t = threadIdx.x + HMD_MIX_GV * blockDim.x; t < total; t += blockDim.x)
+      if ((t & (W - 1u)) < Wc) solve(t, gv[at(t)]);
+    const double vs = hmd_block_sum_fixed(vir, s_w[0]);
+    const double es = hmd_block_sum_fixed(ene, s_w[1]);   // ends with a barrier
+    if (threadIdx.x == 0) {
+      p.partials[2 * hmd_bx] = vs;
+      p.partials[2 * hmd_bx + 1] = es;
+    }
+    hmd_mix_fft(L, A, B, tw, +1);
+  }
+  for (uint32_t t = threadIdx.x; t < total; t += blockDim.x)
+    if ((t & (W - 1u)) < Wc) data[at(t)] = A[t];
+}
+HMD_KERNEL(hmd_fft_axis_mix, FftParams, 256)
+
+// Pass 1: W real lines of n2 = 2n points as n complex points each.
+__device__ __forceinline__ void hmd_fft_r2c_mix_body(const FftParams& p, const uint32_t hmd_bx,
+    const uint32_t hmd_gx) {
+  extern __shared__ float2 s_buf[];
+  const uint32_t n = p.n, nch = n + 1, W = p.lines_per_block;
+  const uint32_t l0 = hmd_bx * W;
+  const uint32_t Wc = min(W, p.n_lines - l0);
+  const HmdMixTile L = hmd_mix_rows(p.radix[0], p.radix[1], Wc);
+  float2* tw = s_buf;
+  float2* wr = tw + n;
+  float2* A = wr + nch;
+  float2* B = A + W * L.la;
+  const float2* in = reinterpret_cast<const float2*>(p.data) + (size_t)l0 * n;
+  {
+    HmdSplit s(threadIdx.x, blockDim.x, n);
+    for (uint32_t t = threadIdx.x; t < Wc * n; t += blockDim.x, s.next())
+      A[s.q * L.la + s.r] = in[t];   // lines are contiguous
+  }
+  for (uint32_t k = threadIdx.x; k < n; k += blockDim.x)
+    tw[k] = reinterpret_cast<const float2*>(p.twiddle)[k];
+  for (uint32_t k = threadIdx.x; k < nch; k += blockDim.x)
+    wr[k] = reinterpret_cast<const float2*>(p.twiddle_r2c)[k];
+  __syncthreads();
+  hmd_mix_fft(L, A, B, tw, -1);
+  float2* out = reinterpret_cast<float2*>(p.out) + (size_t)l0 * nch;
+  HmdSplit s(threadIdx.x, blockDim.x, nch);
+  for (uint32_t t = threadIdx.x; t < Wc * nch; t += blockDim.x, s.next()) {
+    const float2* z = A + s.q * L.la;
+    const uint32_t m = s.r;
+    const float2 zk = z[m == n ? 0u : m];
+    const float2 zc = cconj(z[m == 0u ? 0u : n - m]);
+    const float2 e = make_float2(0.5f * (zk.x + zc.x), 0.5f * (zk.y + zc.y));
+    const float2 o = cmul_si(make_float2(0.5f * (zk.x - zc.x), 0.5f * (zk.y - zc.y)), -1);
+    out[t] = cadd(e, cmul(wr[m], o));
+  }
+}
+HMD_KERNEL(hmd_fft_r2c_mix, FftParams, 256)
+
+// Pass 5 (unnormalised complex -> real).
+__device__ __forceinline__ void hmd_fft_c2r_mix_body(const FftParams& p, const uint32_t hmd_bx,
+    const uint32_t hmd_gx) {
+  extern __shared__ float2 s_buf[];
+  const uint32_t n = p.n, nch = n + 1, W = p.lines_per_block;
+  const uint32_t l0 = hmd_bx * W;
+  const uint32_t Wc = min(W, p.n_lines - l0);
+  const HmdMixTile L = hmd_mix_rows(p.radix[0], p.radix[1], Wc);
+  float2* tw = s_buf;
+  float2* wr = tw + n;
+  float2* A = wr + nch;
+  float2* B = A + W * L.la;
+  for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) {
+    tw[k] = reinterpret_cast<const float2*>(p.twiddle)[k];
+    wr[k] = reinterpret_cast<const float2*>(p.twiddle_r2c)[k];
+  }
+  __syncthreads();
+  const float2* in = reinterpret_cast<const float2*>(p.data) + (size_t)l0 * nch;
+  {
+    HmdSplit s(threadIdx.x, blockDim.x, n);
+    for (uint32_t t = threadIdx.x; t < Wc * n; t += blockDim.x, s.next()) {
+      const float2* x = in + (size_t)s.q * nch;
+      const float2 xk = x[s.r], xc = cconj(x[n - s.r]);
+      const float2 ee = cadd(xk, xc);
+      const float2 oo = cmul(csub(xk, xc), cconj(wr[s.r]));
+      A[s.q * L.la + s.r] = cadd(ee, cmul_si(oo, +1));
+    }
+  }
+  __syncthreads();
+  hmd_mix_fft(L, A, B, tw, +1);
+  float2* out = reinterpret_cast<float2*>(p.out) + (size_t)l0 * n;
+  HmdSplit s(threadIdx.x, blockDim.x, n);
+  for (uint32_t t = threadIdx.x; t < Wc * n; t += blockDim.x, s.next())
+    out[t] = A[s.q * L.la + s.r];
+}
+HMD_KERNEL(hmd_fft_c2r_mix, FftParams, 256)

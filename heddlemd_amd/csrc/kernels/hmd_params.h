@@ -355,6 +355,7 @@ struct FftParams {
   const double* bfac2;
   double* partials;            // [grid blocks][2]: virial, energy
   const float* gv;             // float2[n0][n1][nch]: (G, vf) in f32, or null
+  const double* gv64;          // double2[n0][n1][nch]: (G, vf), or null
 };
 
 struct SpmeReduceParams {

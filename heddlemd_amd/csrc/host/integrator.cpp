@@ -358,6 +358,8 @@ struct Integrator {
     sp.lan = lan(dt);
     sp.free_atoms = n_groups ? free_atoms.ptr : nullptr;
     sp.n_free = n_free;
+    sp.groups_per_block = n_groups <= 4096 ? 16u : 64u;
+    sp.group_blocks = ceil_div(n_groups, sp.groups_per_block);
     sp.dt = dt;
     sp.counter = kind == Kind::LangevinBaoab ? step_counter.ptr : nullptr;
     // the first fused kernel runs the force field's skin check
@@ -389,16 +391,20 @@ struct Integrator {
     const uint32_t nb = ceil_div(p.n, 256);
     if (fused) {
       const StepParams sp = fused_params();
-      const uint32_t nu = ceil_div((uint64_t)n_groups + n_free, 256);
-      launch(c, kind == Kind::VelocityVerlet ? K_hmd_step_vv_first : K_hmd_step_baoa, nu, 256,
-             0, sp);
+      // workgroups of one wave, a thread a group or free atom; the Langevin
+      // kernel draws a workgroup's normals with 256 threads
+      const uint32_t nu = ceil_div((uint64_t)n_groups + n_free, 64);
+      if (kind == Kind::VelocityVerlet)
+        launch(c, K_hmd_step_vv_first, nu, 64, 0, sp);
+      else
+        launch(c, K_hmd_step_baoa, sp.group_blocks + ceil_div(n_free, 256), 256, 0, sp);
       c.mark(kind == Kind::VelocityVerlet ? "kick_drift_settle" : "baoa");
       ff->compute(level(), true);
       if (csvr || baro) {
         post_force_tail(nb);
         return;
       }
-      launch(c, K_hmd_step_kick_last, nu, 256, 0, sp);
+      launch(c, K_hmd_step_kick_last, nu, 64, 0, sp);
       c.mark("kick_settle");
       return;
     }

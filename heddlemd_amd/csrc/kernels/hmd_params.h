@@ -417,6 +417,8 @@ struct StepParams {
   LangevinParams lan;
   const uint32_t* free_atoms;  // [n_free]; null: atoms 0..n_free-1
   uint32_t n_free;
+  uint32_t groups_per_block;   // hmd_step_baoa: groups a workgroup takes (<= 64)
+  uint32_t group_blocks;       // and the workgroups that take groups
   float dt;
   unsigned long long* counter; // Langevin draw counter (null for VV)
   NblDispParams disp;          // the force field's skin check on the new

@@ -16,66 +16,131 @@
 // f64 position sum.  Written with explicit fmaf / fma so the rounding does
 // not depend on the compiler's contraction choices.
 
-// v += F/m dt/2; x += v dt; wrap + image count (integrate.cu:24-170).
-__device__ inline void hmd_vv_kick_drift_atom(const VvParams& p, const uint32_t i) {
-#pragma clang fp contract(off)
-  const float m = p.m[i];
-  const float half_dt = p.dt * 0.5f;
-  float4 pq = reinterpret_cast<float4*>(p.posq)[i];
-  float a[3] = {p.f[i] / m, p.f[p.n + i] / m, p.f[2 * p.n + i] / m};
-  float x[3] = {pq.x, pq.y, pq.z};
-  if (p.compensated) {
+// The state of one atom in registers.  Every sub-step below works on it, so
+// that the kernels of one sub-step (load, sub-step, store) and the fused step
+// kernels (load once, all sub-steps, store once) run the same operations.
+struct HmdAtom {
+  float4 pq;
+  float v[3];
+  double xl[3], vl[3];   // low parts (compensated mode)
+  int im[3];             // image counts added by the wraps
+};
+
+__device__ inline void hmd_load_pos(const float* posq, const double* lo, uint32_t n, uint32_t i,
+                                    HmdAtom& s) {
+  s.pq = reinterpret_cast<const float4*>(posq)[i];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const size_t k = (size_t)d * p.n + i;
-      double ext_v = ((double)p.v[k] + p.vel_lo[k]) + (double)(a[d] * half_dt);
-      float vh = (float)ext_v;
-      double vl = ext_v - (double)vh;
-      p.v[k] = vh;
-      p.vel_lo[k] = vl;
-      double ext_x = fma((double)vh + vl, (double)p.dt, (double)x[d] + p.pos_lo[k]);
-      float xh = (float)ext_x;
-      p.pos_lo[k] = ext_x - (double)xh;
-      x[d] = xh;
-    }
-  } else {
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const size_t k = (size_t)d * p.n + i;
-      float v = fmaf(a[d], half_dt, p.v[k]);
-      p.v[k] = v;
-      x[d] = fmaf(v, p.dt, x[d]);
-    }
+  for (int d = 0; d < 3; ++d) {
+    s.xl[d] = lo ? lo[(size_t)d * n + i] : 0.0;
+    s.im[d] = 0;
   }
-  int ka, kb, kc;
-  hmd_wrap(x[0], x[1], x[2], ka, kb, kc, p.L);
-  p.images[i] += ka;
-  p.images[p.n + i] += kb;
-  p.images[2 * p.n + i] += kc;
-  pq.x = x[0];
-  pq.y = x[1];
-  pq.z = x[2];
-  reinterpret_cast<float4*>(p.posq)[i] = pq;
+}
+__device__ inline void hmd_load_vel(const float* v, const double* lo, uint32_t n, uint32_t i,
+                                    HmdAtom& s) {
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    s.v[d] = v[(size_t)d * n + i];
+    s.vl[d] = lo ? lo[(size_t)d * n + i] : 0.0;
+  }
+}
+__device__ inline void hmd_store_pos(float* posq, double* lo, uint32_t n, uint32_t i,
+                                     const HmdAtom& s) {
+  reinterpret_cast<float4*>(posq)[i] = s.pq;
+  if (lo) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) lo[(size_t)d * n + i] = s.xl[d];
+  }
+}
+__device__ inline void hmd_store_vel(float* v, double* lo, uint32_t n, uint32_t i,
+                                     const HmdAtom& s) {
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    v[(size_t)d * n + i] = s.v[d];
+    if (lo) lo[(size_t)d * n + i] = s.vl[d];
+  }
+}
+__device__ inline void hmd_add_images(int32_t* images, uint32_t n, uint32_t i, const HmdAtom& s) {
+#pragma unroll
+  for (int d = 0; d < 3; ++d) images[(size_t)d * n + i] += s.im[d];
 }
 
 // v += F/m dt/2 (integrate.cu:172-215).
-__device__ inline void hmd_vv_kick_atom(const VvParams& p, const uint32_t i) {
+__device__ inline void hmd_vv_kick_state(const VvParams& p, const float f[3], const float m,
+                                         HmdAtom& s) {
 #pragma clang fp contract(off)
-  const float m = p.m[i];
   const float half_dt = p.dt * 0.5f;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    const size_t k = (size_t)d * p.n + i;
-    const float a = p.f[k] / m;
+    const float a = f[d] / m;
     if (p.compensated) {
-      double ext_v = ((double)p.v[k] + p.vel_lo[k]) + (double)(a * half_dt);
-      float vh = (float)ext_v;
-      p.v[k] = vh;
-      p.vel_lo[k] = ext_v - (double)vh;
+      const double ext_v = ((double)s.v[d] + s.vl[d]) + (double)(a * half_dt);
+      s.v[d] = (float)ext_v;
+      s.vl[d] = ext_v - (double)s.v[d];
     } else {
-      p.v[k] = fmaf(a, half_dt, p.v[k]);
+      s.v[d] = fmaf(a, half_dt, s.v[d]);
     }
   }
+}
+
+// Wrap into the primary image, counting the images.
+__device__ inline void hmd_wrap_state(const HmdLattice& L, HmdAtom& s) {
+  int ka, kb, kc;
+  hmd_wrap(s.pq.x, s.pq.y, s.pq.z, ka, kb, kc, L);
+  s.im[0] += ka;
+  s.im[1] += kb;
+  s.im[2] += kc;
+}
+
+// x += v dt; wrap (integrate.cu:24-170).
+__device__ inline void hmd_vv_drift_state(const VvParams& p, HmdAtom& s) {
+#pragma clang fp contract(off)
+  float x[3] = {s.pq.x, s.pq.y, s.pq.z};
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    if (p.compensated) {
+      const double ext_x =
+          fma((double)s.v[d] + s.vl[d], (double)p.dt, (double)x[d] + s.xl[d]);
+      x[d] = (float)ext_x;
+      s.xl[d] = ext_x - (double)x[d];
+    } else {
+      x[d] = fmaf(s.v[d], p.dt, x[d]);
+    }
+  }
+  s.pq.x = x[0];
+  s.pq.y = x[1];
+  s.pq.z = x[2];
+  hmd_wrap_state(p.L, s);
+}
+
+__device__ inline void hmd_load_force(const VvParams& p, uint32_t i, float f[3], float& m) {
+#pragma unroll
+  for (int d = 0; d < 3; ++d) f[d] = p.f[(size_t)d * p.n + i];
+  m = p.m[i];
+}
+
+// One atom of the velocity-Verlet plan as its own kernel.
+__device__ inline void hmd_vv_kick_drift_atom(const VvParams& p, const uint32_t i) {
+  HmdAtom s;
+  float f[3], m;
+  double* xl = p.compensated ? p.pos_lo : nullptr;
+  double* vl = p.compensated ? p.vel_lo : nullptr;
+  hmd_load_pos(p.posq, xl, p.n, i, s);
+  hmd_load_vel(p.v, vl, p.n, i, s);
+  hmd_load_force(p, i, f, m);
+  hmd_vv_kick_state(p, f, m, s);
+  hmd_vv_drift_state(p, s);
+  hmd_store_vel(p.v, vl, p.n, i, s);
+  hmd_store_pos(p.posq, xl, p.n, i, s);
+  hmd_add_images(p.images, p.n, i, s);
+}
+__device__ inline void hmd_vv_kick_atom(const VvParams& p, const uint32_t i) {
+  HmdAtom s;
+  float f[3], m;
+  double* vl = p.compensated ? p.vel_lo : nullptr;
+  hmd_load_vel(p.v, vl, p.n, i, s);
+  hmd_load_force(p, i, f, m);
+  hmd_vv_kick_state(p, f, m, s);
+  hmd_store_vel(p.v, vl, p.n, i, s);
 }
 
 // ------------------------------------------------------------------ SETTLE --
@@ -93,52 +158,46 @@ __device__ inline void hmd_settle_snapshot_group(const SettleParams& p, const ui
   for (int a = 0; a < 3; ++a) sn[3 * g + a] = ps[p.group_atoms[3 * g + a]];
 }
 
-// Apply a position correction to atom `idx`: f32 path or, in compensated
-// mode, to the extended (hi + lo) value, re-split.
-__device__ inline void hmd_apply_pos(const SettleParams& p, uint32_t idx, float4& pq,
-                                     const float cur[3], const float corr[3],
-                                     float inv_dt) {
+// Apply a position correction to an atom: f32 path or, in compensated mode,
+// to the extended (hi + lo) value, re-split.
+__device__ inline void hmd_apply_pos(const SettleParams& p, HmdAtom& s, const float cur[3],
+                                     const float corr[3], float inv_dt) {
 #pragma clang fp contract(off)
   float out[3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    const size_t k = (size_t)d * p.n + idx;
     if (p.pos_lo) {
-      double ext = (double)cur[d] + p.pos_lo[k] + (double)corr[d];
-      float h = (float)ext;
-      p.pos_lo[k] = ext - (double)h;
-      out[d] = h;
-      double ev = (double)p.v[k] + p.vel_lo[k] + (double)(corr[d] * inv_dt);
-      float vh = (float)ev;
-      p.vel_lo[k] = ev - (double)vh;
-      p.v[k] = vh;
+      const double ext = (double)cur[d] + s.xl[d] + (double)corr[d];
+      out[d] = (float)ext;
+      s.xl[d] = ext - (double)out[d];
+      const double ev = (double)s.v[d] + s.vl[d] + (double)(corr[d] * inv_dt);
+      s.v[d] = (float)ev;
+      s.vl[d] = ev - (double)s.v[d];
     } else {
       out[d] = cur[d] + corr[d];
-      p.v[k] = p.v[k] + corr[d] * inv_dt;
+      s.v[d] = s.v[d] + corr[d] * inv_dt;
     }
   }
-  pq.x = out[0];
-  pq.y = out[1];
-  pq.z = out[2];
+  s.pq.x = out[0];
+  s.pq.y = out[1];
+  s.pq.z = out[2];
 }
 
 // Analytic rigid-water position reset (Miyamoto & Kollman, J. Comput.
 // Chem. 13(8), 952-962, 1992) with the half-step velocity fix and the
-// position-level constraint virial, as settle.cu:145-335.
-__device__ inline void hmd_settle_positions_group(const SettleParams& p, const uint32_t g,
-                                                  const float dt) {
+// position-level constraint virial, as settle.cu:145-335.  s: the group's
+// atoms, sn: their positions before the drift, cv: the virial.
+__device__ inline void hmd_settle_positions_state(const SettleParams& p, HmdAtom s[3],
+                                                  const float4 sn[3], const float dt,
+                                                  float cv[3]) {
 #pragma clang fp contract(off)
   const HmdLattice L = p.L;
-  float4* ps = reinterpret_cast<float4*>(p.posq);
-  const float4* sn = reinterpret_cast<const float4*>(p.snapshot);
-  const uint32_t idx[3] = {p.group_atoms[3 * g], p.group_atoms[3 * g + 1],
-                           p.group_atoms[3 * g + 2]};
-  float4 pq[3] = {ps[idx[0]], ps[idx[1]], ps[idx[2]]};
-  float4 s0 = sn[3 * g], s1 = sn[3 * g + 1], s2 = sn[3 * g + 2];
-  float cur[3][3] = {{pq[0].x, pq[0].y, pq[0].z},
-                     {pq[1].x, pq[1].y, pq[1].z},
-                     {pq[2].x, pq[2].y, pq[2].z}};
-  float snp[3][3] = {{s0.x, s0.y, s0.z}, {s1.x, s1.y, s1.z}, {s2.x, s2.y, s2.z}};
+  float cur[3][3] = {{s[0].pq.x, s[0].pq.y, s[0].pq.z},
+                     {s[1].pq.x, s[1].pq.y, s[1].pq.z},
+                     {s[2].pq.x, s[2].pq.y, s[2].pq.z}};
+  float snp[3][3] = {{sn[0].x, sn[0].y, sn[0].z},
+                     {sn[1].x, sn[1].y, sn[1].z},
+                     {sn[2].x, sn[2].y, sn[2].z}};
   // Reference bond vectors and per-atom drifts, minimum-imaged.
   float b0[3] = {snp[1][0] - snp[0][0], snp[1][1] - snp[0][1], snp[1][2] - snp[0][2]};
   float c0[3] = {snp[2][0] - snp[0][0], snp[2][1] - snp[0][1], snp[2][2] - snp[0][2]};
@@ -224,28 +283,45 @@ __device__ inline void hmd_settle_positions_group(const SettleParams& p, const u
       rcm[d] = ex[d] * pr[a][0] + ey[d] * pr[a][1] + ez[d] * pr[a][2];
       corr[d] = (com[d] + rcm[d]) - unc[a][d];
     }
-    hmd_apply_pos(p, idx[a], pq[a], cur[a], corr, inv_dt);
-    ps[idx[a]] = pq[a];
-    if (p.constraint_virial)
-      p.constraint_virial[3 * g + a] =
-          mass[a] * inv_dt2 * (corr[0] * rcm[0] + corr[1] * rcm[1] + corr[2] * rcm[2]);
+    hmd_apply_pos(p, s[a], cur[a], corr, inv_dt);
+    cv[a] = mass[a] * inv_dt2 * (corr[0] * rcm[0] + corr[1] * rcm[1] + corr[2] * rcm[2]);
+  }
+}
+
+// The same as its own kernel.
+__device__ inline void hmd_settle_positions_group(const SettleParams& p, const uint32_t g,
+                                                  const float dt) {
+  const float4* sm = reinterpret_cast<const float4*>(p.snapshot);
+  HmdAtom s[3];
+  float4 sn[3];
+  float cv[3];
+  uint32_t idx[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    idx[a] = p.group_atoms[3 * g + a];
+    hmd_load_pos(p.posq, p.pos_lo, p.n, idx[a], s[a]);
+    hmd_load_vel(p.v, p.vel_lo, p.n, idx[a], s[a]);
+    sn[a] = sm[3 * g + a];
+  }
+  hmd_settle_positions_state(p, s, sn, dt, cv);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    hmd_store_pos(p.posq, p.pos_lo, p.n, idx[a], s[a]);
+    hmd_store_vel(p.v, p.vel_lo, p.n, idx[a], s[a]);
+    if (p.constraint_virial) p.constraint_virial[3 * g + a] = cv[a];
   }
 }
 
 // Analytic velocity projection: 3x3 Cramer solve for the bond impulses
-// (settle.cu:376-490).
-__device__ inline void hmd_settle_velocities_group(const SettleParams& p, const uint32_t g,
-                                                   const float dt) {
+// (settle.cu:376-490).  The velocity-level constraint virial is added to cv.
+__device__ inline void hmd_settle_velocities_state(const SettleParams& p, HmdAtom s[3],
+                                                   const float dt, float cv[3]) {
 #pragma clang fp contract(off)
   const HmdLattice L = p.L;
-  const float4* ps = reinterpret_cast<const float4*>(p.posq);
-  const uint32_t idx[3] = {p.group_atoms[3 * g], p.group_atoms[3 * g + 1],
-                           p.group_atoms[3 * g + 2]};
   float px[3], py[3], pz[3];
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-    float4 q = ps[idx[a]];
-    px[a] = q.x; py[a] = q.y; pz[a] = q.z;
+    px[a] = s[a].pq.x; py[a] = s[a].pq.y; pz[a] = s[a].pq.z;
   }
 #pragma unroll
   for (int a = 1; a < 3; ++a) {
@@ -258,7 +334,7 @@ __device__ inline void hmd_settle_velocities_group(const SettleParams& p, const 
 #pragma unroll
   for (int a = 0; a < 3; ++a)
 #pragma unroll
-    for (int d = 0; d < 3; ++d) v[a][d] = p.v[(size_t)d * p.n + idx[a]];
+    for (int d = 0; d < 3; ++d) v[a][d] = s[a].v[d];
   const float r1[3] = {px[0] - px[1], py[0] - py[1], pz[0] - pz[1]};
   const float r2[3] = {px[0] - px[2], py[0] - py[2], pz[0] - pz[2]};
   const float r3[3] = {px[1] - px[2], py[1] - py[2], pz[1] - pz[2]};
@@ -305,14 +381,12 @@ __device__ inline void hmd_settle_velocities_group(const SettleParams& p, const 
   for (int a = 0; a < 3; ++a)
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      const size_t k = (size_t)d * p.n + idx[a];
       if (p.vel_lo) {
-        double ev = (double)v[a][d] + p.vel_lo[k] + (double)dv[a][d];
-        float vh = (float)ev;
-        p.vel_lo[k] = ev - (double)vh;
-        p.v[k] = vh;
+        const double ev = (double)v[a][d] + s[a].vl[d] + (double)dv[a][d];
+        s[a].v[d] = (float)ev;
+        s[a].vl[d] = ev - (double)s[a].v[d];
       } else {
-        p.v[k] = v[a][d] + dv[a][d];
+        s[a].v[d] = v[a][d] + dv[a][d];
       }
     }
   if (p.constraint_virial && dt > 0.0f) {
@@ -324,9 +398,29 @@ __device__ inline void hmd_settle_velocities_group(const SettleParams& p, const 
     const float mass[3] = {p.m_o, p.m_h, p.m_h};
 #pragma unroll
     for (int a = 0; a < 3; ++a)
-      p.constraint_virial[3 * g + a] +=
-          mass[a] * inv_dt * (dv[a][0] * (px[a] - cx) + dv[a][1] * (py[a] - cy) +
-                              dv[a][2] * (pz[a] - cz));
+      cv[a] += mass[a] * inv_dt * (dv[a][0] * (px[a] - cx) + dv[a][1] * (py[a] - cy) +
+                                  dv[a][2] * (pz[a] - cz));
+  }
+}
+
+// The same as its own kernel.
+__device__ inline void hmd_settle_velocities_group(const SettleParams& p, const uint32_t g,
+                                                   const float dt) {
+  HmdAtom s[3];
+  float cv[3] = {0.0f, 0.0f, 0.0f};
+  uint32_t idx[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    idx[a] = p.group_atoms[3 * g + a];
+    hmd_load_pos(p.posq, nullptr, p.n, idx[a], s[a]);
+    hmd_load_vel(p.v, p.vel_lo, p.n, idx[a], s[a]);
+    if (p.constraint_virial) cv[a] = p.constraint_virial[3 * g + a];
+  }
+  hmd_settle_velocities_state(p, s, dt, cv);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    hmd_store_vel(p.v, p.vel_lo, p.n, idx[a], s[a]);
+    if (p.constraint_virial) p.constraint_virial[3 * g + a] = cv[a];
   }
 }
 
@@ -374,36 +468,52 @@ __device__ inline float hmd_philox_gaussian(uint32_t sl, uint32_t sh, uint32_t c
 
 // A step: x += v dt/2 (one rounding, as the reference's contracted
 // x + v * half_dt), wrap (langevin.cu:13-50).
-__device__ inline void hmd_lan_drift_half_atom(const LangevinParams& p, const uint32_t i) {
+__device__ inline void hmd_lan_drift_half_state(const LangevinParams& p, HmdAtom& s) {
 #pragma clang fp contract(off)
-  float4 pq = reinterpret_cast<float4*>(p.posq)[i];
   const float h = p.dt * 0.5f;
-  float x = fmaf(p.v[i], h, pq.x), y = fmaf(p.v[p.n + i], h, pq.y),
-        z = fmaf(p.v[2 * p.n + i], h, pq.z);
-  int ka, kb, kc;
-  hmd_wrap(x, y, z, ka, kb, kc, p.L);
-  p.images[i] += ka;
-  p.images[p.n + i] += kb;
-  p.images[2 * p.n + i] += kc;
-  pq.x = x; pq.y = y; pq.z = z;
-  reinterpret_cast<float4*>(p.posq)[i] = pq;
+  s.pq.x = fmaf(s.v[0], h, s.pq.x);
+  s.pq.y = fmaf(s.v[1], h, s.pq.y);
+  s.pq.z = fmaf(s.v[2], h, s.pq.z);
+  hmd_wrap_state(p.L, s);
+}
+
+// The normal of atom i's axis d in this step's O sub-step: Philox keyed by
+// the seed with counter (draw_lo, draw_hi, particle id, axis).
+__device__ inline float hmd_lan_xi(const LangevinParams& p, const unsigned long long step,
+                                   const uint32_t i, const uint32_t d) {
+  return hmd_philox_gaussian(p.seed_lo, p.seed_hi, (uint32_t)(step & 0xFFFFFFFFull),
+                             (uint32_t)(step >> 32), i, d);
 }
 
 // O step: v = a v + sigma xi with sigma = sqrt((1 - a^2) kT / m) in f32
 // (1 - a^2 and a v + (sigma xi) each rounded once, as the reference's
-// contracted expressions), xi from Philox keyed by the seed with counter
-// (draw_lo, draw_hi, particle id, axis) (langevin.cu:52-80).
-__device__ inline void hmd_lan_ou_atom(const LangevinParams& p, const uint32_t i) {
+// contracted expressions) (langevin.cu:52-80).
+__device__ inline void hmd_lan_ou_state(const LangevinParams& p, const float m,
+                                        const float xi[3], HmdAtom& s) {
 #pragma clang fp contract(off)
-  const unsigned long long step = *p.step;
-  const uint32_t cl = (uint32_t)(step & 0xFFFFFFFFull), ch = (uint32_t)(step >> 32);
-  const float sig = sqrtf(fmaf(-p.a, p.a, 1.0f) * p.kt / p.m[i]);
+  const float sig = sqrtf(fmaf(-p.a, p.a, 1.0f) * p.kt / m);
 #pragma unroll
-  for (uint32_t d = 0; d < 3; ++d) {
-    const float xi = hmd_philox_gaussian(p.seed_lo, p.seed_hi, cl, ch, i, d);
-    const size_t k = (size_t)d * p.n + i;
-    p.v[k] = fmaf(p.a, p.v[k], sig * xi);
-  }
+  for (int d = 0; d < 3; ++d) s.v[d] = fmaf(p.a, s.v[d], sig * xi[d]);
+}
+
+// One atom of the Langevin plan's sub-steps as their own kernels.
+__device__ inline void hmd_lan_drift_half_atom(const LangevinParams& p, const uint32_t i) {
+  HmdAtom s;
+  hmd_load_pos(p.posq, nullptr, p.n, i, s);
+  hmd_load_vel(p.v, nullptr, p.n, i, s);
+  hmd_lan_drift_half_state(p, s);
+  hmd_store_pos(p.posq, nullptr, p.n, i, s);
+  hmd_add_images(p.images, p.n, i, s);
+}
+__device__ inline void hmd_lan_ou_atom(const LangevinParams& p, const uint32_t i) {
+  HmdAtom s;
+  hmd_load_vel(p.v, nullptr, p.n, i, s);
+  const unsigned long long step = *p.step;
+  float xi[3];
+#pragma unroll 1
+  for (uint32_t d = 0; d < 3; ++d) xi[d] = hmd_lan_xi(p, step, i, d);
+  hmd_lan_ou_state(p, p.m[i], xi, s);
+  hmd_store_vel(p.v, nullptr, p.n, i, s);
 }
 
 // ---------------------------------------------------- one kernel per op --
@@ -460,33 +570,82 @@ HMD_KERNEL(hmd_lan_ou, LangevinParams, 256)
 
 // ------------------------------------------------------ fused step kernels --
 // The integrator's sub-steps between two force evaluations in one launch.
-// Thread u < n_groups owns SETTLE group u and runs every sub-step for its
-// three atoms in plan order (the constraint couples only the atoms of one
-// group, so no other thread's data is read); thread n_groups + k owns free
-// atom free_atoms[k] (atom k when free_atoms is null).  Each atom sees the
-// same operations, in the same order and with the same rounding, as in the
-// one-kernel-per-sub-step plan.
+// One thread owns a SETTLE group and runs every sub-step for its three atoms
+// in plan order (the constraint couples only the atoms of one group, so no
+// other thread's data is read); free atoms (free_atoms[k], atom k when null)
+// have a thread each.  Each atom sees the same operations, in the same order
+// and with the same rounding, as in the one-kernel-per-sub-step plan.
+//
+// Bound by latency: a box of 65,536 groups is one wave a SIMD.  The state is
+// loaded once, kept in registers through the sub-steps and stored once (the
+// sub-steps' own loads and stores made a chain of ten memory round trips in
+// the Langevin kernel), and the groups are spread over workgroups of one
+// wave.  Traced at 65,536 groups: first velocity-Verlet kernel 21.8 -> 13.8
+// us (compensated, 41 MB), last kick 11.2 -> 7.9 us; Langevin kernel 28.9 ->
+// 14.0 us at 8,192 groups, 25.5 -> 13.6 us at 216.
 __device__ inline bool hmd_unit(const StepParams& p, uint32_t u, uint32_t& g, uint32_t& atom) {
   if (u < p.st.n_groups) { g = u; return true; }
   const uint32_t k = u - p.st.n_groups;
   g = HMD_SENTINEL;
-  atom = p.free_atoms ? p.free_atoms[k] : k;
-  return k < p.n_free;
+  atom = k;
+  if (k >= p.n_free) return false;
+  if (p.free_atoms) atom = p.free_atoms[k];
+  return true;
 }
 
 // The neighbour list's skin check (hmd_nbl_displacement, the same f32
 // arithmetic) on an atom's final position of the step, folded into the
 // kernel that wrote it: one dependent launch less before the force
-// evaluation.
-__device__ inline void hmd_step_disp_check(const NblDispParams& d, uint32_t atom) {
+// evaluation.  r: the atom's position at the last list build.
+__device__ inline bool hmd_step_displaced(const NblDispParams& d, const float4 a, const float4 r) {
 #pragma clang fp contract(off)
-  if (!d.status) return;
-  const float4 a = reinterpret_cast<const float4*>(d.posq)[atom];
-  const float4 r = reinterpret_cast<const float4*>(d.ref_pos)[atom];
   float dx = a.x - r.x, dy = a.y - r.y, dz = a.z - r.z;
   hmd_min_image(dx, dy, dz, d.L);
   const float d2 = dx * dx + dy * dy + dz * dz;
-  if (d2 > d.threshold_sq) atomicOr(d.status, HMD_STATUS_DISPLACED);
+  return d2 > d.threshold_sq;
+}
+__device__ inline float4 hmd_step_ref(const NblDispParams& d, uint32_t atom) {
+  return d.status ? reinterpret_cast<const float4*>(d.ref_pos)[atom]
+                  : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+}
+
+// A group's atoms loaded at once.
+struct HmdGroup {
+  HmdAtom s[3];
+  uint32_t idx[3];
+  float f[3][3], m[3];
+};
+__device__ inline void hmd_load_group(const StepParams& p, const uint32_t g, bool pos_lo,
+                                      HmdGroup& G) {
+  double* xl = p.vv.compensated && pos_lo ? p.vv.pos_lo : nullptr;
+  double* vl = p.vv.compensated ? p.vv.vel_lo : nullptr;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) G.idx[a] = p.st.group_atoms[3 * g + a];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    hmd_load_pos(p.vv.posq, xl, p.vv.n, G.idx[a], G.s[a]);
+    hmd_load_vel(p.vv.v, vl, p.vv.n, G.idx[a], G.s[a]);
+    hmd_load_force(p.vv, G.idx[a], G.f[a], G.m[a]);
+  }
+}
+// Positions, velocities and images back, with the skin check.
+__device__ inline void hmd_store_group(const StepParams& p, const HmdGroup& G,
+                                       const float4 ref[3]) {
+  double* xl = p.vv.compensated ? p.vv.pos_lo : nullptr;
+  double* vl = p.vv.compensated ? p.vv.vel_lo : nullptr;
+  bool moved = false;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    hmd_store_pos(p.vv.posq, xl, p.vv.n, G.idx[a], G.s[a]);
+    hmd_store_vel(p.vv.v, vl, p.vv.n, G.idx[a], G.s[a]);
+    hmd_add_images(p.vv.images, p.vv.n, G.idx[a], G.s[a]);
+    moved |= hmd_step_displaced(p.disp, G.s[a].pq, ref[a]);
+  }
+  if (moved && p.disp.status) atomicOr(p.disp.status, HMD_STATUS_DISPLACED);
+}
+__device__ inline void hmd_snap(const HmdGroup& G, float4 sn[3]) {
+#pragma unroll
+  for (int a = 0; a < 3; ++a) sn[a] = G.s[a].pq;
 }
 
 // velocity Verlet: [snapshot] kick-drift [SETTLE positions] [skin check]
@@ -496,51 +655,107 @@ __device__ __forceinline__ void hmd_step_vv_first_body(const StepParams& p, cons
   uint32_t g, atom;
   if (!hmd_unit(p, u, g, atom)) return;
   if (g != HMD_SENTINEL) {
-    hmd_settle_snapshot_group(p.st, g);
-#pragma unroll 1
-    for (int a = 0; a < 3; ++a) hmd_vv_kick_drift_atom(p.vv, p.st.group_atoms[3 * g + a]);
-    hmd_settle_positions_group(p.st, g, p.dt);
-#pragma unroll 1
-    for (int a = 0; a < 3; ++a) hmd_step_disp_check(p.disp, p.st.group_atoms[3 * g + a]);
+    HmdGroup G;
+    float4 ref[3], sn[3];
+    float cv[3];
+    hmd_load_group(p, g, true, G);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) ref[a] = hmd_step_ref(p.disp, G.idx[a]);
+    hmd_snap(G, sn);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      hmd_vv_kick_state(p.vv, G.f[a], G.m[a], G.s[a]);
+      hmd_vv_drift_state(p.vv, G.s[a]);
+    }
+    hmd_settle_positions_state(p.st, G.s, sn, p.dt, cv);
+    hmd_store_group(p, G, ref);
+    if (p.st.particle_virial) {   // read by the step's last kernel only then
+#pragma unroll
+      for (int a = 0; a < 3; ++a) p.st.constraint_virial[3 * g + a] = cv[a];
+    }
   } else {
     hmd_vv_kick_drift_atom(p.vv, atom);
-    hmd_step_disp_check(p.disp, atom);
+    if (p.disp.status &&
+        hmd_step_displaced(p.disp, reinterpret_cast<const float4*>(p.vv.posq)[atom],
+                           hmd_step_ref(p.disp, atom)))
+      atomicOr(p.disp.status, HMD_STATUS_DISPLACED);
   }
 }
 HMD_KERNEL(hmd_step_vv_first, StepParams, 256)
 
 // Langevin BAOAB up to the force evaluation: B [SETTLE v] [snapshot] A
-// [SETTLE x, dt/2] O [SETTLE v] [snapshot] A [SETTLE x, dt/2] [skin check]
+// [SETTLE x, dt/2] O [SETTLE v] [snapshot] A [SETTLE x, dt/2] [skin check].
+// A workgroup of 256 threads takes groups_per_block groups: all its threads
+// draw the groups' normals first (nine a group; a Philox block and an FP64
+// log, square root and cosine each, half of the kernel's time when the
+// group's own thread drew them one after the other), then a thread a group
+// runs the sub-steps.  Blocks past group_blocks take 256 free atoms each.
+#define HMD_BAOA_GROUPS 64u
 __device__ __forceinline__ void hmd_step_baoa_body(const StepParams& p, const uint32_t hmd_bx,
     const uint32_t hmd_gx) {
-  const uint32_t u = hmd_bx * blockDim.x + threadIdx.x;
-  uint32_t g, atom;
-  if (!hmd_unit(p, u, g, atom)) return;
+  __shared__ float s_xi[9 * HMD_BAOA_GROUPS];
+  const unsigned long long step = *p.lan.step;
+  if (hmd_bx >= p.group_blocks) {
+    const uint32_t k = (hmd_bx - p.group_blocks) * blockDim.x + threadIdx.x;
+    if (k >= p.n_free) return;
+    const uint32_t i = p.free_atoms ? p.free_atoms[k] : k;
+    HmdAtom s;
+    float f[3], m, xi[3];
+    hmd_load_pos(p.lan.posq, nullptr, p.lan.n, i, s);
+    hmd_load_vel(p.lan.v, nullptr, p.lan.n, i, s);
+    hmd_load_force(p.vv, i, f, m);
+    const float4 ref = hmd_step_ref(p.disp, i);
+#pragma unroll 1
+    for (uint32_t d = 0; d < 3; ++d) xi[d] = hmd_lan_xi(p.lan, step, i, d);
+    hmd_vv_kick_state(p.vv, f, m, s);
+    hmd_lan_drift_half_state(p.lan, s);
+    hmd_lan_ou_state(p.lan, m, xi, s);
+    hmd_lan_drift_half_state(p.lan, s);
+    hmd_store_pos(p.lan.posq, nullptr, p.lan.n, i, s);
+    hmd_store_vel(p.lan.v, nullptr, p.lan.n, i, s);
+    hmd_add_images(p.lan.images, p.lan.n, i, s);
+    if (p.disp.status && hmd_step_displaced(p.disp, s.pq, ref))
+      atomicOr(p.disp.status, HMD_STATUS_DISPLACED);
+    return;
+  }
+  const uint32_t g0 = hmd_bx * p.groups_per_block;
+  const uint32_t ng = min(p.groups_per_block, p.st.n_groups - g0);
+  const bool mine = threadIdx.x < ng;
+  const uint32_t g = g0 + threadIdx.x;
+  HmdGroup G;
+  float4 ref[3], sn[3];
+  if (mine) {
+    hmd_load_group(p, g, false, G);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) ref[a] = hmd_step_ref(p.disp, G.idx[a]);
+  }
+  for (uint32_t k = threadIdx.x; k < 9u * ng; k += blockDim.x) {
+    const uint32_t a = k / 3u, d = k - 3u * a;   // a: atom of the block's groups
+    s_xi[k] = hmd_lan_xi(p.lan, step, p.st.group_atoms[3u * g0 + a], d);
+  }
+  __syncthreads();
+  if (!mine) return;
   const float h = 0.5f * p.dt;
-  if (g != HMD_SENTINEL) {
-    const uint32_t* ga = p.st.group_atoms + 3 * g;
-#pragma unroll 1
-    for (int a = 0; a < 3; ++a) hmd_vv_kick_atom(p.vv, ga[a]);
-    hmd_settle_velocities_group(p.st, g, p.dt);
-    hmd_settle_snapshot_group(p.st, g);
-#pragma unroll 1
-    for (int a = 0; a < 3; ++a) hmd_lan_drift_half_atom(p.lan, ga[a]);
-    hmd_settle_positions_group(p.st, g, h);
-#pragma unroll 1
-    for (int a = 0; a < 3; ++a) hmd_lan_ou_atom(p.lan, ga[a]);
-    hmd_settle_velocities_group(p.st, g, p.dt);
-    hmd_settle_snapshot_group(p.st, g);
-#pragma unroll 1
-    for (int a = 0; a < 3; ++a) hmd_lan_drift_half_atom(p.lan, ga[a]);
-    hmd_settle_positions_group(p.st, g, h);
-#pragma unroll 1
-    for (int a = 0; a < 3; ++a) hmd_step_disp_check(p.disp, ga[a]);
-  } else {
-    hmd_vv_kick_atom(p.vv, atom);
-    hmd_lan_drift_half_atom(p.lan, atom);
-    hmd_lan_ou_atom(p.lan, atom);
-    hmd_lan_drift_half_atom(p.lan, atom);
-    hmd_step_disp_check(p.disp, atom);
+  float cv[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int a = 0; a < 3; ++a) hmd_vv_kick_state(p.vv, G.f[a], G.m[a], G.s[a]);
+  hmd_settle_velocities_state(p.st, G.s, p.dt, cv);
+  hmd_snap(G, sn);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) hmd_lan_drift_half_state(p.lan, G.s[a]);
+  hmd_settle_positions_state(p.st, G.s, sn, h, cv);
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+    hmd_lan_ou_state(p.lan, G.m[a], &s_xi[9u * threadIdx.x + 3u * a], G.s[a]);
+  hmd_settle_velocities_state(p.st, G.s, p.dt, cv);
+  hmd_snap(G, sn);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) hmd_lan_drift_half_state(p.lan, G.s[a]);
+  hmd_settle_positions_state(p.st, G.s, sn, h, cv);
+  hmd_store_group(p, G, ref);
+  if (p.st.particle_virial) {   // read by the step's last kernel only then
+#pragma unroll
+    for (int a = 0; a < 3; ++a) p.st.constraint_virial[3 * g + a] = cv[a];
   }
 }
 HMD_KERNEL(hmd_step_baoa, StepParams, 256)
@@ -554,10 +769,25 @@ __device__ __forceinline__ void hmd_step_kick_last_body(const StepParams& p, con
   uint32_t g, atom;
   if (!hmd_unit(p, u, g, atom)) return;
   if (g != HMD_SENTINEL) {
-#pragma unroll 1
-    for (int a = 0; a < 3; ++a) hmd_vv_kick_atom(p.vv, p.st.group_atoms[3 * g + a]);
-    hmd_settle_velocities_group(p.st, g, p.dt);
-    if (p.st.particle_virial) hmd_settle_virial_group(p.st, g);
+    HmdGroup G;
+    float cv[3] = {0.0f, 0.0f, 0.0f}, w[3] = {0.0f, 0.0f, 0.0f};
+    hmd_load_group(p, g, false, G);
+    if (p.st.particle_virial) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        cv[a] = p.st.constraint_virial[3 * g + a];
+        w[a] = p.st.particle_virial[G.idx[a]];
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) hmd_vv_kick_state(p.vv, G.f[a], G.m[a], G.s[a]);
+    hmd_settle_velocities_state(p.st, G.s, p.dt, cv);
+    double* vl = p.vv.compensated ? p.vv.vel_lo : nullptr;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      hmd_store_vel(p.vv.v, vl, p.vv.n, G.idx[a], G.s[a]);
+      if (p.st.particle_virial) p.st.particle_virial[G.idx[a]] = w[a] + cv[a];
+    }
   } else {
     hmd_vv_kick_atom(p.vv, atom);
   }

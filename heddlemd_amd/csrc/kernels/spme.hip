@@ -192,87 +192,155 @@ __device__ inline long long hmd_fixed32_of24(float v) {
   return ((long long)r1 << 8) + (long long)r2;
 }
 
+// Queue entries of the spread: weights of 2 x 256 atoms at order 4 (27 KB
+// beside the brick), of one round of candidates at the higher orders.
+#define HMD_SPREAD_QUEUE(P) ((P) == 4 ? 512u : 256u)
+
+// Spread of one brick per workgroup.
+//
+// The atoms of the eight bins are one candidate list (their ranges joined by a
+// prefix), filtered a workgroup's width at a time: a candidate whose support
+// reaches the brick (a third to a quarter of them) puts its weights and mesh
+// position into an LDS queue.  The queue is then worked off P lanes an atom,
+// lane d taking the support plane d of the fast axis, so that P lanes add to P
+// consecutive mesh points, every lane has the same P^2 adds to do, and lanes
+// of atoms that miss the brick do not idle through the adds of the others.
+// The contributions are the same numbers in whatever order, and integer sums:
+// the mesh does not depend on the split.
+//
+// Bound by the latency of the chain bins -> atoms -> positions -> LDS adds in
+// small systems and by the LDS adds in large ones.  One thread an atom
+// over the eight bins in turn, all P^3 adds its own, took 29.1 us at 648
+// atoms on 24^3 (now 6.0), 31 us at 24,576 on 64^3 (11.6), 47 us at 196,608
+// on 128^3 (42) and 111 us at 4,503 on 40^3 with order 6 (26).
 template <int P>
 __device__ inline void hmd_spread_body(const SpmeSpreadParams& p, const uint32_t hmd_bx,
     const uint32_t hmd_gx) {
+  constexpr uint32_t Q = HMD_SPREAD_QUEUE(P);
   extern __shared__ long long s_acc[];
+  __shared__ float s_w[3][P][Q];          // weights; axis 0 times the charge
+  __shared__ uint16_t s_at[3][Q];         // primary point relative to the brick
+  __shared__ uint32_t s_n;
   const uint32_t bsz = p.b0 * p.b1 * p.b2;
   const uint32_t B = hmd_bx;
   const uint32_t B2 = B % p.nb2, B1 = (B / p.nb2) % p.nb1, B0 = B / (p.nb2 * p.nb1);
   const int o0 = (int)(B0 * p.b0), o1 = (int)(B1 * p.b1), o2 = (int)(B2 * p.b2);
-  for (uint32_t k = threadIdx.x; k < bsz; k += blockDim.x) s_acc[k] = 0;
-  __syncthreads();
-
+  const uint32_t lane = hmd_lane();
+  // ranges of the eight bins (every thread: wave-uniform loads)
+  uint32_t beg[8], cum[9];
+  cum[0] = 0;
+#pragma unroll
   for (uint32_t nb = 0; nb < 8; ++nb) {
     // With a single brick along an axis the +1 neighbour is the brick
     // itself: visit it once.
-    if ((p.nb0 == 1 && (nb & 4u)) || (p.nb1 == 1 && (nb & 2u)) ||
-        (p.nb2 == 1 && (nb & 1u)))
-      continue;
+    const bool skip = (p.nb0 == 1 && (nb & 4u)) || (p.nb1 == 1 && (nb & 2u)) ||
+                      (p.nb2 == 1 && (nb & 1u));
     const uint32_t c0 = (B0 + ((nb >> 2) & 1u)) % p.nb0;
     const uint32_t c1 = (B1 + ((nb >> 1) & 1u)) % p.nb1;
     const uint32_t c2 = (B2 + (nb & 1u)) % p.nb2;
     const uint32_t bin = (c0 * p.nb1 + c1) * p.nb2 + c2;
-    const uint32_t beg = p.bin_start[bin], end = p.bin_start[bin + 1];
-    for (uint32_t k = beg + threadIdx.x; k < end; k += blockDim.x) {
-      const uint32_t a = p.bin_atoms[k];
+    beg[nb] = p.bin_start[bin];
+    cum[nb + 1] = cum[nb] + (skip ? 0u : p.bin_start[bin + 1] - beg[nb]);
+  }
+  const uint32_t total = cum[8];
+  for (uint32_t k = threadIdx.x; k < bsz; k += blockDim.x) s_acc[k] = 0;
+  if (threadIdx.x == 0) s_n = 0;
+  __syncthreads();
+
+  for (uint32_t k0 = 0; k0 < total; k0 += blockDim.x) {
+    const uint32_t k = k0 + threadIdx.x;
+    bool in = false;
+    float wa[P], wb[P], wc[P];
+    uint32_t at[3];
+    if (k < total) {
+      uint32_t at_k = 0;
+#pragma unroll
+      for (uint32_t nb = 0; nb < 8; ++nb)
+        if (k >= cum[nb] && k < cum[nb + 1]) at_k = beg[nb] + (k - cum[nb]);
+      const uint32_t a = p.bin_atoms[at_k];
       const float4 pq = reinterpret_cast<const float4*>(p.posq)[a];
-      if (pq.w == 0.0f) continue;
       float t[3];
       int g[3];
       hmd_spme_setup(pq, p.L, p.n0, p.n1, p.n2, t, g);
-      // Which of the P support planes along each axis fall in this brick;
-      // an atom of a neighbour bin usually reaches it along no plane of
-      // some axis, and is then skipped before its weights are computed.
-      uint32_t ma = 0, mb = 0, mc = 0;
+      // Does any of the P support planes along each axis fall in this brick?
+      const int oo[3] = {o0, o1, o2};
+      const uint32_t nn[3] = {p.n0, p.n1, p.n2}, bb[3] = {p.b0, p.b1, p.b2};
+      in = pq.w != 0.0f;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const int u = g[d] - oo[d];
+        at[d] = (uint32_t)(u + (u < 0 ? (int)nn[d] : 0));
+        // planes at[d], at[d] - 1, ..., at[d] - (P - 1), wrapped: the first
+        // inside the brick, or one of the others after it (or past the wrap)
+        in = in && (at[d] < bb[d] + (uint32_t)(P - 1));
+      }
+      if (in) {
+        hmd_bspline<P>(t[0], wa);
+        hmd_bspline<P>(t[1], wb);
+        hmd_bspline<P>(t[2], wc);
+        const float q24 = pq.w * 16777216.0f;   // charge in 2^-24 units
+#pragma unroll
+        for (int d = 0; d < P; ++d) wa[d] = q24 * wa[d];
+      }
+    }
+    const uint64_t m = __ballot(in);
+    uint32_t slot = 0;
+    if (m != 0ull) {
+      const uint32_t leader = (uint32_t)__builtin_ctzll(m);
+      if (lane == leader) slot = atomicAdd(&s_n, (uint32_t)__builtin_popcountll(m));
+      slot = hmd_readlane(slot, leader) +
+             (uint32_t)__builtin_popcountll(m & ((lane == 0) ? 0ull : (~0ull >> (64 - lane))));
+    }
+    if (in) {
 #pragma unroll
       for (int d = 0; d < P; ++d) {
-        int la = g[0] - d - o0, lb = g[1] - d - o1, lc = g[2] - d - o2;
-        la += (la < 0) ? (int)p.n0 : 0;
-        lb += (lb < 0) ? (int)p.n1 : 0;
-        lc += (lc < 0) ? (int)p.n2 : 0;
-        ma |= (la < (int)p.b0) ? (1u << d) : 0u;
-        mb |= (lb < (int)p.b1) ? (1u << d) : 0u;
-        mc |= (lc < (int)p.b2) ? (1u << d) : 0u;
+        s_w[0][d][slot] = wa[d];
+        s_w[1][d][slot] = wb[d];
+        s_w[2][d][slot] = wc[d];
       }
-      if (ma == 0u || mb == 0u || mc == 0u) continue;
-      float wa[P], wb[P], wc[P];
-      hmd_bspline<P>(t[0], wa);
-      hmd_bspline<P>(t[1], wb);
-      hmd_bspline<P>(t[2], wc);
-      int lc_of[P];
 #pragma unroll
-      for (int dc = 0; dc < P; ++dc) {
-        int lc = g[2] - dc - o2;
-        lc_of[dc] = lc + ((lc < 0) ? (int)p.n2 : 0);
-      }
-      const float q24 = pq.w * 16777216.0f;   // charge in 2^-24 units
+      for (int d = 0; d < 3; ++d) s_at[d][slot] = (uint16_t)at[d];
+    }
+    __syncthreads();
+    const uint32_t cnt = s_n;
+    __syncthreads();   // every thread has the same count before it grows again
+    // room for another round of candidates: go on collecting
+    if (k0 + blockDim.x < total && cnt + blockDim.x <= Q) continue;
+    for (uint32_t task = threadIdx.x; task < cnt * (uint32_t)P; task += blockDim.x) {
+      const uint32_t e = task / (uint32_t)P, dc = task - e * (uint32_t)P;
+      int lc = (int)s_at[2][e] - (int)dc;
+      lc += (lc < 0) ? (int)p.n2 : 0;
+      if (lc >= (int)p.b2) continue;
+      const float w = s_w[2][dc][e];
+      const int a0 = (int)s_at[0][e], b0 = (int)s_at[1][e];
+      float wbv[P];
+#pragma unroll
+      for (int db = 0; db < P; ++db) wbv[db] = s_w[1][db][e];
 #pragma unroll
       for (int da = 0; da < P; ++da) {
-        if (!((ma >> da) & 1u)) continue;
-        int la = g[0] - da - o0;
+        int la = a0 - da;
         la += (la < 0) ? (int)p.n0 : 0;
-        const float qa = q24 * wa[da];
+        if (la >= (int)p.b0) continue;
+        const float qa = s_w[0][da][e];
+        long long* plane = s_acc + (uint32_t)la * p.b1 * p.b2 + (uint32_t)lc;
 #pragma unroll
         for (int db = 0; db < P; ++db) {
-          if (!((mb >> db) & 1u)) continue;
-          int lb = g[1] - db - o1;
+          int lb = b0 - db;
           lb += (lb < 0) ? (int)p.n1 : 0;
-          const float qab = qa * wb[db];
-          long long* row = s_acc + ((uint32_t)la * p.b1 + (uint32_t)lb) * p.b2;
-#pragma unroll
-          for (int dc = 0; dc < P; ++dc) {
-            if (!((mc >> dc) & 1u)) continue;
-            atomicAdd(reinterpret_cast<unsigned long long*>(&row[lc_of[dc]]),
-                      (unsigned long long)hmd_fixed32_of24(qab * wc[dc]));
-          }
+          if (lb >= (int)p.b1) continue;
+          atomicAdd(reinterpret_cast<unsigned long long*>(&plane[(uint32_t)lb * p.b2]),
+                    (unsigned long long)hmd_fixed32_of24((qa * wbv[db]) * w));
         }
       }
     }
+    __syncthreads();
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
   }
-  __syncthreads();
+  const float ib2 = 1.0f / (float)p.b2, ib1 = 1.0f / (float)p.b1;
   for (uint32_t k = threadIdx.x; k < bsz; k += blockDim.x) {
-    const uint32_t lc = k % p.b2, lb = (k / p.b2) % p.b1, la = k / (p.b2 * p.b1);
+    const uint32_t row = hmd_div_small(k, ib2), lc = k - row * p.b2;
+    const uint32_t la = hmd_div_small(row, ib1), lb = row - la * p.b1;
     const size_t gi = ((size_t)(o0 + la) * p.n1 + (o1 + lb)) * p.n2 + (o2 + lc);
     p.rho[gi] = hmd_from_fixed(s_acc[k], HMD_SPREAD_SHIFT);
   }

@@ -23,7 +23,8 @@ struct Mlp {
   // per-system work buffers
   uint32_t n = 0, n_pad = 0, n_waves = 0;
   DevBuf<long long> desc_acc, force_acc;
-  DevBuf<float> desc, desc_canon, df, resid, partials, scratch_f, target;
+  DevBuf<uint16_t> desc;
+  DevBuf<float> desc_canon, df, resid, partials, scratch_f, target;
   DevBuf<double> red, red_out;
   uint32_t red_blocks = 0;
   // training frames
@@ -146,7 +147,7 @@ struct Mlp {
     NnPassParams q = pass_params(ff);
     launch(c, K_hmd_nn_backward, (uint32_t)c.num_cus, 256, 0, q);
     NnGradReduceParams gp{partials.ptr, n_waves, grad.ptr};
-    launch(c, K_hmd_nn_grad_reduce, HMD_NN_PARAMS, 256, 0, gp);
+    launch(c, K_hmd_nn_grad_reduce, HMD_NN_PARTIAL / 64, 1024, 0, gp);
   }
 
   void adam() {

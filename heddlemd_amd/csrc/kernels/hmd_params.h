@@ -518,7 +518,7 @@ struct NnPassParams {
   float r_cut2, inv_r_cut;     // r_nn^2, 1/r_nn
   float force_scale;           // s_out
   long long* desc_acc;         // [16][n_pad] fixed point (descriptor pass)
-  const float* desc;           // [n_pad][16] sorted (forward/backward)
+  const uint16_t* desc;        // [n_pad][16] bf16, sorted (forward/backward)
   const uint16_t* ops;         // packed operands (forward/backward)
   const float* vec;            // b1, b2, w3, b3
   long long* force_acc;        // [3][n_pad] fixed point dF (forward)
@@ -530,7 +530,7 @@ struct NnDescFinalizeParams {
   long long* desc_acc;         // [16][n_pad], cleared after reading
   uint32_t n_pad, n;
   const uint32_t* sorted_id;   // sorted slot -> canonical id
-  float* desc;                 // [n_pad][16] sorted
+  uint16_t* desc;              // [n_pad][16] bf16, sorted
   float* desc_canon;           // [n][16] canonical (optional)
 };
 

@@ -365,3 +365,44 @@ def test_judged_block_that_overflowed_is_re_run_from_its_start(gpu_ctx):
     assert ja == jb
     for k in ("posq", "vel", "force", "images"):
         assert np.array_equal(a[k].view(np.uint32), b[k].view(np.uint32)), k
+
+
+@pytest.mark.parametrize("n, spread_nm", [(2, 0.4), (7, 0.4), (9, 0.4), (34, 0.5), (65, 0.6),
+                                          (131, 1.2)])
+def test_batch_tails_match_oracle(gpu_ctx, n, spread_nm):
+    """Droplets in a 4 nm box: 1, 21, 36 pairs in one entry (a tail of a
+    batch, more than one half of it, one batch and a tail), then full queues
+    over two and three clusters with a last cluster of 1 or 3 atoms.  The
+    tolerance is the module's (bf16 rounding points of the operands)."""
+    from heddlemd_amd import systems
+    rng = np.random.default_rng(100 + n)
+    L = 4.0 * U.NM
+    pos = np.zeros((0, 3))
+    while len(pos) < n:                     # no two atoms within 0.08 nm
+        p = rng.uniform(-0.5, 0.5, (1, 3)) * spread_nm * U.NM
+        if len(pos) == 0 or np.linalg.norm(pos - p, axis=1).min() > 0.08 * U.NM:
+            pos = np.concatenate([pos, p])
+    q = rng.uniform(-0.8, 0.8, n)
+    types = (np.arange(n) % 3 > 0).astype(np.uint32)
+    posq = np.concatenate([pos, q[:, None]], 1).astype(np.float32)
+    lattice = np.array([L, L, L, 0, 0, 0])
+    part = api.ParticleBuffers(gpu_ctx, posq, np.full(n, 1000.0), lattice, types=types)
+    ff = systems.water_forcefield(grid=(32, 32, 32),
+                                  exclusions=(np.zeros(n + 1, np.uint32),
+                                              np.zeros(0, np.uint32)))
+    field = api.ForceField(gpu_ctx, part, ff)
+    net = make_net(gpu_ctx, scale=2e-3, seed=5)
+    params = net.params.astype(np.float64)
+    target = rng.normal(scale=2e-3, size=(n, 3)).astype(np.float32)
+    dF = net.forward(field)
+    loss, g = net.loss_grad(field, target)
+    D = net.descriptors(field).astype(np.float64)
+    x = posq.astype(np.float64)
+    args = (x[:, :3], x[:, 3], types.astype(np.int64), lattice, R_NN, 2e-3)
+    ref = N.forward(params, *args, D=D, bf16_mode=True)
+    l_ref, g_ref, _ = N.loss_grad(params, *args, target.astype(np.float64), D=D, bf16_mode=True)
+    errs = rel_rms(dF, ref), abs(loss - l_ref) / abs(l_ref), rel_rms(g, g_ref)
+    print(f"{n} atoms: dF {errs[0]:.2e}, loss {errs[1]:.2e}, gradient {errs[2]:.2e}")
+    for h in (net, field, part):
+        h.close()
+    assert errs[0] <= NET_TOL and errs[1] <= 1e-4 and errs[2] <= NET_TOL

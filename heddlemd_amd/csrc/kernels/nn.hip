@@ -8,8 +8,8 @@
 // x_ij = [phi, one-hot(species_i + species_j), D_i, D_j];
 // g_ij = s_out fc(s_ij) (N(x_ij) + N(x_ji)) / 2; dF_i = sum_j g_ij r^_ij.
 //
-// Traversal: the force field's packed half list (one wave per contiguous
-// share of the work list, as the pair kernel).  The network passes compact the in-range
+// Traversal: the force field's packed half list (the pair
+// kernel's).  The network passes compact the in-range
 // pairs of each entry into an LDS queue and evaluate them 32 pairs (64
 // rows: both orientations) at a time:
 //  * layer 1 is Z1^T = W1 X^T and layer 2 Z2^T = W2 H1^T as chains of
@@ -140,6 +140,26 @@ hmd_nn_pack(const NnPackParams p) {
   if (tid == 0u) p.vec[192] = b3[0];
 }
 
+// How the passes share the list: an item is an entry, or one of its
+// 2^split groups of i-sub-clusters, and wave v of n takes the items v, v + n,
+// ...  An entry of a dense liquid holds 0 to 4,096 pairs (about 1,000 on
+// average), so a wave needs several items of different entries before the
+// waves' totals even out: the list is split until there are `want` items (or
+// eight groups an entry).  Whole entries in contiguous shares left a CU with
+// 1.2 of 8 waves running on average at 9,999 atoms.
+struct HmdNnItems {
+  uint32_t n, split;
+  __device__ HmdNnItems(uint32_t entries, uint32_t want) : split(0) {
+    while (split < 3u && (entries << split) < want) ++split;
+    n = entries << split;
+  }
+  __device__ uint32_t entry(uint32_t w) const { return w >> split; }
+  __device__ uint32_t mask(uint32_t w) const {
+    const uint32_t group = 8u >> split;
+    return ((1u << group) - 1u) << (group * (w & ((1u << split) - 1u)));
+  }
+};
+
 // Single-image shift of a cluster (compare jit_composed.rs:1396-1430, as in
 // the pair kernel): valid when every atom within r_cut + r_skin/2 of the
 // cluster lies within half a box of its centre; positions are then moved to
@@ -171,8 +191,7 @@ __device__ inline float4 hmd_nn_apply_shift(float4 a, const HmdNnShift& sh, cons
 }
 
 // ------------------------------------------------------- descriptors ----
-// The pair kernel's traversal: one wave per contiguous share of the work
-// list, lane = j-atom of the entry (shifted once to the image nearest the
+// The pair kernel's traversal: lane = j-atom of the entry (shifted once to the image nearest the
 // i-cluster's centre), the i-atoms broadcast from a per-wave LDS table one
 // per step, over the 8-atom i-sub-clusters the entry's mask admits.  Per
 // pair the 16 basis values come from two exponentials each half (the
@@ -197,11 +216,8 @@ hmd_nn_descriptors(const NnPassParams p) {
   const uint32_t waves_per_block = blockDim.x / HMD_WAVE;
   const uint32_t n_waves = gridDim.x * waves_per_block;
   const uint32_t gw = blockIdx.x * waves_per_block + wv;
-  const uint32_t nw = *p.n_work;
-  const uint32_t per = (nw + n_waves - 1) / n_waves;
-  const uint32_t w0 = gw * per;
-  const uint32_t w1 = min(w0 + per, nw);
-  if (w0 >= w1) return;
+  const HmdNnItems items(__builtin_amdgcn_readfirstlane(*p.n_work), 2u * n_waves);
+  if (gw >= items.n) return;
   const float4* ps = reinterpret_cast<const float4*>(p.posq_sorted);
   const HmdLattice L = p.L;
   long long* acc = p.desc_acc;
@@ -219,8 +235,10 @@ hmd_nn_descriptors(const NnPassParams p) {
       if (vi) hmd_atomic_add_fixed(&acc[k * stride + si], hmd_to_fixed(v, HMD_NN_DESC_SHIFT));
     }
   };
-  for (uint32_t w = w0; w < w1; ++w) {
-    const uint32_t slot = p.work[w];
+  for (uint32_t w = gw; w < items.n; w += n_waves) {
+    const uint32_t slot = __builtin_amdgcn_readfirstlane(p.work[items.entry(w)]);
+    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w);
+    if (pend == 0u) continue;
     const uint32_t c = slot / p.cap_entries;
     const uint32_t c0 = c * HMD_CLUSTER;
     if (c != cur_c) {
@@ -242,7 +260,6 @@ hmd_nn_descriptors(const NnPassParams p) {
     // entries whose j-atoms all lie in later clusters need only the cutoff
     // test (i < j holds); the cluster's own entry also needs i < j
     const bool later = __ballot(valid_j && my_j < c0 + HMD_CLUSTER) == 0ull;
-    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & 0xFFu;
     float dj[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k) dj[k] = 0.0f;
@@ -493,11 +510,8 @@ hmd_nn_forward(const NnPassParams p) {
   const uint32_t wv = threadIdx.x / HMD_WAVE;
   const uint32_t n_waves = gridDim.x * (blockDim.x / HMD_WAVE);
   const uint32_t gw = blockIdx.x * (blockDim.x / HMD_WAVE) + wv;
-  const uint32_t nw = *p.n_work;
-  const uint32_t per = (nw + n_waves - 1) / n_waves;
-  const uint32_t w0 = gw * per;
-  const uint32_t w1 = min(w0 + per, nw);
-  if (w0 >= w1) return;
+  const HmdNnItems items(__builtin_amdgcn_readfirstlane(*p.n_work), 8u * n_waves);
+  if (gw >= items.n) return;
   HmdNnTables& W = Wv[wv];
   long long(*acc)[3][HMD_WAVE] = s_acc[wv];
   const float4* ps = reinterpret_cast<const float4*>(p.posq_sorted);
@@ -529,11 +543,12 @@ hmd_nn_forward(const NnPassParams p) {
   uint32_t cur_c = HMD_SENTINEL, si = 0, n_i = 0;
   bool vi = false;
   HmdNnShift sh{false, 0.0f, 0.0f, 0.0f};
-  for (uint32_t w = w0; w < w1; ++w) {
-    const uint32_t slot = __builtin_amdgcn_readfirstlane(p.work[w]);
+  for (uint32_t w = gw; w < items.n; w += n_waves) {
+    const uint32_t slot = __builtin_amdgcn_readfirstlane(p.work[items.entry(w)]);
+    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w);
+    if (pend == 0u) continue;
     const uint32_t c = slot / p.cap_entries;
     const uint32_t my_j = p.entry_j[(size_t)slot * HMD_ENTRY + lane];
-    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & 0xFFu;
     hmd_wave_sync();
     if (c != cur_c) {
       if (cur_c != HMD_SENTINEL) {
@@ -786,10 +801,7 @@ hmd_nn_backward(const NnPassParams p) {
   const uint32_t wv = threadIdx.x / HMD_WAVE;
   const uint32_t n_waves = gridDim.x * (blockDim.x / HMD_WAVE);
   const uint32_t gw = blockIdx.x * (blockDim.x / HMD_WAVE) + wv;
-  const uint32_t nw = *p.n_work;
-  const uint32_t per = (nw + n_waves - 1) / n_waves;
-  const uint32_t w0 = gw * per;
-  const uint32_t w1 = min(w0 + per, nw);
+  const HmdNnItems items(__builtin_amdgcn_readfirstlane(*p.n_work), 8u * n_waves);
   HmdNnWave& W = Wv[wv];
   const float4* ps = reinterpret_cast<const float4*>(p.posq_sorted);
   if (lane < 32u) W.xin[lane][3] = __builtin_bit_cast(hmd_bf16x8, hmd_u32x4{0u, 0u, 0u, 0u});
@@ -806,11 +818,12 @@ hmd_nn_backward(const NnPassParams p) {
 
   uint32_t cur_c = HMD_SENTINEL, n_i = 0;
   HmdNnShift sh{false, 0.0f, 0.0f, 0.0f};
-  for (uint32_t w = w0; w < w1; ++w) {
-    const uint32_t slot = __builtin_amdgcn_readfirstlane(p.work[w]);
+  for (uint32_t w = gw; w < items.n; w += n_waves) {
+    const uint32_t slot = __builtin_amdgcn_readfirstlane(p.work[items.entry(w)]);
+    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w);
+    if (pend == 0u) continue;
     const uint32_t c = slot / p.cap_entries;
     const uint32_t my_j = p.entry_j[(size_t)slot * HMD_ENTRY + lane];
-    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & 0xFFu;
     hmd_wave_sync();
     if (c != cur_c) {
       cur_c = c;

@@ -52,6 +52,14 @@ void Scanner::run(Context& c, const uint32_t* in, uint32_t* out,
   launch(c, K_hmd_scan_add, tiles, 1024, 0, p3);
 }
 
+uint32_t Scanner::run_tiles(Context& c, const uint32_t* in, uint32_t* out, const uint32_t* gate,
+                            uint32_t gate_mask) {
+  const uint32_t tiles = ceil_div(len, 4096);
+  ScanParams p{in, out, tile_sums.ptr, len, gate, gate_mask, 0u};
+  launch(c, K_hmd_scan_tiles, tiles, 1024, 0, p);
+  return tiles;
+}
+
 double reduce_f64(Context& c, Particles& p, const float* x, uint32_t mode) {
   const uint32_t blocks = p.red_partials.count;
   ReduceParams r{};

@@ -382,6 +382,7 @@ void ForceField::make_side_stream() {
   check(hipStreamCreateWithFlags(&side, hipStreamNonBlocking), "hipStreamCreate");
   check(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming), "hipEventCreate");
   check(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming), "hipEventCreate");
+  check(hipEventCreateWithFlags(&ev_binned, hipEventDisableTiming), "hipEventCreate");
 }
 
 // The box requirement (r_c below half of every perpendicular width) and
@@ -456,6 +457,7 @@ void ForceField::init_neighbor_list(const hmd_forcefield_desc& d) {
   atom_key.alloc(n);
   cell_count.alloc(n_keys);
   cell_start.alloc(n_keys + 1);
+  cell_list.alloc(n);
   sorted_id.alloc(n_pad);
   slot_of.alloc(n);
   type_sorted.alloc(n_pad);
@@ -675,6 +677,7 @@ ForceField::~ForceField() {
   if (side) (void)hipStreamSynchronize(side);
   if (ev_fork) (void)hipEventDestroy(ev_fork);
   if (ev_join) (void)hipEventDestroy(ev_join);
+  if (ev_binned) (void)hipEventDestroy(ev_binned);
   if (side) (void)hipStreamDestroy(side);
 }
 
@@ -707,29 +710,40 @@ void ForceField::rebuild_chain() {
 // positions (every step).
 void ForceField::rebuild_sort() {
   const uint32_t* gate = status.ptr;
-  const HmdLattice L = p.lattice;
-  NblKeyParams kp{p.posq.ptr, n, L, g[0], g[1], g[2], grid_bits, atom_key.ptr, cell_count.ptr,
-                  cell_start.ptr, sorted_id.ptr, gate};
-  launch(c, K_hmd_nbl_keys, ceil_div(n, 256), 256, 0, kp);
-  cell_scan.run(c, cell_count.ptr, cell_start.ptr, gate, HMD_STATUS_DISPLACED);
-  launch(c, K_hmd_nbl_scatter, ceil_div(n, 256), 256, 0, kp);
-  NblSortParams sp{cell_start.ptr, n_keys, sorted_id.ptr, gate};
-  launch(c, K_hmd_nbl_sort_cells, ceil_div(n_keys, 256), 256, 0, sp);
+  NblKeyParams kp{p.posq.ptr, n, p.lattice, g[0], g[1], g[2], grid_bits, atom_key.ptr,
+                  cell_count.ptr, cell_start.ptr, n_keys, 0u, cell_scan.tile_sums.ptr,
+                  cell_list.ptr, sorted_id.ptr, slot_of.ptr, gate};
+  // One workgroup sorts a system whose cells and ids fit its LDS and whose
+  // atoms are few per thread (kNblSortSmall); beyond that the four launches
+  // win on the steps that do rebuild.
+  const size_t small_lds = 4 * (size_t)((n_keys + 255u) & ~255u) + 2 * (size_t)((n + 3u) & ~3u);
+  if (n <= kNblSortSmall && small_lds + 64 <= c.max_lds) {
+    if (n > kNblKeysInline) {   // the keys' arithmetic is too much for one CU
+      kp.cell_count = nullptr;
+      launch(c, K_hmd_nbl_keys, ceil_div(n, 256), 256, 0, kp);
+    }
+    launch(c, K_hmd_nbl_sort_small, 1, 1024, small_lds, kp);
+  } else {
+    launch(c, K_hmd_nbl_keys, ceil_div(n, 256), 256, 0, kp);
+    if (n_keys <= 256u * 4096u)
+      kp.n_tiles = cell_scan.run_tiles(c, cell_count.ptr, cell_start.ptr, gate,
+                                       HMD_STATUS_DISPLACED);
+    else
+      cell_scan.run(c, cell_count.ptr, cell_start.ptr, gate, HMD_STATUS_DISPLACED);
+    launch(c, K_hmd_nbl_scatter, ceil_div(n, 256), 256, 0, kp);
+    launch(c, K_hmd_nbl_rank, ceil_div(n, 256), 256, 0, kp);
+  }
   NblGatherParams gp{p.posq.ptr, p.type.ptr, n, n_pad, sorted_id.ptr, slot_of.ptr,
                      posq_sorted.ptr, type_sorted.ptr, ref_pos.ptr, gate, p.lattice,
-                     image_sorted.ptr};
+                     image_sorted.ptr, bbox.ptr, sub_bbox.ptr, excl_off.ptr, excl_par.ptr,
+                     excl_slot.ptr};
   launch(c, K_hmd_nbl_gather, ceil_div(n_pad, 256), 256, 0, gp);
 }
 
-// Cluster boxes, the cluster-pair list and the work list (gated on a
-// rebuild).
+// The cluster-pair list and the work list (gated on a rebuild).
 void ForceField::rebuild_list() {
   const uint32_t* gate = status.ptr;
   const HmdLattice L = p.lattice;
-  NblBboxParams bp{posq_sorted.ptr, n, n_clusters, bbox.ptr, sub_bbox.ptr, gate,
-                   sorted_id.ptr, slot_of.ptr, excl_off.ptr, excl_par.ptr,
-                   excl_slot.ptr, n_pad};
-  launch(c, K_hmd_nbl_bbox, ceil_div(n_clusters, 4), 256, 0, bp);
   NblBuildParams bd{};
   bd.posq_sorted = posq_sorted.ptr;
   bd.sorted_id = sorted_id.ptr;
@@ -761,11 +775,13 @@ void ForceField::rebuild_list() {
 #endif
   launch(c, K_hmd_nbl_build, n_clusters, 64 * HMD_NBL_WAVES, chunk_lds + (size_t)bd.lds_slots * 4,
          bd);
-  entry_scan.run(c, entry_count.ptr, entry_offset.ptr, gate, HMD_STATUS_DISPLACED);
-  NblWorkParams wp{entry_count.ptr, entry_offset.ptr, n_clusters, cap_entries,
+  // up to kNblCountInline clusters every workgroup of the work-list kernel adds
+  // up the counts below its own (16 KB at most); beyond, they are scanned
+  const bool scan = n_clusters > kNblCountInline;
+  if (scan) entry_scan.run(c, entry_count.ptr, entry_offset.ptr, gate, HMD_STATUS_DISPLACED);
+  NblWorkParams wp{entry_count.ptr, scan ? entry_offset.ptr : nullptr, n_clusters, cap_entries,
                    work.ptr, n_work.ptr, status.ptr};
   launch(c, K_hmd_nbl_worklist, ceil_div(n_clusters, 4u), 256, 0, wp);
-  launch(c, K_hmd_nbl_close, 1, 64, 0, wp);
 }
 
 NblDispParams ForceField::disp_params() const {
@@ -881,7 +897,7 @@ void ForceField::pair_forces(bool fev) {
   c.mark("pair_force");
 }
 
-void ForceField::spme_forces(bool fev) {
+void ForceField::spme_forces(bool fev, bool mark_binned) {
   const HmdLattice L = p.lattice;
   const uint32_t n0 = grid[0], n1 = grid[1], n2 = grid[2];
   SpmeBinParams bp{p.posq.ptr, sorted_id.ptr, n, L, n0, n1, n2, brick[0], brick[1], brick[2],
@@ -891,6 +907,7 @@ void ForceField::spme_forces(bool fev) {
   bin_scan.run(c, bin_count.ptr, bin_start.ptr, nullptr, 0);
   launch(c, K_hmd_spme_bin_scatter, ceil_div(n, 256), 256, 0, bp);
   c.mark("spme_bin");
+  if (mark_binned) check(hipEventRecord(ev_binned, c.stream), "hipEventRecord");
 
   SpmeSpreadParams sp{p.posq.ptr, n, L, n0, n1, n2, brick[0], brick[1], brick[2],
                       nb[0], nb[1], nb[2], bin_start.ptr, bin_atoms.ptr, rho.ptr};
@@ -1056,12 +1073,20 @@ void ForceField::compute(int level, bool displacement_checked) {
   // combines after the join: the result is the same bytes either way.  Not
   // while recording a batched replica step or marking per-stage events.
   const bool fork = spme_on && spme_stream && side && !c.rec && !c.profiling;
+  // The force-only pair kernel fills the LDS of every CU (five workgroups of
+  // 30 KB) from a queue of thousands: started before the spread's workgroups
+  // are placed, it holds them off and SPME's chain of launches ends last.  So
+  // it waits until SPME has binned its atoms (196,608 atoms: 13.0 -> 12.3 ms
+  // per 25 steps, 24,576: 3.89 -> 3.75).  The energy variant leaves room (three
+  // of 50 KB) and does not wait (39,993 atoms: 4.12 ms per 20 steps, 4.30
+  // waiting).
+  const bool gate_pair = fork && !fev;
   auto fork_spme = [&]() {
     check(hipEventRecord(ev_fork, c.stream), "hipEventRecord");
     check(hipStreamWaitEvent(side, ev_fork, 0), "hipStreamWaitEvent");
     std::swap(c.stream, side);
     try {
-      spme_forces(fev);
+      spme_forces(fev, gate_pair);
     } catch (...) {
       std::swap(c.stream, side);
       throw;
@@ -1071,6 +1096,7 @@ void ForceField::compute(int level, bool displacement_checked) {
   };
   if (fork) neighbor_pre_step(fork_spme, displacement_checked);
   else neighbor_pre_step({}, displacement_checked);
+  if (gate_pair) check(hipStreamWaitEvent(c.stream, ev_binned, 0), "hipStreamWaitEvent");
   pair_forces(fev);
   bonded_forces(fev);
   if (spme_on && !fork) spme_forces(fev);

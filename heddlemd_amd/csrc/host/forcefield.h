@@ -30,6 +30,16 @@ constexpr size_t kNblBuildStaticLds = 24576;
 // 415-445): grow by 1.5x, and grow ahead of any dropped entry once a build
 // fills more than 0.8 of the capacity.
 constexpr double kNblGrowth = 1.5;
+// Atoms up to which one workgroup does the cell sort of a rebuild, and up to
+// which it also computes the keys.  On a step without a rebuild a launch less
+// saves about 2 us (argon 10,000 with the other merged launches: 57 -> 46 us a
+// step); on one with a rebuild the one workgroup takes as long as the launches
+// it replaces, but for the keys of many atoms (8,997: 27 us with them, half of
+// it theirs).  Beyond, 16-bit ids and counts no longer fit the LDS.
+constexpr uint32_t kNblSortSmall = 12288;
+constexpr uint32_t kNblKeysInline = 5120;
+// Clusters up to which the work-list kernel adds up the entry counts itself.
+constexpr uint32_t kNblCountInline = 4096;
 constexpr double kNblFillThreshold = 0.8;
 
 struct ForceField {
@@ -77,7 +87,7 @@ struct ForceField {
   // SPME enqueued on a second stream beside the pair kernel (fork / join)
   uint32_t spme_stream = 1;
   hipStream_t side = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_binned = nullptr;
   void make_side_stream();
   // Launch-shape autotuner: times candidate pair grids, FFT grids and SPME
   // bricks on this system and keeps the fastest; set_tuning applies a
@@ -104,7 +114,7 @@ struct ForceField {
   uint32_t n_keys = 1, n_clusters = 0, n_pad = 0, cap_entries = 0;
   uint32_t lds_entries = 0;         // list entries staged in LDS (0: as many as fit)
   DevBuf<uint32_t> status;          // [0] flags [1] generation [2] high water
-  DevBuf<uint32_t> atom_key, cell_count, cell_start, sorted_id, slot_of, type_sorted;
+  DevBuf<uint32_t> atom_key, cell_count, cell_start, cell_list, sorted_id, slot_of, type_sorted;
   DevBuf<float> posq_sorted, ref_pos, bbox, sub_bbox;
   DevBuf<int32_t> image_sorted;   // int4[n_pad]
   DevBuf<uint32_t> entry_j, entry_mask, entry_count, entry_offset, work, n_work;
@@ -188,7 +198,7 @@ struct ForceField {
                          bool displacement_checked = false);
   NblDispParams disp_params() const;
   void pair_forces(bool fev);
-  void spme_forces(bool fev);
+  void spme_forces(bool fev, bool mark_binned = false);
   // One force evaluation, enqueued only (no host synchronisation): safe to
   // capture into a graph.
   // displacement_checked: the caller's kernel has already run the skin

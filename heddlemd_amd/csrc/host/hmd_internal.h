@@ -18,8 +18,8 @@
 #define HMD_KERNEL_LIST(X)                                                   \
   X(hmd_scan_tiles) X(hmd_scan_add)                                          \
   X(hmd_nbl_displacement) X(hmd_nbl_keys) X(hmd_nbl_scatter)                 \
-  X(hmd_nbl_sort_cells) X(hmd_nbl_gather) X(hmd_nbl_bbox) X(hmd_nbl_build)   \
-  X(hmd_nbl_worklist) X(hmd_nbl_close) X(hmd_nbl_pairs)                     \
+  X(hmd_nbl_rank) X(hmd_nbl_sort_small) X(hmd_nbl_gather) X(hmd_nbl_build)   \
+  X(hmd_nbl_worklist) X(hmd_nbl_pairs)                                       \
   X(hmd_pair_force_f) X(hmd_pair_force_fev) X(hmd_pair_force_lj_f)           \
   X(hmd_pair_force_lj_fev) X(hmd_pair_force_coul_f) X(hmd_pair_force_coul_fev)\
   X(hmd_pair_finalize) X(hmd_pair_scaled) X(hmd_slot_add)                   \
@@ -196,6 +196,10 @@ struct Scanner {
   void init(uint32_t len_);
   void run(Context& c, const uint32_t* in, uint32_t* out, const uint32_t* gate,
            uint32_t gate_mask);
+  // Within 4,096-element tiles only, the tiles' totals in tile_sums; returns
+  // the number of tiles.
+  uint32_t run_tiles(Context& c, const uint32_t* in, uint32_t* out, const uint32_t* gate,
+                     uint32_t gate_mask);
 };
 
 }  // namespace hmd

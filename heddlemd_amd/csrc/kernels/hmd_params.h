@@ -67,48 +67,35 @@ struct NblKeyParams {
   uint32_t g0, g1, g2;      // fine cells per axis (2^bits each)
   uint32_t bits;
   uint32_t* atom_key;       // [n]
-  uint32_t* cell_count;     // [n_keys]  (zero on entry, zero again after scatter)
-  const uint32_t* cell_start;  // [n_keys+1] (scatter only)
-  uint32_t* sorted_id;      // [n_pad]   (scatter only)
+  uint32_t* cell_count;     // [n_keys]  (zero on entry, zero again after scatter), or null
+  const uint32_t* cell_start;  // [n_keys+1]; within the 4,096-cell tile if n_tiles
+  uint32_t n_keys;
+  uint32_t n_tiles;            // tile totals to add to cell_start (at most 256), or 0
+  const uint32_t* tile_sums;   // [n_tiles]
+  uint32_t* cell_list;      // [n] ids by cell, in any order within a cell
+  uint32_t* sorted_id;      // [n_pad]
+  uint32_t* slot_of;        // [n]
   const uint32_t* status;   // rebuild gate
 };
-
-struct NblSortParams {
-  const uint32_t* cell_start;
-  uint32_t n_keys;
-  uint32_t* sorted_id;
-  const uint32_t* status;
-};
-
 struct NblGatherParams {
   const float* posq;        // canonical float4[n]
   const uint32_t* type;     // canonical [n]
   uint32_t n, n_pad;
-  const uint32_t* sorted_id;   // [n_pad] (pad entries written here)
-  uint32_t* slot_of;        // [n]
+  const uint32_t* sorted_id;   // [n_pad]
+  const uint32_t* slot_of;  // [n]
   float* posq_sorted;       // float4[n_pad]
   uint32_t* type_sorted;    // [n_pad]
   float* ref_pos;           // float4[n] canonical positions at rebuild
   const uint32_t* status;   // rebuild extras gated on the DISPLACED bit
   HmdLattice L;
   int32_t* image;           // int4[n_pad]: lattice images removed at the rebuild
-};
-
-struct NblBboxParams {
-  const float* posq_sorted;
-  uint32_t n;
-  uint32_t n_clusters;
   float* bbox;              // float4[2*n_clusters]: (cx,cy,cz,-), (hx,hy,hz,-)
   float* sub_bbox;          // float4[16*n_clusters]: 8 sub-cluster boxes
-  const uint32_t* status;
   // exclusion partners as sorted slots, for the list build: slot s's m-th
   // partner (canonical CSR order, at most 8) at excl_slot[m * n_pad + s]
-  const uint32_t* sorted_id;
-  const uint32_t* slot_of;
   const uint32_t* excl_offsets;   // canonical CSR [n+1]
   const uint32_t* excl_partners;
   uint32_t* excl_slot;            // [8][n_pad], sentinel-filled
-  uint32_t n_pad;
 };
 
 struct NblBuildParams {
@@ -130,18 +117,18 @@ struct NblBuildParams {
   uint64_t* entry_excl;        // [n_clusters*cap_entries*64]
   uint32_t* entry_count;       // [n_clusters] (entries written / needed)
   uint32_t* excl_entries;      // [n_clusters] leading entries with masks
-  const uint32_t* excl_slot;   // [8][n_pad] partners' sorted slots (hmd_nbl_bbox)
+  const uint32_t* excl_slot;   // [8][n_pad] partners' sorted slots (hmd_nbl_gather)
   uint32_t n_pad;
   uint32_t* status;
 };
 
 struct NblWorkParams {
   const uint32_t* entry_count;   // [n_clusters]
-  const uint32_t* entry_offset;  // [n_clusters+1] exclusive scan
+  const uint32_t* entry_offset;  // [n_clusters+1] exclusive scan, or null
   uint32_t n_clusters, cap_entries;
   uint32_t* work;                // [total]
   uint32_t* n_work;              // [1]
-  uint32_t* status;              // [0] flags, [1] generation, [2] high water
+  uint32_t* status;              // [0] flags, [1] generation, [2] high water, [3] ticket
 };
 
 struct NblDispParams {

@@ -107,6 +107,16 @@ __device__ __forceinline__ void hmd_nbl_displacement_body(const NblDispParams& p
 }
 HMD_KERNEL(hmd_nbl_displacement, NblDispParams, 256)
 
+// Inclusive prefix sum over the 64 lanes.
+__device__ inline uint32_t hmd_wave_scan_incl(uint32_t v, uint32_t lane) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t t = (uint32_t)__shfl_up((int)v, (unsigned)o, HMD_WAVE);
+    if (lane >= (uint32_t)o) v += t;
+  }
+  return v;
+}
+
 // Fine-cell Hilbert key + histogram.
 __device__ __forceinline__ void hmd_nbl_keys_body(const NblKeyParams& p, const uint32_t hmd_bx,
     const uint32_t hmd_gx) {
@@ -118,108 +128,177 @@ __device__ __forceinline__ void hmd_nbl_keys_body(const NblKeyParams& p, const u
   hmd_fine_cell(a.x, a.y, a.z, p.L, p.g0, p.g1, p.g2, c0, c1, c2);
   const uint32_t key = hmd_hilbert3(c0, c1, c2, p.bits);
   p.atom_key[i] = key;
-  atomicAdd(&p.cell_count[key], 1u);
+  if (p.cell_count) atomicAdd(&p.cell_count[key], 1u);   // else counted by hmd_nbl_sort_small
 }
 HMD_KERNEL(hmd_nbl_keys, NblKeyParams, 256)
 
+// Exclusive prefix of up to 256 scan-tile totals into s_off, by the 256
+// threads of the workgroup: the second level of the cell scan, taken by every
+// workgroup of the kernels that read the scan instead of by two launches of
+// their own (a gated launch costs a step without a rebuild about 2 us).
+__device__ inline void hmd_nbl_tile_offsets(const NblKeyParams& p, uint32_t* s_off,
+                                            uint32_t* s_wave) {
+  const uint32_t t = threadIdx.x, lane = hmd_lane();
+  const uint32_t v = t < p.n_tiles ? p.tile_sums[t] : 0u;
+  const uint32_t incl = hmd_wave_scan_incl(v, lane);
+  if (lane == HMD_WAVE - 1) s_wave[t / HMD_WAVE] = incl;
+  __syncthreads();
+  uint32_t off = incl - v;
+  for (uint32_t w = 0; w < t / HMD_WAVE; ++w) off += s_wave[w];
+  s_off[t] = off;
+  __syncthreads();
+}
+
 // Scatter into cells.  The count array doubles as the cursor and is driven
 // back to zero, ready for the next rebuild.  Order inside a cell is fixed
-// afterwards by hmd_nbl_sort_cells.
+// afterwards by hmd_nbl_rank.
 __device__ __forceinline__ void hmd_nbl_scatter_body(const NblKeyParams& p, const uint32_t hmd_bx,
     const uint32_t hmd_gx) {
   if (!hmd_gate(p.status, HMD_STATUS_DISPLACED)) return;
+  __shared__ uint32_t s_off[256], s_wave[4];
+  if (p.n_tiles) hmd_nbl_tile_offsets(p, s_off, s_wave);
   uint32_t i = hmd_bx * blockDim.x + threadIdx.x;
   if (i >= p.n) return;
-  uint32_t key = p.atom_key[i];
-  uint32_t k = atomicSub(&p.cell_count[key], 1u) - 1u;
-  p.sorted_id[p.cell_start[key] + k] = i;
+  const uint32_t key = p.atom_key[i];
+  const uint32_t k = atomicSub(&p.cell_count[key], 1u) - 1u;
+  p.cell_list[p.cell_start[key] + (p.n_tiles ? s_off[key >> 12] : 0u) + k] = i;
 }
 HMD_KERNEL(hmd_nbl_scatter, NblKeyParams, 256)
 
-// Canonical (cell, atom id) order: insertion sort inside each fine cell
-// (a cell holds a couple of atoms; compare kernels/neighbor.cu:218-238).
-__device__ __forceinline__ void hmd_nbl_sort_cells_body(const NblSortParams& p, const uint32_t hmd_bx,
+// Canonical (cell, atom id) order (compare kernels/neighbor.cu:218-238): an
+// atom's slot is its cell's start plus the number of lower ids in the cell
+// (a cell holds a couple of atoms).
+__device__ __forceinline__ void hmd_nbl_rank_body(const NblKeyParams& p, const uint32_t hmd_bx,
     const uint32_t hmd_gx) {
   if (!hmd_gate(p.status, HMD_STATUS_DISPLACED)) return;
-  uint32_t c = hmd_bx * blockDim.x + threadIdx.x;
-  if (c >= p.n_keys) return;
-  uint32_t s = p.cell_start[c], e = p.cell_start[c + 1];
-  for (uint32_t k = s + 1; k < e; ++k) {
-    uint32_t key = p.sorted_id[k];
-    uint32_t pos = k;
-    while (pos > s && p.sorted_id[pos - 1] > key) {
-      p.sorted_id[pos] = p.sorted_id[pos - 1];
-      --pos;
-    }
-    p.sorted_id[pos] = key;
-  }
+  __shared__ uint32_t s_off[256], s_wave[4];
+  if (p.n_tiles) hmd_nbl_tile_offsets(p, s_off, s_wave);
+  uint32_t i = hmd_bx * blockDim.x + threadIdx.x;
+  if (i >= p.n) return;
+  const uint32_t key = p.atom_key[i], nx = key + 1u;
+  const uint32_t beg = p.cell_start[key] + (p.n_tiles ? s_off[key >> 12] : 0u);
+  const uint32_t end =
+      nx < p.n_keys ? p.cell_start[nx] + (p.n_tiles ? s_off[nx >> 12] : 0u) : p.n;
+  uint32_t s = beg;
+  for (uint32_t k = beg; k < end; ++k) s += p.cell_list[k] < i ? 1u : 0u;
+  p.sorted_id[s] = i;
+  p.slot_of[i] = s;
 }
-HMD_KERNEL(hmd_nbl_sort_cells, NblSortParams, 256)
+HMD_KERNEL(hmd_nbl_rank, NblKeyParams, 256)
 
-// Sorted views.  Every step it refreshes the sorted positions
-// (kernels/neighbor.cu:251-285 does the same refresh every step in
-// ForceField::run); in a rebuilding step it also writes the inverse map, the
-// sorted types, the rebuild-time reference positions and the padding lanes.
-// The sorted positions carry the lattice images that the rebuild's cell
-// assignment removed (hmd_wrap of the rebuild-time position, kept per slot
-// and applied every step with the same operations): at the rebuild they are
-// the wrapped positions the cells were taken from, so every cluster's box is
-// compact even for atoms that a constraint step left just outside the primary
-// cell, and between rebuilds they move continuously.
-__device__ __forceinline__ void hmd_nbl_gather_body(const NblGatherParams& p, const uint32_t hmd_bx,
-    const uint32_t hmd_gx) {
-#pragma clang fp contract(off)
-  const bool rebuild = hmd_gate(p.status, HMD_STATUS_DISPLACED);
-  uint32_t s = hmd_bx * blockDim.x + threadIdx.x;
-  if (s >= p.n_pad) return;
-  float4* ps = reinterpret_cast<float4*>(p.posq_sorted);
-  if (s >= p.n) {
-    if (rebuild) {
-      // Padding lanes: far away and uncharged; their slots never pass the
-      // validity test of the force kernel.
-      ps[s] = make_float4(1.0e18f, 1.0e18f, 1.0e18f, 0.0f);
-      p.type_sorted[s] = 0u;
+// The whole cell sort of a small system in one workgroup: keys (unless
+// hmd_nbl_keys has written them: cell_count null), histogram, scan, scatter
+// and ranks through LDS (cell counts, then starts, then cursors; the
+// unordered cell lists as 16-bit ids).  The order is that of
+// the four kernels above.  What it saves is launches: on a step without a
+// rebuild each of the four (six with a two-level scan) costs about 2 us.
+__device__ __forceinline__ void hmd_nbl_sort_small_body(const NblKeyParams& p,
+                                                        const uint32_t hmd_bx,
+                                                        const uint32_t hmd_gx) {
+  if (!hmd_gate(p.status, HMD_STATUS_DISPLACED)) return;
+  extern __shared__ uint32_t s_cells[];
+  __shared__ uint32_t s_wave[16];
+  // cells of a wave's share: a multiple of the 256 it scans at a time
+  const uint32_t share = max(256u, p.n_keys >> 4);      // a power of two
+  const uint32_t sh = 31u - (uint32_t)__builtin_clz(share);
+  const uint32_t n_pad_keys = (p.n_keys + 255u) & ~255u;
+  uint16_t* s_list = reinterpret_cast<uint16_t*>(s_cells + n_pad_keys);
+  const uint32_t t = threadIdx.x, lane = hmd_lane(), wave = t / HMD_WAVE;
+  for (uint32_t k = t; k < n_pad_keys / 4; k += blockDim.x)
+    reinterpret_cast<uint4*>(s_cells)[k] = make_uint4(0u, 0u, 0u, 0u);
+  __syncthreads();
+  // four atoms a thread at a time: their loads are in flight together
+  constexpr uint32_t U = 4u;
+  if (!p.cell_count) {
+    for (uint32_t i0 = t; i0 < p.n; i0 += U * 1024u) {
+      uint32_t key[U];
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) key[u] = p.atom_key[min(i0 + 1024u * u, p.n - 1u)];
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u)
+        if (i0 + 1024u * u < p.n) atomicAdd(&s_cells[key[u]], 1u);
     }
-    return;
   }
-  uint32_t id = p.sorted_id[s];
-  const float4 a = reinterpret_cast<const float4*>(p.posq)[id];
-  int4* img = reinterpret_cast<int4*>(p.image);
-  int4 im;
-  if (rebuild) {
-    float x = a.x, y = a.y, z = a.z;
-    hmd_wrap(x, y, z, im.x, im.y, im.z, p.L);
-    im.w = 0;
-    img[s] = im;
-    p.slot_of[id] = s;
-    p.type_sorted[s] = p.type[id];
-    reinterpret_cast<float4*>(p.ref_pos)[id] = a;
-  } else {
-    im = img[s];
+  for (uint32_t i0 = t; p.cell_count && i0 < p.n; i0 += U * 1024u) {
+    float4 a[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u)
+      a[u] = reinterpret_cast<const float4*>(p.posq)[min(i0 + 1024u * u, p.n - 1u)];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      const uint32_t i = i0 + 1024u * u;
+      if (i >= p.n) break;
+      uint32_t c0, c1, c2;
+      hmd_fine_cell(a[u].x, a[u].y, a[u].z, p.L, p.g0, p.g1, p.g2, c0, c1, c2);
+      const uint32_t key = hmd_hilbert3(c0, c1, c2, p.bits);
+      p.atom_key[i] = key;                  // read back by this thread alone
+      atomicAdd(&s_cells[key], 1u);
+    }
   }
-  const float ka = (float)im.x, kb = (float)im.y, kc = (float)im.z;
-  float4 w = a;
-  w.x -= ka * p.L.lx + kb * p.L.xy + kc * p.L.xz;
-  w.y -= kb * p.L.ly + kc * p.L.yz;
-  w.z -= kc * p.L.lz;
-  ps[s] = w;
+  __syncthreads();
+  // exclusive scan of each wave's share, four cells a lane
+  uint32_t run = 0;
+  for (uint32_t b = wave * share; b < min((wave + 1u) * share, n_pad_keys); b += 256u) {
+    uint4* q = reinterpret_cast<uint4*>(s_cells + b) + lane;
+    const uint4 v = *q;
+    const uint32_t sum = v.x + v.y + v.z + v.w;
+    const uint32_t incl = hmd_wave_scan_incl(sum, lane);
+    const uint32_t e = run + incl - sum;
+    *q = make_uint4(e, e + v.x, e + v.x + v.y, e + v.x + v.y + v.z);
+    run += hmd_readlane(incl, HMD_WAVE - 1);
+  }
+  if (lane == 0) s_wave[wave] = run;
+  __syncthreads();
+  if (t < 16u) {
+    uint32_t off = 0;
+    for (uint32_t w = 0; w < t; ++w) off += s_wave[w];
+    __builtin_amdgcn_wave_barrier();
+    s_wave[t] = off;                        // one wave, reads before writes
+  }
+  __syncthreads();
+  for (uint32_t i0 = t; i0 < p.n; i0 += U * 1024u) {
+    uint32_t key[U], at[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) key[u] = p.atom_key[min(i0 + 1024u * u, p.n - 1u)];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u)
+      at[u] = i0 + 1024u * u < p.n ? atomicAdd(&s_cells[key[u]], 1u) + s_wave[key[u] >> sh] : 0u;
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u)
+      if (i0 + 1024u * u < p.n) s_list[at[u]] = (uint16_t)(i0 + 1024u * u);
+  }
+  __syncthreads();
+  // the cursors now hold each cell's end, which is the next one's start
+  for (uint32_t i0 = t; i0 < p.n; i0 += U * 1024u) {
+    uint32_t key[U], beg[U], end[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) key[u] = p.atom_key[min(i0 + 1024u * u, p.n - 1u)];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      end[u] = s_cells[key[u]] + s_wave[key[u] >> sh];
+      beg[u] = key[u] ? s_cells[key[u] - 1u] + s_wave[(key[u] - 1u) >> sh] : 0u;
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      const uint32_t i = i0 + 1024u * u;
+      if (i >= p.n) break;
+      uint32_t s = beg[u];
+      for (uint32_t k = beg[u]; k < end[u]; ++k) s += s_list[k] < i ? 1u : 0u;
+      p.sorted_id[s] = i;
+      p.slot_of[i] = s;
+    }
+  }
 }
-HMD_KERNEL(hmd_nbl_gather, NblGatherParams, 256)
+HMD_KERNEL(hmd_nbl_sort_small, NblKeyParams, 1024)
 
 // Per-cluster axis-aligned bounding box (centre and half extents) of the
 // valid atoms, one wave per cluster (compare compute_block_bbox,
 // kernels/neighbor.cu:291-361), plus the boxes of the cluster's eight
 // 8-atom sub-clusters (consecutive sorted atoms) against which the list build
 // tests each j-atom.
-__device__ __forceinline__ void hmd_nbl_bbox_body(const NblBboxParams& p, const uint32_t hmd_bx,
-    const uint32_t hmd_gx) {
-  if (!hmd_gate(p.status, HMD_STATUS_DISPLACED)) return;
-  uint32_t c = hmd_bx * (blockDim.x / HMD_WAVE) + threadIdx.x / HMD_WAVE;
-  if (c >= p.n_clusters) return;
-  uint32_t lane = hmd_lane();
-  uint32_t s = c * HMD_CLUSTER + lane;
-  bool valid = s < p.n;
-  float4 a = reinterpret_cast<const float4*>(p.posq_sorted)[s];
+__device__ inline void hmd_nbl_boxes(const NblGatherParams& p, uint32_t s, bool valid, float4 a,
+                                     uint32_t lane) {
+  const uint32_t c = s / HMD_CLUSTER;
   float lo[3] = {valid ? a.x : 3.0e38f, valid ? a.y : 3.0e38f, valid ? a.z : 3.0e38f};
   float hi[3] = {valid ? a.x : -3.0e38f, valid ? a.y : -3.0e38f, valid ? a.z : -3.0e38f};
   float4* sub = reinterpret_cast<float4*>(p.sub_bbox);
@@ -245,12 +324,62 @@ __device__ __forceinline__ void hmd_nbl_bbox_body(const NblBboxParams& p, const 
     b[2 * c + 1] = make_float4(0.5f * (hi[0] - lo[0]), 0.5f * (hi[1] - lo[1]),
                                0.5f * (hi[2] - lo[2]), 0.0f);
   }
+}
+
+// Sorted views.  Every step it refreshes the sorted positions
+// (kernels/neighbor.cu:251-285 does the same refresh every step in
+// ForceField::run); in a rebuilding step it also writes the
+// sorted types, the rebuild-time reference positions, the padding lanes, the
+// cluster boxes (a wave holds one cluster) and the exclusion partners' slots.
+// The sorted positions carry the lattice images that the rebuild's cell
+// assignment removed (hmd_wrap of the rebuild-time position, kept per slot
+// and applied every step with the same operations): at the rebuild they are
+// the wrapped positions the cells were taken from, so every cluster's box is
+// compact even for atoms that a constraint step left just outside the primary
+// cell, and between rebuilds they move continuously.
+__device__ __forceinline__ void hmd_nbl_gather_body(const NblGatherParams& p, const uint32_t hmd_bx,
+    const uint32_t hmd_gx) {
+#pragma clang fp contract(off)
+  const bool rebuild = hmd_gate(p.status, HMD_STATUS_DISPLACED);
+  const uint32_t s = hmd_bx * blockDim.x + threadIdx.x;
+  if (s >= p.n_pad) return;                 // whole waves
+  const bool valid = s < p.n;
+  if (!valid && !rebuild) return;
+  float4* ps = reinterpret_cast<float4*>(p.posq_sorted);
+  // Padding lanes: far away and uncharged; their slots never pass the
+  // validity test of the force kernel.
+  float4 w = make_float4(1.0e18f, 1.0e18f, 1.0e18f, 0.0f);
+  uint32_t id = 0, ty = 0;
+  if (valid) {
+    id = p.sorted_id[s];
+    const float4 a = reinterpret_cast<const float4*>(p.posq)[id];
+    int4* img = reinterpret_cast<int4*>(p.image);
+    int4 im;
+    if (rebuild) {
+      float x = a.x, y = a.y, z = a.z;
+      hmd_wrap(x, y, z, im.x, im.y, im.z, p.L);
+      im.w = 0;
+      img[s] = im;
+      ty = p.type[id];
+      reinterpret_cast<float4*>(p.ref_pos)[id] = a;
+    } else {
+      im = img[s];
+    }
+    const float ka = (float)im.x, kb = (float)im.y, kc = (float)im.z;
+    w = a;
+    w.x -= ka * p.L.lx + kb * p.L.xy + kc * p.L.xz;
+    w.y -= kb * p.L.ly + kc * p.L.yz;
+    w.z -= kc * p.L.lz;
+  }
+  ps[s] = w;
+  if (!rebuild) return;
+  p.type_sorted[s] = ty;
+  hmd_nbl_boxes(p, s, valid, w, hmd_lane());
   // The atom's exclusion partners as sorted slots (a chain of dependent
-  // loads: id, CSR row, partner, its slot), resolved here for every atom at
+  // loads: CSR row, partner, its slot), resolved here for every atom at
   // once so that the list build reads them with one load.
   uint32_t b0 = 0, b1 = 0;
   if (valid) {
-    const uint32_t id = p.sorted_id[s];
     b0 = p.excl_offsets[id];
     b1 = p.excl_offsets[id + 1];
   }
@@ -261,7 +390,7 @@ __device__ __forceinline__ void hmd_nbl_bbox_body(const NblBboxParams& p, const 
     p.excl_slot[(size_t)m * p.n_pad + s] = slot;
   }
 }
-HMD_KERNEL(hmd_nbl_bbox, NblBboxParams, 256)
+HMD_KERNEL(hmd_nbl_gather, NblGatherParams, 256)
 
 // Conservative min-image gap between two boxes (compare
 // packed_block_bbox_dist_sq, kernels/neighbor.cu:365-388).  Used only as a
@@ -324,16 +453,6 @@ __device__ inline float hmd_box_gap2(float4 ca, float4 ha, float4 cb, float4 hb,
 
 typedef __attribute__((address_space(4))) const float4 hmd_const_f4;
 
-// Inclusive prefix sum over the 64 lanes.
-__device__ inline uint32_t hmd_wave_scan_incl(uint32_t v, uint32_t lane) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t t = (uint32_t)__shfl_up((int)v, (unsigned)o, HMD_WAVE);
-    if (lane >= (uint32_t)o) v += t;
-  }
-  return v;
-}
-
 // Placement key of a kept j-atom (see above).
 __device__ inline uint32_t hmd_nbl_key(uint32_t m8, bool own) {
   return own ? 0u : 1u + (uint32_t)__builtin_ctz(m8) + (31u - (uint32_t)__builtin_clz(m8));
@@ -384,7 +503,7 @@ __device__ __forceinline__ void hmd_nbl_build_body(const NblBuildParams& p, cons
 
   for (uint32_t e = threadIdx.x; e < HMD_NBL_EMASK_CAP; e += blockDim.x) s_emask[e] = 0u;
   // wave 0: the sorted slots of each i-atom's exclusion partners (resolved
-  // by hmd_nbl_bbox), and their positions in the cluster's list once placed
+  // by hmd_nbl_gather), and their positions in the cluster's list once placed
   const uint32_t si = c * HMD_CLUSTER + lane;
   uint32_t ex_slot[HMD_MAX_INLINE_EXCL], ex_pos[HMD_MAX_INLINE_EXCL];
 #pragma unroll
@@ -686,34 +805,46 @@ __device__ __forceinline__ void hmd_nbl_build_body(const NblBuildParams& p, cons
 }
 HMD_KERNEL(hmd_nbl_build, NblBuildParams, 64 * HMD_NBL_WAVES, HMD_NBL_BUILD_WAVES_PER_EU)
 
-// Flatten (cluster, entry) into the work list the force kernel walks, one
-// wave per cluster (entry_offset is the exclusive scan of entry_count with
-// the total at [n_clusters]).
+// Work list: cluster c's entries at the sum of the lower clusters' counts
+// (n_offsets == 0: taken here, every workgroup of four clusters adding up the
+// counts below its own, 12 KB at 196,608 atoms; else scanned by a launch
+// before).  The last workgroup to finish closes the rebuild -- work-list
+// length, status flags, generation -- when every one has read the gate.
 __device__ __forceinline__ void hmd_nbl_worklist_body(const NblWorkParams& p, const uint32_t hmd_bx,
     const uint32_t hmd_gx) {
   if (!hmd_gate(p.status, HMD_STATUS_DISPLACED)) return;
-  const uint32_t c = hmd_bx * (blockDim.x / HMD_WAVE) + threadIdx.x / HMD_WAVE;
-  if (c >= p.n_clusters) return;
-  const uint32_t cnt = p.entry_count[c];
-  const uint32_t off = p.entry_offset[c];
-  for (uint32_t k = hmd_lane(); k < cnt; k += HMD_WAVE) p.work[off + k] = c * p.cap_entries + k;
-}
-HMD_KERNEL(hmd_nbl_worklist, NblWorkParams, 256)
-
-// Close the rebuild: work-list length, status flags and generation (a kernel
-// of its own, after every block of the work-list kernel has read the gate).
-__device__ __forceinline__ void hmd_nbl_close_body(const NblWorkParams& p, const uint32_t hmd_bx,
-    const uint32_t hmd_gx) {
-  if (!hmd_gate(p.status, HMD_STATUS_DISPLACED)) return;
+  __shared__ uint32_t s_sum[4];
+  const uint32_t wave = threadIdx.x / HMD_WAVE, lane = hmd_lane();
+  const uint32_t c0 = 4u * hmd_bx, c = c0 + wave;
+  uint32_t off = 0;
+  if (p.entry_offset) {
+    if (c < p.n_clusters) off = p.entry_offset[c];
+  } else {
+    for (uint32_t k = threadIdx.x; k < c0; k += 256u) off += p.entry_count[k];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) off += (uint32_t)__shfl_xor((int)off, o, HMD_WAVE);
+    if (lane == 0) s_sum[wave] = off;
+    __syncthreads();
+    off = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+    for (uint32_t k = c0; k < min(c, p.n_clusters); ++k) off += p.entry_count[k];
+  }
+  if (c < p.n_clusters) {
+    const uint32_t cnt = p.entry_count[c];
+    for (uint32_t k = lane; k < cnt; k += HMD_WAVE) p.work[off + k] = c * p.cap_entries + k;
+    if (c == p.n_clusters - 1u && lane == 0) p.n_work[0] = off + cnt;
+  }
+  __syncthreads();
   if (threadIdx.x == 0) {
-    p.n_work[0] = p.entry_offset[p.n_clusters];
     uint32_t* st = p.status;
-    const uint32_t s = st[0];
-    st[0] = (s & ~HMD_STATUS_DISPLACED) | HMD_STATUS_REBUILT;
-    st[1] += 1u;   // rebuild generation
+    // status[3]: workgroups of this launch that have finished
+    if (atomicAdd(&st[3], 1u) == hmd_gx - 1u) {
+      st[3] = 0u;
+      st[0] = (st[0] & ~HMD_STATUS_DISPLACED) | HMD_STATUS_REBUILT;
+      st[1] += 1u;   // rebuild generation
+    }
   }
 }
-HMD_KERNEL(hmd_nbl_close, NblWorkParams, 64)
+HMD_KERNEL(hmd_nbl_worklist, NblWorkParams, 256)
 
 // Decode the list into the exact pair set (canonical (min, max) ids of every
 // listed pair whose f32 min-image distance is <= r_search), one wave per

@@ -832,9 +832,13 @@ void ForceField::pair_forces(bool fev) {
   pp.shift_margin = r_cut + 0.5f * r_skin;
   pp.acc = acc.ptr;
   pp.acc_stride = n_pad;
-  // four waves per block, and never more waves than the list has entries
+  pp.team_below = kPairTeam;
+  // a workgroup per entry of a short list, four waves of whole entries per
+  // workgroup of a long one, and never more waves than the list has work for
   // (small systems would otherwise launch mostly idle blocks)
-  const uint32_t entry_blocks = ceil_div((uint64_t)n_clusters * cap_entries, 4);
+  const uint64_t entries = (uint64_t)n_clusters * cap_entries;
+  const uint32_t entry_blocks = std::max(
+      ceil_div(entries, 4), (uint32_t)std::min<uint64_t>(entries, kPairTeamBlocks));
   const uint32_t blocks =
       std::max(1u, std::min((uint32_t)c.num_cus * pair_blocks_per_cu, entry_blocks));
   KernelId k = lj_on && coul_on ? (fev ? K_hmd_pair_force_fev : K_hmd_pair_force_f)

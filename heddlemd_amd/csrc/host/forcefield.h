@@ -38,6 +38,13 @@ constexpr double kNblGrowth = 1.5;
 // it theirs).  Beyond, 16-bit ids and counts no longer fit the LDS.
 constexpr uint32_t kNblSortSmall = 12288;
 constexpr uint32_t kNblKeysInline = 5120;
+// List entries below which a pair-kernel workgroup shares an entry, and the
+// workgroups then launched.  Measured with sharing on and off: 648 atoms 111 ->
+// 97 us a step, 4,503 flexible (about 1,000 entries) 149 -> 135, argon 10,000
+// 45 -> 38, sixteen replicas 430 -> 420; 8,997 atoms (about 1,900) 294 -> 307
+// us a frame, 24,576 156 -> 161.
+constexpr uint32_t kPairTeam = 1536;
+constexpr uint32_t kPairTeamBlocks = 1280;
 // Clusters up to which the work-list kernel adds up the entry counts itself.
 constexpr uint32_t kNblCountInline = 4096;
 constexpr double kNblFillThreshold = 0.8;

@@ -187,6 +187,7 @@ struct PairParams {
   float shift_margin;          // r_cut + r_skin/2: per-cluster shift eligibility
   long long* acc;              // [5][n_pad] fixed-point F_x,F_y,F_z,E,W (sorted)
   uint32_t acc_stride;         // n_pad
+  uint32_t team_below;         // entries below which a workgroup shares an entry
 };
 
 // Listed partner pairs with a non-zero exclusion scale (1-4 pairs and the

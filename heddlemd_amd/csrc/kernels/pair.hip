@@ -214,16 +214,32 @@ __device__ inline void hmd_pair_isteps(const PairParams& p, const float4* s_lj,
   }
 }
 
+// Quarter `part` of the sub-clusters in an entry's mask: those whose rank among
+// the m set bits lies in [part m / 4, (part + 1) m / 4).
+__device__ inline uint32_t hmd_pair_part(uint32_t m8, uint32_t part) {
+  const uint32_t m = (uint32_t)__builtin_popcount(m8);
+  const uint32_t lo = (part * m) >> 2, hi = ((part + 1u) * m) >> 2;
+  uint32_t out = 0;
+  for (uint32_t r = 0; r < hi; ++r) {
+    const uint32_t bit = m8 & (0u - m8);
+    m8 ^= bit;
+    if (r >= lo) out |= bit;
+  }
+  return out;
+}
+
 // One entry: lane k gathers j-atom k (shifted to the image nearest the
 // cluster centre when SHIFT), the i-sub-clusters it reaches come from the
 // entry's mask, and the entry's exclusion rows (lane = i-atom, bits over the
 // j-slots) are transposed so that each j lane holds its bits over the
-// i-atoms.  The j reaction is flushed once per entry.
+// i-atoms.  The j reaction is flushed once per entry: to memory, or, where the
+// workgroup's waves share the entry (s_j set, `part` of four), to the
+// workgroup's sums in LDS.  Returns the lane's j-atom.
 template <bool FEV, bool LJ, bool COUL, bool SHIFT>
 __device__ inline void hmd_pair_entry(const PairParams& p, const float4* s_lj,
                                       const float4* s_ct, const float4* s_ip,
-                                      const uint32_t* s_it, float* s_fi, uint32_t slot,
-                                      uint32_t c, float cx, float cy, float cz,
+                                      const uint32_t* s_it, float* s_fi, long long* s_j,
+                                      bool team, uint32_t part, uint32_t slot, uint32_t c, float cx, float cy, float cz,
                                       uint64_t lj_ibits, uint32_t lane) {
 #pragma clang fp contract(off)   // as in hmd_pair_isteps: fused multiply-adds written out
   const float4* ps = reinterpret_cast<const float4*>(p.posq_sorted);
@@ -231,7 +247,11 @@ __device__ inline void hmd_pair_entry(const PairParams& p, const float4* s_lj,
   const size_t ebase = (size_t)slot * HMD_ENTRY;
   const uint32_t my_j = p.entry_j[ebase + lane];
   // bits 0-7: i-sub-clusters reached; bit 8: the entry holds an exclusion
-  const uint32_t emask = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]);
+  uint32_t emask = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]);
+  if (team) {
+    emask = (emask & 0x100u) | hmd_pair_part(emask & 0xFFu, part);
+    if ((emask & 0xFFu) == 0u) return;
+  }
   const uint64_t ex = (emask & 0x100u) ? p.entry_excl[ebase + lane] : 0ull;
   const bool valid_j = my_j != HMD_SENTINEL;
   const uint32_t jj_l = valid_j ? my_j : 0u;
@@ -262,8 +282,14 @@ __device__ inline void hmd_pair_entry(const PairParams& p, const float4* s_lj,
     constexpr uint32_t NC = FEV ? 5u : 3u;
     long long* acc = p.acc;
 #pragma unroll
-    for (uint32_t cc = 0; cc < NC; ++cc)
-      hmd_atomic_add_fixed(&acc[cc * p.acc_stride + my_j], hmd_to_fixed(fj[cc], HMD_FIXED_SHIFT));
+    for (uint32_t cc = 0; cc < NC; ++cc) {
+      const long long v = hmd_to_fixed(fj[cc], HMD_FIXED_SHIFT);
+      if (team)
+        atomicAdd(reinterpret_cast<unsigned long long*>(&s_j[cc * HMD_CLUSTER + lane]),
+                  static_cast<unsigned long long>(v));
+      else
+        hmd_atomic_add_fixed(&acc[cc * p.acc_stride + my_j], v);
+    }
   }
 }
 
@@ -282,11 +308,38 @@ __device__ inline void hmd_fold_i(float* s_fi, long long (&fix)[5], uint32_t lan
   }
 }
 
-// The running totals of the wave's share of one cluster to the accumulators.
+// The workgroup's LDS sums to the accumulators of atom s of the lane (a
+// component per wave), and cleared.
 template <bool FEV>
-__device__ inline void hmd_flush_i(const PairParams& p, long long (&fix)[5], uint32_t si,
-                                   bool vi) {
+__device__ inline void hmd_flush_shared(const PairParams& p, long long* s_j, uint32_t s,
+                                        bool valid, uint32_t wv, uint32_t lane) {
   constexpr uint32_t NC = FEV ? 5u : 3u;
+  for (uint32_t cc = wv; cc < NC; cc += 4u) {
+    const long long v = s_j[cc * HMD_CLUSTER + lane];
+    s_j[cc * HMD_CLUSTER + lane] = 0;
+    if (valid) hmd_atomic_add_fixed(&p.acc[cc * p.acc_stride + s], v);
+  }
+}
+
+// The running totals of the wave's share of one cluster to the accumulators,
+// those of a team of four waves summed in LDS first.
+template <bool FEV>
+__device__ inline void hmd_flush_i(const PairParams& p, long long (&fix)[5], long long* s_j,
+                                   bool team, uint32_t si, bool vi, uint32_t wv,
+                                   uint32_t lane) {
+  constexpr uint32_t NC = FEV ? 5u : 3u;
+  if (team) {
+#pragma unroll
+    for (uint32_t cc = 0; cc < NC; ++cc) {
+      atomicAdd(reinterpret_cast<unsigned long long*>(&s_j[cc * HMD_CLUSTER + lane]),
+                static_cast<unsigned long long>(fix[cc]));
+      fix[cc] = 0;
+    }
+    __syncthreads();
+    hmd_flush_shared<FEV>(p, s_j, si, vi, wv, lane);
+    __syncthreads();
+    return;
+  }
 #pragma unroll
   for (uint32_t cc = 0; cc < NC; ++cc) {
     if (vi) hmd_atomic_add_fixed(&p.acc[cc * p.acc_stride + si], fix[cc]);
@@ -306,6 +359,21 @@ __device__ inline void hmd_pair_body(const PairParams& p, const uint32_t hmd_bx,
   __shared__ float4 s_ip[4][HMD_CLUSTER];
   __shared__ uint32_t s_it[4][HMD_CLUSTER];
   __shared__ float s_fi[4][(FEV ? 5 : 3) * HMD_CLUSTER];
+  __shared__ long long s_team[(FEV ? 5 : 3) * HMD_CLUSTER];
+  // A long list gives every wave a contiguous share of whole entries.  A list
+  // of fewer than team_below entries would leave the chip's waves one entry
+  // each or none, so there a workgroup shares an entry: each wave takes a
+  // quarter of the i-sub-clusters it reaches, and the four waves' sums meet in
+  // LDS, so that memory sees the atomics of one entry.  The rule reads the
+  // list alone: the sums, converted part by part, do not depend on the launch
+  // shape.
+  const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / HMD_WAVE);
+  const uint32_t lane = hmd_lane();
+  const uint32_t nw = __builtin_amdgcn_readfirstlane(*p.n_work);
+  const bool team = nw < p.team_below;
+  const uint32_t n_units = team ? hmd_gx : 4u * hmd_gx;
+  const uint32_t per = (nw + n_units - 1) / n_units;
+  if ((team ? hmd_bx : 4u * hmd_bx) * per >= nw) return;   // the whole workgroup
   const uint32_t nt2 = p.n_types * p.n_types;
   for (uint32_t k = threadIdx.x; k < nt2; k += blockDim.x) {
     const float2 cc = reinterpret_cast<const float2*>(p.lj_c6c12)[k];
@@ -316,19 +384,14 @@ __device__ inline void hmd_pair_body(const PairParams& p, const uint32_t hmd_bx,
     for (uint32_t k = threadIdx.x; k < (FEV ? 2u : 1u) * HMD_COUL_BINS; k += blockDim.x)
       s_ct[k] = ct[k];
   }
-  const uint32_t wv = threadIdx.x / HMD_WAVE;
-  const uint32_t lane = hmd_lane();
   float* fi = s_fi[wv];
 #pragma unroll
   for (uint32_t cc = 0; cc < (FEV ? 5u : 3u); ++cc) fi[cc * HMD_CLUSTER + lane] = 0.0f;
+  for (uint32_t k = threadIdx.x; k < (FEV ? 5u : 3u) * HMD_CLUSTER; k += blockDim.x)
+    s_team[k] = 0;
   __syncthreads();
 
-  const uint32_t waves_per_block = blockDim.x / HMD_WAVE;
-  const uint32_t n_waves = hmd_gx * waves_per_block;
-  const uint32_t gw = hmd_bx * waves_per_block + wv;
-  const uint32_t nw = *p.n_work;
-  const uint32_t per = (nw + n_waves - 1) / n_waves;
-  const uint32_t w0 = gw * per;
+  const uint32_t w0 = (team ? hmd_bx : 4u * hmd_bx + wv) * per;
   const uint32_t w1 = min(w0 + per, nw);
   if (w0 >= w1) return;
 
@@ -345,10 +408,10 @@ __device__ inline void hmd_pair_body(const PairParams& p, const uint32_t hmd_bx,
   float cx = 0, cy = 0, cz = 0;
   long long fix[5] = {0, 0, 0, 0, 0};
   for (uint32_t w = w0; w < w1; ++w) {
-    const uint32_t slot = p.work[w];
+    const uint32_t slot = __builtin_amdgcn_readfirstlane(p.work[w]);
     const uint32_t c = slot / p.cap_entries;
     if (c != cur_c) {
-      if (cur_c != HMD_SENTINEL) hmd_flush_i<FEV>(p, fix, si, vi);
+      if (cur_c != HMD_SENTINEL) hmd_flush_i<FEV>(p, fix, s_team, team, si, vi, wv, lane);
       cur_c = c;
       si = c * HMD_CLUSTER + lane;
       vi = si < p.n;
@@ -387,17 +450,23 @@ __device__ inline void hmd_pair_body(const PairParams& p, const uint32_t hmd_bx,
       __builtin_amdgcn_wave_barrier();
     }
     if (shift)
-      hmd_pair_entry<FEV, LJ, COUL, true>(p, s_lj, s_ct, s_ip[wv], s_it[wv], fi, slot, c, cx, cy,
-                                          cz, lj_ibits, lane);
+      hmd_pair_entry<FEV, LJ, COUL, true>(p, s_lj, s_ct, s_ip[wv], s_it[wv], fi, s_team, team, wv,
+                                          slot, c, cx, cy, cz, lj_ibits, lane);
     else
-      hmd_pair_entry<FEV, LJ, COUL, false>(p, s_lj, s_ct, s_ip[wv], s_it[wv], fi, slot, c, cx,
-                                           cy, cz, lj_ibits, lane);
+      hmd_pair_entry<FEV, LJ, COUL, false>(p, s_lj, s_ct, s_ip[wv], s_it[wv], fi, s_team, team,
+                                           wv, slot, c, cx, cy, cz, lj_ibits, lane);
     // the entry's i-side sums go to fixed point on their own: the totals are
     // then the same however the work list is split among waves (launch
     // shape, CU count), not only run to run
     hmd_fold_i<FEV>(fi, fix, lane);
+    if (team) {
+      __syncthreads();
+      const uint32_t my_j = p.entry_j[(size_t)slot * HMD_ENTRY + lane];
+      hmd_flush_shared<FEV>(p, s_team, my_j, my_j != HMD_SENTINEL, wv, lane);
+      __syncthreads();
+    }
   }
-  hmd_flush_i<FEV>(p, fix, si, vi);
+  hmd_flush_i<FEV>(p, fix, s_team, team, si, vi, wv, lane);
 }
 
 // Minimum waves per SIMD the register allocation must allow (1: no limit).

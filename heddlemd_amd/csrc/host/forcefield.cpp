@@ -907,9 +907,13 @@ void ForceField::spme_forces(bool fev, bool mark_binned) {
   SpmeBinParams bp{p.posq.ptr, sorted_id.ptr, n, L, n0, n1, n2, brick[0], brick[1], brick[2],
                    nb[0], nb[1], nb[2], atom_bin.ptr, bin_count.ptr, bin_start.ptr,
                    bin_atoms.ptr};
-  launch(c, K_hmd_spme_bin, ceil_div(n, 256), 256, 0, bp);
-  bin_scan.run(c, bin_count.ptr, bin_start.ptr, nullptr, 0);
-  launch(c, K_hmd_spme_bin_scatter, ceil_div(n, 256), 256, 0, bp);
+  if (n <= HMD_SPME_BIN_SMALL && n_bins <= 4096u) {
+    launch(c, K_hmd_spme_bin_small, 1, 1024, 0, bp);
+  } else {
+    launch(c, K_hmd_spme_bin, ceil_div(n, 256), 256, 0, bp);
+    bin_scan.run(c, bin_count.ptr, bin_start.ptr, nullptr, 0);
+    launch(c, K_hmd_spme_bin_scatter, ceil_div(n, 256), 256, 0, bp);
+  }
   c.mark("spme_bin");
   if (mark_binned) check(hipEventRecord(ev_binned, c.stream), "hipEventRecord");
 
@@ -1048,12 +1052,9 @@ void ForceField::spme_forces(bool fev, bool mark_binned) {
   }
   }
   c.mark("spme_fft_solve");
-  SpmeReduceParams rp{partials.ptr, partial_blocks, spme_out.ptr};
-  launch(c, K_hmd_spme_reduce, 1, 256, 0, rp);
-
   SpmeGatherParams gp{p.posq.ptr, n, L, n0, n1, n2, brick[0], brick[1], brick[2],
                       nb[0], nb[1], nb[2], bin_start.ptr, bin_atoms.ptr, V.ptr,
-                      u_self.ptr, spme_out.ptr, slow_f.ptr, slow_e.ptr, slow_w.ptr,
+                      u_self.ptr, partials.ptr, partial_blocks, spme_out.ptr, slow_f.ptr, slow_e.ptr, slow_w.ptr,
                       fev ? 1u : 0u};
   const size_t sh_gather = (size_t)(brick[0] + order - 1) * (brick[1] + order - 1) *
                            (brick[2] + order - 1) * 4;

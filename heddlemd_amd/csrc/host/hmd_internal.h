@@ -23,12 +23,12 @@
   X(hmd_pair_force_f) X(hmd_pair_force_fev) X(hmd_pair_force_lj_f)           \
   X(hmd_pair_force_lj_fev) X(hmd_pair_force_coul_f) X(hmd_pair_force_coul_fev)\
   X(hmd_pair_finalize) X(hmd_pair_scaled) X(hmd_slot_add)                   \
-  X(hmd_spme_bin) X(hmd_spme_bin_scatter)                                    \
+  X(hmd_spme_bin) X(hmd_spme_bin_scatter) X(hmd_spme_bin_small)              \
   X(hmd_spme_spread_p4) X(hmd_spme_gather_p4)                                \
   X(hmd_spme_spread_p5) X(hmd_spme_gather_p5)                                \
   X(hmd_spme_spread_p6) X(hmd_spme_gather_p6)                                \
   X(hmd_spme_spread_p8) X(hmd_spme_gather_p8)                                \
-  X(hmd_fft_r2c_c) X(hmd_fft_c2r_c) X(hmd_fft_axis) X(hmd_spme_reduce)       \
+  X(hmd_fft_r2c_c) X(hmd_fft_c2r_c) X(hmd_fft_axis)                          \
   X(hmd_fft_axis_mix) X(hmd_fft_r2c_mix) X(hmd_fft_c2r_mix)                  \
   X(hmd_fft_axis_16) X(hmd_fft_r2c_16) X(hmd_fft_c2r_16)                     \
   X(hmd_fft_axis_32) X(hmd_fft_r2c_32) X(hmd_fft_c2r_32)                     \

@@ -298,34 +298,6 @@ __device__ __forceinline__ void hmd_fft_axis_body(const FftParams& p, const uint
 }
 HMD_KERNEL(hmd_fft_axis, FftParams, 256)
 
-// Fixed-order reduction of the per-block partials: out[0] = W_recip =
-// 0.5 * sum hw vf |rho_hat|^2, out[1] = U_recip = 0.5 * sum hw G |rho_hat|^2
-// (kernels/spme_recip.cu:376-402 with the 0.5 half-sum factor).
-__device__ __forceinline__ void hmd_spme_reduce_body(const SpmeReduceParams& p, const uint32_t hmd_bx,
-    const uint32_t hmd_gx) {
-  __shared__ double s[2][256];
-  double a = 0.0, b = 0.0;
-  for (uint32_t i = threadIdx.x; i < p.n_partials; i += blockDim.x) {
-    a += p.partials[2 * i];
-    b += p.partials[2 * i + 1];
-  }
-  s[0][threadIdx.x] = a;
-  s[1][threadIdx.x] = b;
-  __syncthreads();
-  for (uint32_t st = blockDim.x / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) {
-      s[0][threadIdx.x] += s[0][threadIdx.x + st];
-      s[1][threadIdx.x] += s[1][threadIdx.x + st];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    p.out[0] = 0.5 * s[0][0];
-    p.out[1] = 0.5 * s[1][0];
-  }
-}
-HMD_KERNEL(hmd_spme_reduce, SpmeReduceParams, 256)
-
 // ---------------------------------------------------------------------------
 // Power-of-two line lengths n = N1 N2 (16 ... 256): compile-time two-stage
 // transform, n = N2 n1 + n2 -> k = k1 + N1 k2:

@@ -283,9 +283,10 @@ struct SpmeBinParams {
   uint32_t nb0, nb1, nb2;      // bricks per axis
   uint32_t* atom_bin;          // [n] bin of each sorted slot
   uint32_t* bin_count;         // [n_bins] zero on entry, zero after scatter
-  const uint32_t* bin_start;   // [n_bins+1]
+  uint32_t* bin_start;         // [n_bins+1] (written by hmd_spme_bin_small alone)
   uint32_t* bin_atoms;         // [n]
 };
+#define HMD_SPME_BIN_SMALL 6144u   // atoms of the one-workgroup binning
 
 struct SpmeSpreadParams {
   const float* posq;
@@ -310,7 +311,9 @@ struct SpmeGatherParams {
   const uint32_t* bin_atoms;
   const float* V;              // real mesh
   const float* u_self;         // [n]
-  const double* w_recip;       // [1] scalar reciprocal virial (total)
+  const double* partials;      // [n_partials][2] of the a-axis pass
+  uint32_t n_partials;
+  double* totals;              // [2] reciprocal virial and energy
   float* f;                    // [3][n] canonical, overwritten
   float* e;                    // [n]
   float* w;                    // [n]
@@ -344,12 +347,6 @@ struct FftParams {
   double* partials;            // [grid blocks][2]: virial, energy
   const float* gv;             // float2[n0][n1][nch]: (G, vf) in f32, or null
   const double* gv64;          // double2[n0][n1][nch]: (G, vf), or null
-};
-
-struct SpmeReduceParams {
-  const double* partials;
-  uint32_t n_partials;
-  double* out;                 // [2]: W_recip, U_recip (half sums applied)
 };
 
 // ------------------------------------------------------- integrators ---

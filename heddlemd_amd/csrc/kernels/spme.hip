@@ -180,6 +180,63 @@ __device__ __forceinline__ void hmd_spme_bin_scatter_body(const SpmeBinParams& p
 }
 HMD_KERNEL(hmd_spme_bin_scatter, SpmeBinParams, 256)
 
+// The three launches of the binning (bin, scan, scatter) in one workgroup,
+// for systems of at most HMD_SPME_BIN_SMALL atoms and 4,096 bins: an atom's
+// rank in its bin comes from the LDS count, so one pass over the atoms is
+// enough.  The launches were 4.5 + 4.7 + 6.5 us at 648 atoms, each waiting
+// for the one before.
+__device__ __forceinline__ void hmd_spme_bin_small_body(const SpmeBinParams& p,
+                                                        const uint32_t hmd_bx,
+                                                        const uint32_t hmd_gx) {
+  __shared__ uint32_t s_bins[4096];
+  __shared__ uint32_t s_wave[16];
+  constexpr uint32_t U = HMD_SPME_BIN_SMALL / 1024u;
+  const uint32_t t = threadIdx.x, lane = hmd_lane(), wave = t / HMD_WAVE;
+  const uint32_t n_bins = p.nb0 * p.nb1 * p.nb2;
+  reinterpret_cast<uint4*>(s_bins)[t] = make_uint4(0u, 0u, 0u, 0u);
+  uint32_t id[U], bin[U], rank[U];
+#pragma unroll
+  for (uint32_t u = 0; u < U; ++u)
+    id[u] = p.sorted_id[min(t + 1024u * u, p.n - 1u)];
+  float4 pq[U];
+#pragma unroll
+  for (uint32_t u = 0; u < U; ++u) pq[u] = reinterpret_cast<const float4*>(p.posq)[id[u]];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t u = 0; u < U; ++u) {
+    if (t + 1024u * u < p.n) {
+      bin[u] = hmd_spme_bin_of(p, pq[u]);
+      rank[u] = atomicAdd(&s_bins[bin[u]], 1u);
+    }
+  }
+  __syncthreads();
+  // exclusive scan, four bins a thread
+  const uint4 v = reinterpret_cast<const uint4*>(s_bins)[t];
+  const uint32_t sum = v.x + v.y + v.z + v.w;
+  uint32_t incl = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t w = (uint32_t)__shfl_up((int)incl, (unsigned)o, HMD_WAVE);
+    if (lane >= (uint32_t)o) incl += w;
+  }
+  if (lane == HMD_WAVE - 1) s_wave[wave] = incl;
+  __syncthreads();
+  uint32_t e = incl - sum;
+  for (uint32_t w = 0; w < wave; ++w) e += s_wave[w];
+  const uint32_t start[4] = {e, e + v.x, e + v.x + v.y, e + v.x + v.y + v.z};
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    s_bins[4u * t + k] = start[k];
+    if (4u * t + k < n_bins) p.bin_start[4u * t + k] = start[k];
+  }
+  if (t == 0) p.bin_start[n_bins] = p.n;
+  __syncthreads();
+#pragma unroll
+  for (uint32_t u = 0; u < U; ++u)
+    if (t + 1024u * u < p.n) p.bin_atoms[s_bins[bin[u]] + rank[u]] = id[u];
+}
+HMD_KERNEL(hmd_spme_bin_small, SpmeBinParams, 1024)
+
 // A contribution v (in units of 2^-24 e, |v| < 2^31) as the i64 count of
 // 2^-32 e rounded to nearest, from two i32 roundings: r1 = rint(v), the
 // remainder v - r1 (exact in f32, |.| <= 1/2) scaled by 2^8 and rounded,
@@ -356,8 +413,38 @@ __device__ inline void hmd_gather_body(const SpmeGatherParams& p, const uint32_t
   const int o0 = (int)(B0 * p.b0) - (P - 1);
   const int o1 = (int)(B1 * p.b1) - (P - 1);
   const int o2 = (int)(B2 * p.b2) - (P - 1);
+  // The solve's virial and energy partials, summed in FP64 in a fixed order by
+  // every workgroup that hands the virial out (and by the first, which keeps
+  // the totals): a launch of its own for this sum took 2.4 to 4.7 us.  W = 0.5
+  // sum hw vf |rho|^2, U = 0.5 sum hw G |rho|^2 (kernels/spme_recip.cu:376-402).
+  double tot_e = 0.0, tot_w = 0.0;
+  if (p.fev || hmd_bx == 0) {
+    __shared__ double s_part[2][4];
+    for (uint32_t k = threadIdx.x; k < p.n_partials; k += blockDim.x) {
+      tot_w += p.partials[2 * k];
+      tot_e += p.partials[2 * k + 1];
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      tot_e += __shfl_xor(tot_e, o, HMD_WAVE);
+      tot_w += __shfl_xor(tot_w, o, HMD_WAVE);
+    }
+    if (hmd_lane() == 0) {
+      s_part[0][threadIdx.x / HMD_WAVE] = tot_e;
+      s_part[1][threadIdx.x / HMD_WAVE] = tot_w;
+    }
+    __syncthreads();
+    tot_e = 0.5 * ((s_part[0][0] + s_part[0][1]) + (s_part[0][2] + s_part[0][3]));
+    tot_w = 0.5 * ((s_part[1][0] + s_part[1][1]) + (s_part[1][2] + s_part[1][3]));
+    if (hmd_bx == 0 && threadIdx.x == 0) {
+      p.totals[0] = tot_w;
+      p.totals[1] = tot_e;
+    }
+  }
+  const float ih2 = 1.0f / (float)h2, ih1 = 1.0f / (float)h1;
   for (uint32_t k = threadIdx.x; k < h0 * h1 * h2; k += blockDim.x) {
-    const uint32_t lc = k % h2, lb = (k / h2) % h1, la = k / (h2 * h1);
+    const uint32_t row = hmd_div_small(k, ih2), lc = k - row * h2;
+    const uint32_t la = hmd_div_small(row, ih1), lb = row - la * h1;
     int ga = o0 + (int)la, gb = o1 + (int)lb, gc = o2 + (int)lc;
     ga += ga < 0 ? (int)p.n0 : 0;
     gb += gb < 0 ? (int)p.n1 : 0;
@@ -374,7 +461,7 @@ __device__ inline void hmd_gather_body(const SpmeGatherParams& p, const uint32_t
               ba_z = (L.xy * L.yz - L.xz * L.ly) * ilx * ily * ilz;
   const float bb_y = ily, bb_z = -L.yz * ily * ilz;
   const float bc_z = ilz;
-  const float w_share = (float)(p.w_recip[0] / (double)p.n);
+  const float w_share = (float)(tot_w / (double)p.n);
 
   const uint32_t beg = p.bin_start[B], end = p.bin_start[B + 1];
   for (uint32_t k = beg + threadIdx.x; k < end; k += blockDim.x) {

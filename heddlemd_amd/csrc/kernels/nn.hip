@@ -8,10 +8,9 @@
 // x_ij = [phi, one-hot(species_i + species_j), D_i, D_j];
 // g_ij = s_out fc(s_ij) (N(x_ij) + N(x_ji)) / 2; dF_i = sum_j g_ij r^_ij.
 //
-// Traversal: the force field's packed half list (the pair
-// kernel's).  The network passes compact the in-range
-// pairs of each entry into an LDS queue and evaluate them 32 pairs (64
-// rows: both orientations) at a time:
+// Traversal: the force field's packed half list (the pair kernel's).  The
+// network passes compact the in-range pairs of each entry into an LDS queue
+// and evaluate them 32 pairs (64 rows: both orientations) at a time:
 //  * layer 1 is Z1^T = W1 X^T and layer 2 Z2^T = W2 H1^T as chains of
 //    v_mfma_f32_16x16x32_bf16 (A = weights, B = activations); each lane
 //    reads its slices of X^T whole from the wave's LDS tables;
@@ -143,10 +142,11 @@ hmd_nn_pack(const NnPackParams p) {
 // How the passes share the list: an item is an entry, or one of its
 // 2^split groups of i-sub-clusters, and wave v of n takes the items v, v + n,
 // ...  An entry of a dense liquid holds 0 to 4,096 pairs (about 1,000 on
-// average), so a wave needs several items of different entries before the
-// waves' totals even out: the list is split until there are `want` items (or
-// eight groups an entry).  Whole entries in contiguous shares left a CU with
-// 1.2 of 8 waves running on average at 9,999 atoms.
+// average), so a short list is split until there are HMD_NN_ITEMS items (or
+// eight groups an entry): eight of the 2,048 waves the chip holds of the
+// forward pass.  Whole entries in contiguous shares left a CU with 1.2 of 8
+// waves running on average at 9,999 atoms.
+#define HMD_NN_ITEMS 16384u
 struct HmdNnItems {
   uint32_t n, split;
   __device__ HmdNnItems(uint32_t entries, uint32_t want) : split(0) {
@@ -154,9 +154,12 @@ struct HmdNnItems {
     n = entries << split;
   }
   __device__ uint32_t entry(uint32_t w) const { return w >> split; }
-  __device__ uint32_t mask(uint32_t w) const {
+  // the group turns with the wave's round: the first and last i-sub-clusters
+  // of an entry hold different numbers of pairs, and the number of waves is a
+  // multiple of eight
+  __device__ uint32_t mask(uint32_t w, uint32_t round) const {
     const uint32_t group = 8u >> split;
-    return ((1u << group) - 1u) << (group * (w & ((1u << split) - 1u)));
+    return ((1u << group) - 1u) << (group * ((w + round) & ((1u << split) - 1u)));
   }
 };
 
@@ -191,32 +194,28 @@ __device__ inline float4 hmd_nn_apply_shift(float4 a, const HmdNnShift& sh, cons
 }
 
 // ------------------------------------------------------- descriptors ----
-// The pair kernel's traversal: lane = j-atom of the entry (shifted once to the image nearest the
-// i-cluster's centre), the i-atoms broadcast from a per-wave LDS table one
-// per step, over the 8-atom i-sub-clusters the entry's mask admits.  Per
-// pair the 16 basis values come from two exponentials each half (the
+// The pair kernel's traversal: lane = j-atom of the entry (shifted once to
+// the image nearest the i-cluster's centre), the i-atoms broadcast from an LDS
+// table one per step, over the 8-atom i-sub-clusters the entry's mask admits
+// (and the wave's item holds).  Per pair the 16 basis values come from two exponentials each half (the
 // product recurrence of hmd_nn_rbf8) with the cutoff folded into their
 // start; the j-atom's sums stay in the lane for the whole entry; the
 // i-atom's 16 sums of the step are reduced over the wave by two transposed
 // butterflies (totals of component m and 8 + m in lane 8m + 7) and added to
 // the wave's i accumulators in LDS.  Sums go to i64 fixed point (2^32): the
 // j side per entry, the i side per cluster share of the wave.
-extern "C" __global__ void __launch_bounds__(256)
+extern "C" __global__ void __launch_bounds__(64)
 hmd_nn_descriptors(const NnPassParams p) {
 #pragma clang fp contract(off)
-  __shared__ float4 s_ip[4][HMD_CLUSTER];
+  __shared__ float4 s_ip[HMD_CLUSTER];
   // i accumulators, component k of atom l at k * 65 + l (the odd stride
   // keeps the 8 lanes that add one atom's components on different banks)
-  __shared__ float s_di[4][16 * 65];
-  const uint32_t lane = hmd_lane();
-  const uint32_t wv = threadIdx.x / HMD_WAVE;
-  float* di = s_di[wv];
+  __shared__ float di[16 * 65];
+  const uint32_t lane = threadIdx.x;
 #pragma unroll
   for (int k = 0; k < 16; ++k) di[k * 65 + lane] = 0.0f;
-  const uint32_t waves_per_block = blockDim.x / HMD_WAVE;
-  const uint32_t n_waves = gridDim.x * waves_per_block;
-  const uint32_t gw = blockIdx.x * waves_per_block + wv;
-  const HmdNnItems items(__builtin_amdgcn_readfirstlane(*p.n_work), 2u * n_waves);
+  const uint32_t n_waves = gridDim.x, gw = blockIdx.x;
+  const HmdNnItems items(__builtin_amdgcn_readfirstlane(*p.n_work), HMD_NN_ITEMS);
   if (gw >= items.n) return;
   const float4* ps = reinterpret_cast<const float4*>(p.posq_sorted);
   const HmdLattice L = p.L;
@@ -235,9 +234,9 @@ hmd_nn_descriptors(const NnPassParams p) {
       if (vi) hmd_atomic_add_fixed(&acc[k * stride + si], hmd_to_fixed(v, HMD_NN_DESC_SHIFT));
     }
   };
-  for (uint32_t w = gw; w < items.n; w += n_waves) {
+  for (uint32_t w = gw, round = 0; w < items.n; w += n_waves, ++round) {
     const uint32_t slot = __builtin_amdgcn_readfirstlane(p.work[items.entry(w)]);
-    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w);
+    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w, round);
     if (pend == 0u) continue;
     const uint32_t c = slot / p.cap_entries;
     const uint32_t c0 = c * HMD_CLUSTER;
@@ -250,7 +249,7 @@ hmd_nn_descriptors(const NnPassParams p) {
       float4 a = hmd_nn_apply_shift(ps[si], sh, L);
       if (!vi) a.x = a.y = a.z = 1.0e18f;   // padding lanes fail every cutoff test
       hmd_wave_sync();
-      s_ip[wv][lane] = a;
+      s_ip[lane] = a;
       hmd_wave_sync();
     }
     const uint32_t my_j = p.entry_j[(size_t)slot * HMD_ENTRY + lane];
@@ -269,7 +268,7 @@ hmd_nn_descriptors(const NnPassParams p) {
 #pragma unroll 2
       for (uint32_t u = 0; u < 8; ++u) {
         const uint32_t i = 8u * sb + u;
-        const float4 a = s_ip[wv][i];
+        const float4 a = s_ip[i];
         float dx = a.x - pj.x, dy = a.y - pj.y, dz = a.z - pj.z;
         if (!sh.on) hmd_min_image(dx, dy, dz, L);
         const float r2 = dx * dx + dy * dy + dz * dz;
@@ -440,7 +439,7 @@ struct HmdNnFwdRegs {
 // exponential and a reciprocal each).  Weights and biases stay in registers
 // (two waves per SIMD) and results in architectural VGPRs; with weights in
 // LDS, one tile in flight and the results moved out of the accumulation
-// registers, 24,576 atoms took 1,585 us and 196,608 atoms 6.18 ms, now 1,216
+// registers, 24,576 atoms took 1,585 us and 196,608 atoms 6.18 ms, then 1,216
 // us and 4.64 ms.
 __device__ inline void hmd_nn_forward_batch(const NnPassParams& p, const HmdNnFwdRegs& R,
                                             HmdNnTables& W, long long (*acc)[3][HMD_WAVE],
@@ -502,18 +501,17 @@ __device__ inline void hmd_nn_forward_batch(const NnPassParams& p, const HmdNnFw
   hmd_wave_sync();
 }
 
-extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+// One wave a workgroup: nothing is shared between waves, and a workgroup of
+// four held three idle SIMDs until its slowest wave was done (62% of the SIMDs
+// had a wave on average): 24,576 atoms 1,000 -> 741 us a pass.
+extern "C" __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 hmd_nn_forward(const NnPassParams p) {
-  __shared__ HmdNnTables Wv[4];
-  __shared__ long long s_acc[4][2][3][HMD_WAVE];
-  const uint32_t lane = hmd_lane();
-  const uint32_t wv = threadIdx.x / HMD_WAVE;
-  const uint32_t n_waves = gridDim.x * (blockDim.x / HMD_WAVE);
-  const uint32_t gw = blockIdx.x * (blockDim.x / HMD_WAVE) + wv;
-  const HmdNnItems items(__builtin_amdgcn_readfirstlane(*p.n_work), 8u * n_waves);
+  __shared__ HmdNnTables W;
+  __shared__ long long acc[2][3][HMD_WAVE];
+  const uint32_t lane = threadIdx.x;
+  const uint32_t n_waves = gridDim.x, gw = blockIdx.x;
+  const HmdNnItems items(__builtin_amdgcn_readfirstlane(*p.n_work), HMD_NN_ITEMS);
   if (gw >= items.n) return;
-  HmdNnTables& W = Wv[wv];
-  long long(*acc)[3][HMD_WAVE] = s_acc[wv];
   const float4* ps = reinterpret_cast<const float4*>(p.posq_sorted);
   const uint32_t stride = p.n_pad;
   const uint32_t g = lane >> 4;
@@ -543,9 +541,9 @@ hmd_nn_forward(const NnPassParams p) {
   uint32_t cur_c = HMD_SENTINEL, si = 0, n_i = 0;
   bool vi = false;
   HmdNnShift sh{false, 0.0f, 0.0f, 0.0f};
-  for (uint32_t w = gw; w < items.n; w += n_waves) {
+  for (uint32_t w = gw, round = 0; w < items.n; w += n_waves, ++round) {
     const uint32_t slot = __builtin_amdgcn_readfirstlane(p.work[items.entry(w)]);
-    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w);
+    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w, round);
     if (pend == 0u) continue;
     const uint32_t c = slot / p.cap_entries;
     const uint32_t my_j = p.entry_j[(size_t)slot * HMD_ENTRY + lane];
@@ -801,7 +799,7 @@ hmd_nn_backward(const NnPassParams p) {
   const uint32_t wv = threadIdx.x / HMD_WAVE;
   const uint32_t n_waves = gridDim.x * (blockDim.x / HMD_WAVE);
   const uint32_t gw = blockIdx.x * (blockDim.x / HMD_WAVE) + wv;
-  const HmdNnItems items(__builtin_amdgcn_readfirstlane(*p.n_work), 8u * n_waves);
+  const HmdNnItems items(__builtin_amdgcn_readfirstlane(*p.n_work), HMD_NN_ITEMS);
   HmdNnWave& W = Wv[wv];
   const float4* ps = reinterpret_cast<const float4*>(p.posq_sorted);
   if (lane < 32u) W.xin[lane][3] = __builtin_bit_cast(hmd_bf16x8, hmd_u32x4{0u, 0u, 0u, 0u});
@@ -818,9 +816,9 @@ hmd_nn_backward(const NnPassParams p) {
 
   uint32_t cur_c = HMD_SENTINEL, n_i = 0;
   HmdNnShift sh{false, 0.0f, 0.0f, 0.0f};
-  for (uint32_t w = gw; w < items.n; w += n_waves) {
+  for (uint32_t w = gw, round = 0; w < items.n; w += n_waves, ++round) {
     const uint32_t slot = __builtin_amdgcn_readfirstlane(p.work[items.entry(w)]);
-    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w);
+    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w, round);
     if (pend == 0u) continue;
     const uint32_t c = slot / p.cap_entries;
     const uint32_t my_j = p.entry_j[(size_t)slot * HMD_ENTRY + lane];

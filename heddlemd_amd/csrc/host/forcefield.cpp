@@ -145,31 +145,38 @@ static bool mix_factors(uint32_t n, uint32_t f[2]) {
   return best != 0;
 }
 
-// Launch shapes of the mixed two-stage passes.  Columns: 8 adjacent lines a
-// workgroup (whole 64-byte segments of the mesh) while that gives every CU a
-// workgroup, else 4; the energy partials follow the grid.  Rows: 8 lines or
-// more, up to 32 once every CU has two workgroups.
+// Launch shapes of the mixed two-stage passes of a mesh, one of `boxes` that
+// share the launch.  Columns: 8 adjacent lines a workgroup (whole 64-byte
+// segments of the mesh) while that gives every CU a workgroup, else 4; 16 in a
+// batch whose boxes do so together (64 boxes of 24^3 to 48^3: 159 us a step
+// with widths picked for each box alone, 107 with 8, 80 with 16; four boxes
+// 124 us a step with any).  The energy partials follow the grid.  Rows: 8
+// lines or more, up to 32 once every CU has two workgroups (the same 64 boxes:
+// 56 us a step with 8, 36 with 16, 25 with 32).
 static ForceField::FftPass plan_mix_axis(uint32_t n, uint32_t n_outer, uint32_t cols,
-                                         uint32_t num_cus) {
+                                         uint32_t num_cus, uint32_t boxes) {
   ForceField::FftPass ps;
   if (!mix_factors(n, ps.f)) return ps;
   ps.mix = true;
   ps.k = K_hmd_fft_axis_mix;
-  ps.W = (uint64_t)n_outer * ceil_div(cols, 8) >= num_cus ? 8u : 4u;
-  ps.grid = n_outer * ceil_div(cols, ps.W);
-  ps.shmem = 8 * ((size_t)n + (size_t)n * ps.W + (size_t)ps.f[1] * (ps.f[0] | 1u) * ps.W);
-  return ps;
+  for (ps.W = boxes > 1 ? 16u : 8u;; ps.W /= 2) {
+    ps.grid = n_outer * ceil_div(cols, ps.W);
+    ps.shmem =
+        8 * ((size_t)n + (size_t)n * ps.W + (size_t)ps.f[1] * (ps.f[0] | 1u) * ps.W);
+    if (ps.W == 4 || ((uint64_t)ps.grid * boxes >= num_cus && ps.shmem <= 65536)) return ps;
+  }
 }
 
 static ForceField::FftPass plan_mix_lines(uint32_t n, uint32_t n_lines, uint32_t num_cus,
-                                          bool r2c) {
+                                          uint32_t boxes, bool r2c) {
   ForceField::FftPass ps;
   if (!mix_factors(n, ps.f)) return ps;
   ps.mix = true;
   ps.k = r2c ? K_hmd_fft_r2c_mix : K_hmd_fft_c2r_mix;
   const size_t per_line = 8 * ((n | 1u) + (size_t)ps.f[0] * (ps.f[1] | 1u));
   const uint32_t fit = (uint32_t)(49152 / per_line);   // 12 lines at n = 240
-  ps.W = std::min(fit, std::max(8u, std::min(32u, n_lines / (2 * num_cus))));
+  const uint64_t lines = (uint64_t)n_lines * boxes / (2 * num_cus);
+  ps.W = std::min(fit, (uint32_t)std::max<uint64_t>(8, std::min<uint64_t>(32, lines)));
   ps.grid = ceil_div(n_lines, ps.W);
   ps.shmem = 8 * (2 * (size_t)n + 1) + ps.W * per_line;
   return ps;
@@ -587,10 +594,10 @@ void ForceField::plan_fft() {
   pass_b = plan_axis(n1, n0, nch, target);
   pass_a = plan_axis(n0, n1, nch, target, 2);
   const uint32_t cus = (uint32_t)c.num_cus;
-  if (!pass_r2c.p2) pass_r2c = plan_mix_lines(n2 / 2, n0 * n1, cus, true);
-  if (!pass_c2r.p2) pass_c2r = plan_mix_lines(n2 / 2, n0 * n1, cus, false);
-  if (!pass_b.p2) pass_b = plan_mix_axis(n1, n0, nch, cus);
-  if (!pass_a.p2) pass_a = plan_mix_axis(n0, n1, nch, cus);
+  if (!pass_r2c.p2) pass_r2c = plan_mix_lines(n2 / 2, n0 * n1, cus, 1, true);
+  if (!pass_c2r.p2) pass_c2r = plan_mix_lines(n2 / 2, n0 * n1, cus, 1, false);
+  if (!pass_b.p2) pass_b = plan_mix_axis(n1, n0, nch, cus, 1);
+  if (!pass_a.p2) pass_a = plan_mix_axis(n0, n1, nch, cus, 1);
   slab = FftSlab{};
   if (n0 == n1 && n1 == n2 && (n0 == 128 || n0 == 64)) {
     const size_t nc = n2 / 2;
@@ -716,9 +723,10 @@ void ForceField::rebuild_sort() {
   // One workgroup sorts a system whose cells and ids fit its LDS and whose
   // atoms are few per thread (kNblSortSmall); beyond that the four launches
   // win on the steps that do rebuild.
+  const uint32_t n_rule = std::max(n, c.batch.atoms);
   const size_t small_lds = 4 * (size_t)((n_keys + 255u) & ~255u) + 2 * (size_t)((n + 3u) & ~3u);
-  if (n <= kNblSortSmall && small_lds + 64 <= c.max_lds) {
-    if (n > kNblKeysInline) {   // the keys' arithmetic is too much for one CU
+  if (n_rule <= kNblSortSmall && small_lds + 64 <= c.max_lds) {
+    if (n_rule > kNblKeysInline) {   // the keys' arithmetic is too much for one CU
       kp.cell_count = nullptr;
       launch(c, K_hmd_nbl_keys, ceil_div(n, 256), 256, 0, kp);
     }
@@ -777,7 +785,7 @@ void ForceField::rebuild_list() {
          bd);
   // up to kNblCountInline clusters every workgroup of the work-list kernel adds
   // up the counts below its own (16 KB at most); beyond, they are scanned
-  const bool scan = n_clusters > kNblCountInline;
+  const bool scan = std::max(n_clusters, ceil_div(c.batch.atoms, HMD_CLUSTER)) > kNblCountInline;
   if (scan) entry_scan.run(c, entry_count.ptr, entry_offset.ptr, gate, HMD_STATUS_DISPLACED);
   NblWorkParams wp{entry_count.ptr, scan ? entry_offset.ptr : nullptr, n_clusters, cap_entries,
                    work.ptr, n_work.ptr, status.ptr};
@@ -907,7 +915,8 @@ void ForceField::spme_forces(bool fev, bool mark_binned) {
   SpmeBinParams bp{p.posq.ptr, sorted_id.ptr, n, L, n0, n1, n2, brick[0], brick[1], brick[2],
                    nb[0], nb[1], nb[2], atom_bin.ptr, bin_count.ptr, bin_start.ptr,
                    bin_atoms.ptr};
-  if (n <= HMD_SPME_BIN_SMALL && n_bins <= 4096u) {
+  if (std::max(n, c.batch.atoms) <= HMD_SPME_BIN_SMALL &&
+      std::max(n_bins, c.batch.bins) <= 4096u) {
     launch(c, K_hmd_spme_bin_small, 1, 1024, 0, bp);
   } else {
     launch(c, K_hmd_spme_bin, ceil_div(n, 256), 256, 0, bp);
@@ -919,6 +928,22 @@ void ForceField::spme_forces(bool fev, bool mark_binned) {
 
   SpmeSpreadParams sp{p.posq.ptr, n, L, n0, n1, n2, brick[0], brick[1], brick[2],
                       nb[0], nb[1], nb[2], bin_start.ptr, bin_atoms.ptr, rho.ptr};
+  // A batch fills the chip together (above).  With energies the a-axis pass
+  // keeps the box's own shape: its partials' order is that of the box alone,
+  // and so is every bit of the virials.
+  FftPass r2c = pass_r2c, c2r = pass_c2r, axis_a = pass_a, axis_b = pass_b;
+  uint32_t n_partials = partial_blocks;
+  if (c.rec && !slab.on) {
+    const uint32_t cus = (uint32_t)c.num_cus, nbox = c.batch.boxes;
+    if (r2c.mix) r2c = plan_mix_lines(n2 / 2, n0 * n1, cus, nbox, true);
+    if (c2r.mix) c2r = plan_mix_lines(n2 / 2, n0 * n1, cus, nbox, false);
+    if (axis_b.mix) axis_b = plan_mix_axis(n1, n0, nch, cus, nbox);
+    if (axis_a.mix && !fev) {
+      axis_a = plan_mix_axis(n0, n1, nch, cus, nbox);
+      n_partials = axis_a.grid;   // no more than the box alone has
+    }
+  }
+
   const size_t sh_spread = (size_t)brick[0] * brick[1] * brick[2] * 8;
   KernelId ks = order == 4 ? K_hmd_spme_spread_p4
                 : order == 5 ? K_hmd_spme_spread_p5
@@ -971,9 +996,9 @@ void ForceField::spme_forces(bool fev, bool mark_binned) {
     FftParams& r = q;
     r.n_stages = (uint32_t)rad_c.size();
     for (size_t k = 0; k < rad_c.size(); ++k) r.radix[k] = rad_c[k];
-    if (pass_r2c.p2 || pass_r2c.mix) {
-      pass_r2c.set(q);
-      launch(c, pass_r2c.k, pass_r2c.grid, 256, pass_r2c.shmem, q);
+    if (r2c.p2 || r2c.mix) {
+      r2c.set(q);
+      launch(c, r2c.k, r2c.grid, 256, r2c.shmem, q);
     } else {
       launch(c, K_hmd_fft_r2c_c, ceil_div(q.n_lines, q.lines_per_block), 256,
              2 * (size_t)q.lines_per_block * (q.n + 1) * 8, q);
@@ -995,10 +1020,10 @@ void ForceField::spme_forces(bool fev, bool mark_binned) {
   for (size_t k = 0; k < rad_b.size(); ++k) fb.radix[k] = rad_b[k];
   const size_t sh_b = 2 * (size_t)fb.lines_per_block * (n1 + 1) * 8;
   auto launch_b = [&]() {
-    if (pass_b.p2 || pass_b.mix) {
+    if (axis_b.p2 || axis_b.mix) {
       FftParams q = fb;
-      pass_b.set(q);
-      launch(c, pass_b.k, pass_b.grid, 256, pass_b.shmem, q);
+      axis_b.set(q);
+      launch(c, axis_b.k, axis_b.grid, 256, axis_b.shmem, q);
     } else {
       launch(c, K_hmd_fft_axis, ceil_div(fb.n_lines, fb.lines_per_block), 256, sh_b, fb);
     }
@@ -1020,9 +1045,9 @@ void ForceField::spme_forces(bool fev, bool mark_binned) {
   set_radix(rad_a);
   fa.n_stages = f.n_stages;
   for (int k = 0; k < 8; ++k) fa.radix[k] = f.radix[k];
-  if (pass_a.p2 || pass_a.mix) {
-    pass_a.set(fa);
-    launch(c, pass_a.k, pass_a.grid, 256, pass_a.shmem, fa);   // data + (G, vf) tiles
+  if (axis_a.p2 || axis_a.mix) {
+    axis_a.set(fa);
+    launch(c, axis_a.k, axis_a.grid, 256, axis_a.shmem, fa);   // data + (G, vf) tiles
   } else {
     launch(c, K_hmd_fft_axis, ceil_div(fa.n_lines, fa.lines_per_block), 256,
            2 * (size_t)fa.lines_per_block * (n0 + 1) * 8, fa);
@@ -1042,9 +1067,9 @@ void ForceField::spme_forces(bool fev, bool mark_binned) {
     q.sign = +1;
     q.n_stages = (uint32_t)rad_c.size();
     for (size_t k = 0; k < rad_c.size(); ++k) q.radix[k] = rad_c[k];
-    if (pass_c2r.p2 || pass_c2r.mix) {
-      pass_c2r.set(q);
-      launch(c, pass_c2r.k, pass_c2r.grid, 256, pass_c2r.shmem, q);
+    if (c2r.p2 || c2r.mix) {
+      c2r.set(q);
+      launch(c, c2r.k, c2r.grid, 256, c2r.shmem, q);
     } else {
       launch(c, K_hmd_fft_c2r_c, ceil_div(q.n_lines, q.lines_per_block), 256,
              2 * (size_t)q.lines_per_block * (q.n + 1) * 8, q);
@@ -1054,8 +1079,8 @@ void ForceField::spme_forces(bool fev, bool mark_binned) {
   c.mark("spme_fft_solve");
   SpmeGatherParams gp{p.posq.ptr, n, L, n0, n1, n2, brick[0], brick[1], brick[2],
                       nb[0], nb[1], nb[2], bin_start.ptr, bin_atoms.ptr, V.ptr,
-                      u_self.ptr, partials.ptr, partial_blocks, spme_out.ptr, slow_f.ptr, slow_e.ptr, slow_w.ptr,
-                      fev ? 1u : 0u};
+                      u_self.ptr, partials.ptr, n_partials, spme_out.ptr, slow_f.ptr,
+                      slow_e.ptr, slow_w.ptr, fev ? 1u : 0u};
   const size_t sh_gather = (size_t)(brick[0] + order - 1) * (brick[1] + order - 1) *
                            (brick[2] + order - 1) * 4;
   KernelId kg = order == 4 ? K_hmd_spme_gather_p4

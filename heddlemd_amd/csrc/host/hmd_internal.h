@@ -83,6 +83,15 @@ struct LaunchRec {
   std::vector<unsigned char> params;
 };
 
+// Extents of the set of boxes that a batched step is recorded for.  Its boxes
+// share each stage's launch, so a stage takes the variant that suits its
+// largest box (two variants run one after the other: SPME binning of 64 boxes
+// either side of 6,144 atoms 43.9 us a step, 33.6 with one) and the launch
+// shapes that suit all of them together.
+struct BatchExtents {
+  uint32_t boxes = 1, atoms = 0, bins = 0;
+};
+
 struct Context {
   int device = 0;
   int num_cus = 0;
@@ -95,6 +104,7 @@ struct Context {
   hipFunction_t fn_batch[K_COUNT] = {};   // NAME_batch twins (null where absent)
   // When set, launches are appended here instead of being issued.
   std::vector<LaunchRec>* rec = nullptr;
+  BatchExtents batch;   // while recording
   // Optional per-stage event recording (profile mode, eager only).
   bool profiling = false;
   std::vector<std::pair<std::string, hipEvent_t>> marks;

@@ -621,16 +621,25 @@ struct ReplicaSet {
     release();
     const size_t R = its.size();
     std::vector<std::vector<LaunchRec>> recs(R);
+    BatchExtents ext;
+    ext.boxes = (uint32_t)R;
+    for (auto* it : its) {
+      ext.atoms = std::max(ext.atoms, it->ff->n);
+      ext.bins = std::max(ext.bins, it->ff->n_bins);
+    }
     for (size_t r = 0; r < R; ++r) {
       Context& c = its[r]->c;
       c.rec = &recs[r];
+      c.batch = ext;
       try {
         its[r]->enqueue_step();
       } catch (...) {
         c.rec = nullptr;
+        c.batch = BatchExtents{};
         throw;
       }
       c.rec = nullptr;
+      c.batch = BatchExtents{};
     }
     struct Item {
       const LaunchRec* first;                // kernel, block size

@@ -101,3 +101,47 @@ def test_per_replica_logs_byte_reproducible(tmp_path):
         a = (tmp_path / "a" / f"replica{rid}.out.log").read_bytes()
         b = (tmp_path / "b" / f"replica{rid}.out.log").read_bytes()
         assert a == b and a.count(b"\n") == 1 + STEPS // 10 + 1
+
+
+# A box of 216 molecules beside one across a bound at which the box alone takes
+# other kernels: 6,144 atoms (SPME binning), 12,288 atoms (cell sort).
+@pytest.mark.parametrize("n_mol, mesh", [(4006, 48), (4200, 50)])
+def test_batch_of_unlike_boxes_takes_one_variant(n_mol, mesh):
+    """Every stage is one launch over both boxes (the launches of the larger
+    box alone), and both end as they do alone, byte by byte."""
+    specs = [SPECS[25], {"replica": 900, "n_mol": n_mol, "r_cut_nm": 1.0,
+                         "mesh": (mesh, mesh, mesh), "seed": 77}]
+
+    def run_set(ids, batched):
+        reps = []
+        for k in ids:
+            ctx = api.GpuContext(0)
+            sysw, ff, part, field, integ = replica_case(ctx, specs[k], relax=20,
+                                                        kind="langevin-baoab",
+                                                        temperature=U.kelvin(300.0))
+            part.upload(vel=api.generate_velocities(sysw["mass"], U.kelvin(300.0), 5 + k,
+                                                    n_constraints=3 * sysw["n_mol"]))
+            reps.append((ctx, part, field, integ, sysw))
+        try:
+            plan = None
+            if batched:
+                rs = api.ReplicaSet([r[3] for r in reps], mode="batched")
+                try:
+                    rs.step(12)
+                    plan = rs.plan()
+                finally:
+                    rs.close()
+            else:
+                reps[0][3].replay(12)
+            return state(reps), plan
+        finally:
+            close(reps)
+
+    both, (nb, ns) = run_set([0, 1], True)
+    _, (nb1, ns1) = run_set([1], True)
+    print(f"launches: {nb} + {ns} for both, {nb1} + {ns1} for the larger alone")
+    assert (nb, ns) == (nb1 + ns1, 0)
+    for k in (0, 1):
+        alone, _ = run_set([k], False)
+        assert alone[0][0].tobytes() == both[k][0].tobytes()
+        assert alone[0][1].tobytes() == both[k][1].tobytes()

@@ -1077,6 +1077,12 @@ void ForceField::spme_forces(bool fev, bool mark_binned) {
   }
   }
   c.mark("spme_fft_solve");
+  // (in a batch one launch sums them for every box)
+  if (fev && (c.rec || (uint64_t)n_partials * n_bins > kSpmeSumInGather)) {
+    const SpmeReduceParams rp{partials.ptr, n_partials, spme_out.ptr};
+    launch(c, K_hmd_spme_reduce, 1, 256, 0, rp);
+    n_partials = 0;
+  }
   SpmeGatherParams gp{p.posq.ptr, n, L, n0, n1, n2, brick[0], brick[1], brick[2],
                       nb[0], nb[1], nb[2], bin_start.ptr, bin_atoms.ptr, V.ptr,
                       u_self.ptr, partials.ptr, n_partials, spme_out.ptr, slow_f.ptr,

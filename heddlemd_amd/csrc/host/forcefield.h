@@ -45,6 +45,13 @@ constexpr uint32_t kNblKeysInline = 5120;
 // us a frame, 24,576 156 -> 161.
 constexpr uint32_t kPairTeam = 1536;
 constexpr uint32_t kPairTeamBlocks = 1280;
+// Partials times bricks up to which the workgroups of the gather add up the
+// solve's partials themselves on an evaluation with energies (1.57 million).
+// Summed there or in a launch of their own, us an evaluation: 90,000 atoms on
+// 108^3 (0.55 million) 343.5 and 345.8, 60,000 on 96^3 (1.16 million) 275.5 and
+// 279.4, 120,000 on 120^3 (3.2 million) 417.5 and 414.4, 196,608 on 144^3 (2.1
+// million) 565 and 562, on 256^3 (19 million) 940 and 925.
+constexpr uint64_t kSpmeSumInGather = 3u << 19;
 // Clusters up to which the work-list kernel adds up the entry counts itself.
 constexpr uint32_t kNblCountInline = 4096;
 constexpr double kNblFillThreshold = 0.8;

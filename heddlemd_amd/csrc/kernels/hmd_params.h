@@ -300,6 +300,12 @@ struct SpmeSpreadParams {
   float* rho;                  // real mesh [n0*n1*n2]
 };
 
+struct SpmeReduceParams {
+  const double* partials;      // [n_partials][2] of the a-axis pass
+  uint32_t n_partials;
+  double* totals;              // [2] reciprocal virial and energy
+};
+
 struct SpmeGatherParams {
   const float* posq;
   uint32_t n;
@@ -312,7 +318,7 @@ struct SpmeGatherParams {
   const float* V;              // real mesh
   const float* u_self;         // [n]
   const double* partials;      // [n_partials][2] of the a-axis pass
-  uint32_t n_partials;
+  uint32_t n_partials;         // 0: hmd_spme_reduce has summed them
   double* totals;              // [2] reciprocal virial and energy
   float* f;                    // [3][n] canonical, overwritten
   float* e;                    // [n]

@@ -403,6 +403,41 @@ __device__ inline void hmd_spread_body(const SpmeSpreadParams& p, const uint32_t
   }
 }
 
+// The solve's reciprocal virial and energy (x, y) from its partials, summed in
+// FP64 in a fixed order by a workgroup of 256: W = 0.5 sum hw vf |rho|^2,
+// U = 0.5 sum hw G |rho|^2 (kernels/spme_recip.cu:376-402).
+__device__ inline double2 hmd_spme_totals(const double* partials, uint32_t n) {
+  __shared__ double2 s_part[4];
+  double2 t = make_double2(0.0, 0.0);
+  for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) {
+    t.x += partials[2 * k];
+    t.y += partials[2 * k + 1];
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    t.x += __shfl_xor(t.x, o, HMD_WAVE);
+    t.y += __shfl_xor(t.y, o, HMD_WAVE);
+  }
+  if (hmd_lane() == 0) s_part[threadIdx.x / HMD_WAVE] = t;
+  __syncthreads();
+  t.x = 0.5 * ((s_part[0].x + s_part[1].x) + (s_part[2].x + s_part[3].x));
+  t.y = 0.5 * ((s_part[0].y + s_part[1].y) + (s_part[2].y + s_part[3].y));
+  return t;
+}
+
+// The totals in a launch of their own, where the gather's workgroups would
+// read too much for it (kSpmeSumInGather).
+__device__ __forceinline__ void hmd_spme_reduce_body(const SpmeReduceParams& p,
+                                                     const uint32_t hmd_bx,
+                                                     const uint32_t hmd_gx) {
+  const double2 t = hmd_spme_totals(p.partials, p.n_partials);
+  if (threadIdx.x == 0) *reinterpret_cast<double2*>(p.totals) = t;
+}
+HMD_KERNEL(hmd_spme_reduce, SpmeReduceParams, 256)
+
+// The partials of the solve are summed by every workgroup that hands the
+// virial out (and by the first, which keeps the totals) while there are few:
+// hmd_spme_reduce costs a launch.
 template <int P>
 __device__ inline void hmd_gather_body(const SpmeGatherParams& p, const uint32_t hmd_bx,
     const uint32_t hmd_gx) {
@@ -413,33 +448,12 @@ __device__ inline void hmd_gather_body(const SpmeGatherParams& p, const uint32_t
   const int o0 = (int)(B0 * p.b0) - (P - 1);
   const int o1 = (int)(B1 * p.b1) - (P - 1);
   const int o2 = (int)(B2 * p.b2) - (P - 1);
-  // The solve's virial and energy partials, summed in FP64 in a fixed order by
-  // every workgroup that hands the virial out (and by the first, which keeps
-  // the totals): a launch of its own for this sum took 2.4 to 4.7 us.  W = 0.5
-  // sum hw vf |rho|^2, U = 0.5 sum hw G |rho|^2 (kernels/spme_recip.cu:376-402).
-  double tot_e = 0.0, tot_w = 0.0;
-  if (p.fev || hmd_bx == 0) {
-    __shared__ double s_part[2][4];
-    for (uint32_t k = threadIdx.x; k < p.n_partials; k += blockDim.x) {
-      tot_w += p.partials[2 * k];
-      tot_e += p.partials[2 * k + 1];
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      tot_e += __shfl_xor(tot_e, o, HMD_WAVE);
-      tot_w += __shfl_xor(tot_w, o, HMD_WAVE);
-    }
-    if (hmd_lane() == 0) {
-      s_part[0][threadIdx.x / HMD_WAVE] = tot_e;
-      s_part[1][threadIdx.x / HMD_WAVE] = tot_w;
-    }
-    __syncthreads();
-    tot_e = 0.5 * ((s_part[0][0] + s_part[0][1]) + (s_part[0][2] + s_part[0][3]));
-    tot_w = 0.5 * ((s_part[1][0] + s_part[1][1]) + (s_part[1][2] + s_part[1][3]));
-    if (hmd_bx == 0 && threadIdx.x == 0) {
-      p.totals[0] = tot_w;
-      p.totals[1] = tot_e;
-    }
+  double2 tot = make_double2(0.0, 0.0);
+  if (p.n_partials == 0) {
+    if (p.fev) tot = *reinterpret_cast<const double2*>(p.totals);
+  } else if (p.fev || hmd_bx == 0) {
+    tot = hmd_spme_totals(p.partials, p.n_partials);
+    if (hmd_bx == 0 && threadIdx.x == 0) *reinterpret_cast<double2*>(p.totals) = tot;
   }
   const float ih2 = 1.0f / (float)h2, ih1 = 1.0f / (float)h1;
   for (uint32_t k = threadIdx.x; k < h0 * h1 * h2; k += blockDim.x) {
@@ -461,7 +475,7 @@ __device__ inline void hmd_gather_body(const SpmeGatherParams& p, const uint32_t
               ba_z = (L.xy * L.yz - L.xz * L.ly) * ilx * ily * ilz;
   const float bb_y = ily, bb_z = -L.yz * ily * ilz;
   const float bc_z = ilz;
-  const float w_share = (float)(tot_w / (double)p.n);
+  const float w_share = (float)(tot.x / (double)p.n);
 
   const uint32_t beg = p.bin_start[B], end = p.bin_start[B + 1];
   for (uint32_t k = beg + threadIdx.x; k < end; k += blockDim.x) {

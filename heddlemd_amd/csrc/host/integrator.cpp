@@ -358,12 +358,7 @@ struct Integrator {
     sp.lan = lan(dt);
     sp.free_atoms = n_groups ? free_atoms.ptr : nullptr;
     sp.n_free = n_free;
-    // a small box alone is latency: few groups a workgroup, the normals in one
-    // round; the boxes of a batch fill the chip together, where 16 of 256 lanes
-    // in the constraint solves cost more (64 boxes: 71 us a launch, the batch
-    // 1.16 ms a step, 1.12 with full waves; 16 boxes: the same)
-    sp.groups_per_block = n_groups <= 4096 && !c.rec ? 16u : 64u;
-    sp.group_blocks = ceil_div(n_groups, sp.groups_per_block);
+    sp.group_blocks = ceil_div(n_groups, HMD_BAOA_GROUPS);
     sp.dt = dt;
     sp.counter = kind == Kind::LangevinBaoab ? step_counter.ptr : nullptr;
     // the first fused kernel runs the force field's skin check

@@ -400,6 +400,7 @@ struct LangevinParams {
   uint32_t n;
 };
 
+#define HMD_BAOA_GROUPS 64u    // groups a workgroup of hmd_step_baoa takes
 // Fused integrator sub-steps (hmd_step_*): the per-op parameter blocks,
 // the free (unconstrained) atoms and the Langevin draw counter.
 struct StepParams {
@@ -408,8 +409,7 @@ struct StepParams {
   LangevinParams lan;
   const uint32_t* free_atoms;  // [n_free]; null: atoms 0..n_free-1
   uint32_t n_free;
-  uint32_t groups_per_block;   // hmd_step_baoa: groups a workgroup takes (<= 64)
-  uint32_t group_blocks;       // and the workgroups that take groups
+  uint32_t group_blocks;       // hmd_step_baoa: workgroups that take groups
   float dt;
   unsigned long long* counter; // Langevin draw counter (null for VV)
   NblDispParams disp;          // the force field's skin check on the new

@@ -685,12 +685,13 @@ HMD_KERNEL(hmd_step_vv_first, StepParams, 256)
 
 // Langevin BAOAB up to the force evaluation: B [SETTLE v] [snapshot] A
 // [SETTLE x, dt/2] O [SETTLE v] [snapshot] A [SETTLE x, dt/2] [skin check].
-// A workgroup of 256 threads takes groups_per_block groups: all its threads
+// A workgroup of 256 threads takes HMD_BAOA_GROUPS groups: all its threads
 // draw the groups' normals first (nine a group; a Philox block and an FP64
 // log, square root and cosine each, half of the kernel's time when the
 // group's own thread drew them one after the other), then a thread a group
-// runs the sub-steps.  Blocks past group_blocks take 256 free atoms each.
-#define HMD_BAOA_GROUPS 64u
+// runs the sub-steps: one full wave (16 groups a workgroup, which draw in one
+// round, took 1.1 us a step more at 216 and at 1,000 groups, 1.6 at 4,096, 7 at
+// 16,384).  Blocks past group_blocks take 256 free atoms each.
 __device__ __forceinline__ void hmd_step_baoa_body(const StepParams& p, const uint32_t hmd_bx,
     const uint32_t hmd_gx) {
   __shared__ float s_xi[9 * HMD_BAOA_GROUPS];
@@ -718,8 +719,8 @@ __device__ __forceinline__ void hmd_step_baoa_body(const StepParams& p, const ui
       atomicOr(p.disp.status, HMD_STATUS_DISPLACED);
     return;
   }
-  const uint32_t g0 = hmd_bx * p.groups_per_block;
-  const uint32_t ng = min(p.groups_per_block, p.st.n_groups - g0);
+  const uint32_t g0 = hmd_bx * HMD_BAOA_GROUPS;
+  const uint32_t ng = min(HMD_BAOA_GROUPS, p.st.n_groups - g0);
   const bool mine = threadIdx.x < ng;
   const uint32_t g = g0 + threadIdx.x;
   HmdGroup G;

@@ -86,7 +86,7 @@ struct LaunchRec {
 // Extents of the set of boxes that a batched step is recorded for.  Its boxes
 // share each stage's launch, so a stage takes the variant that suits its
 // largest box (two variants run one after the other: SPME binning of 64 boxes
-// either side of 6,144 atoms 43.9 us a step, 33.6 with one) and the launch
+// either side of its bound 43.9 us a step, 33.6 with one) and the launch
 // shapes that suit all of them together.
 struct BatchExtents {
   uint32_t boxes = 1, atoms = 0, bins = 0;

@@ -286,7 +286,10 @@ struct SpmeBinParams {
   uint32_t* bin_start;         // [n_bins+1] (written by hmd_spme_bin_small alone)
   uint32_t* bin_atoms;         // [n]
 };
-#define HMD_SPME_BIN_SMALL 6144u   // atoms of the one-workgroup binning
+// Atoms of the one-workgroup binning.  Against the three launches, us a step:
+// 648 atoms 83.7 and 91.5, 2,400 103.0 and 107.4, 4,500 122.2 and 122.8, 5,400
+// 116.9 and 116.5, 6,144 125.7 and 123.7.
+#define HMD_SPME_BIN_SMALL 5120u
 
 struct SpmeSpreadParams {
   const float* posq;

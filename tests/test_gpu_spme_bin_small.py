@@ -1,4 +1,4 @@
-"""SPME binning in one workgroup (at most 6,144 atoms and 4,096 bins) and the
+"""SPME binning in one workgroup (at most 5,120 atoms and 4,096 bins) and the
 reciprocal sums taken by the gather, at the edges of both: a partial round of
 atoms per thread, the last size of the path and the first beyond, a full and
 an overfull table of bins.  Bars of the other mesh tests (f32 mesh)."""
@@ -16,7 +16,8 @@ FORCE_TOL, ENERGY_TOL = 1e-5, 1e-6
 
 @pytest.mark.parametrize("n_mol, mesh, brick", [
     (216, (24, 24, 24), (0, 0, 0)), (341, (24, 24, 24), (8, 8, 8)), (342, (32, 24, 20), (4, 4, 4)),
-    (1366, (32, 32, 32), (8, 8, 8)), (2048, (48, 48, 48), (0, 0, 0)),
+    (1366, (32, 32, 32), (8, 8, 8)), (1706, (48, 48, 48), (0, 0, 0)),
+    (1707, (48, 48, 48), (0, 0, 0)), (2048, (48, 48, 48), (0, 0, 0)),
     (2049, (48, 48, 48), (0, 0, 0)), (1024, (64, 64, 64), (4, 4, 4)),
     (1024, (72, 64, 64), (4, 4, 4))])
 def test_small_binning(gpu_ctx, n_mol, mesh, brick):

@@ -782,8 +782,6 @@ void ForceField::rebuild_list() {
 #endif
   launch(c, K_hmd_nbl_build, n_clusters, 64 * HMD_NBL_WAVES, chunk_lds + (size_t)bd.lds_slots * 4,
          bd);
-  // up to kNblCountInline clusters every workgroup of the work-list kernel adds
-  // up the counts below its own (16 KB at most); beyond, they are scanned
   const bool scan = std::max(n_clusters, ceil_div(c.batch.atoms, HMD_CLUSTER)) > kNblCountInline;
   if (scan) entry_scan.run(c, entry_count.ptr, entry_offset.ptr, gate, HMD_STATUS_DISPLACED);
   NblWorkParams wp{entry_count.ptr, scan ? entry_offset.ptr : nullptr, n_clusters, cap_entries,

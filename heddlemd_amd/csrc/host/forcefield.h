@@ -54,8 +54,13 @@ constexpr uint32_t kPairTeamBlocks = 1280;
 // 279.4, 120,000 on 120^3 (3.2 million) 417.5 and 414.4, 196,608 on 144^3 (2.1
 // million) 565 and 562, on 256^3 (19 million) 940 and 925.
 constexpr uint64_t kSpmeSumInGather = 3u << 19;
-// Clusters up to which the work-list kernel adds up the entry counts itself.
-constexpr uint32_t kNblCountInline = 4096;
+// Clusters up to which every workgroup of the work-list kernel adds up the entry
+// counts below its own (32 KB at most) instead of reading their scan.  An
+// evaluation that rebuilds, us: 100,000 atoms 197.5 and 202 with the scan,
+// 300,000 502 and 515, 524,288 (8,192 clusters) 915 and 922, 1,000,000 1,819
+// and 1,808; a step without a rebuild saves the scan's launches, 1.6 us for one
+// tile of counts and 5 for more (10,000, 300,000 atoms).
+constexpr uint32_t kNblCountInline = 8192;
 constexpr double kNblFillThreshold = 0.8;
 
 struct ForceField {

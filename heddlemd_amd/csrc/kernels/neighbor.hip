@@ -806,8 +806,8 @@ __device__ __forceinline__ void hmd_nbl_build_body(const NblBuildParams& p, cons
 HMD_KERNEL(hmd_nbl_build, NblBuildParams, 64 * HMD_NBL_WAVES, HMD_NBL_BUILD_WAVES_PER_EU)
 
 // Work list: cluster c's entries at the sum of the lower clusters' counts
-// (n_offsets == 0: taken here, every workgroup of four clusters adding up the
-// counts below its own, 12 KB at 196,608 atoms; else scanned by a launch
+// (entry_offset null: taken here, every workgroup of four clusters adding up the
+// counts below its own, 12 KB at 196,608 atoms; else scanned by launches
 // before).  The last workgroup to finish closes the rebuild -- work-list
 // length, status flags, generation -- when every one has read the gate.
 __device__ __forceinline__ void hmd_nbl_worklist_body(const NblWorkParams& p, const uint32_t hmd_bx,

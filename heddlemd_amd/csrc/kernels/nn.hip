@@ -27,6 +27,7 @@
 //    turned by the transposing LDS read; per-wave partials are summed in a fixed
 //    order by hmd_nn_grad_reduce.
 #include "hmd_device.h"
+#include "nn_items.h"
 
 typedef __bf16 hmd_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float hmd_f32x4 __attribute__((ext_vector_type(4)));
@@ -139,30 +140,6 @@ hmd_nn_pack(const NnPackParams p) {
   if (tid == 0u) p.vec[192] = b3[0];
 }
 
-// How the passes share the list: an item is an entry, or one of its
-// 2^split groups of i-sub-clusters, and wave v of n takes the items v, v + n,
-// ...  An entry of a dense liquid holds 0 to 4,096 pairs (about 1,000 on
-// average), so a short list is split until there are HMD_NN_ITEMS items (or
-// eight groups an entry): eight of the 2,048 waves the chip holds of the
-// forward pass.  Whole entries in contiguous shares left a CU with 1.2 of 8
-// waves running on average at 9,999 atoms.
-#define HMD_NN_ITEMS 16384u
-struct HmdNnItems {
-  uint32_t n, split;
-  __device__ HmdNnItems(uint32_t entries, uint32_t want) : split(0) {
-    while (split < 3u && (entries << split) < want) ++split;
-    n = entries << split;
-  }
-  __device__ uint32_t entry(uint32_t w) const { return w >> split; }
-  // the group turns with the wave's round: the first and last i-sub-clusters
-  // of an entry hold different numbers of pairs, and the number of waves is a
-  // multiple of eight
-  __device__ uint32_t mask(uint32_t w, uint32_t round) const {
-    const uint32_t group = 8u >> split;
-    return ((1u << group) - 1u) << (group * ((w + round) & ((1u << split) - 1u)));
-  }
-};
-
 // Single-image shift of a cluster (compare jit_composed.rs:1396-1430, as in
 // the pair kernel): valid when every atom within r_cut + r_skin/2 of the
 // cluster lies within half a box of its centre; positions are then moved to
@@ -234,9 +211,9 @@ hmd_nn_descriptors(const NnPassParams p) {
       if (vi) hmd_atomic_add_fixed(&acc[k * stride + si], hmd_to_fixed(v, HMD_NN_DESC_SHIFT));
     }
   };
-  for (uint32_t w = gw, round = 0; w < items.n; w += n_waves, ++round) {
+  for (uint32_t w = gw; w < items.n; w += n_waves) {
     const uint32_t slot = __builtin_amdgcn_readfirstlane(p.work[items.entry(w)]);
-    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w, round);
+    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w, n_waves);
     if (pend == 0u) continue;
     const uint32_t c = slot / p.cap_entries;
     const uint32_t c0 = c * HMD_CLUSTER;
@@ -541,9 +518,9 @@ hmd_nn_forward(const NnPassParams p) {
   uint32_t cur_c = HMD_SENTINEL, si = 0, n_i = 0;
   bool vi = false;
   HmdNnShift sh{false, 0.0f, 0.0f, 0.0f};
-  for (uint32_t w = gw, round = 0; w < items.n; w += n_waves, ++round) {
+  for (uint32_t w = gw; w < items.n; w += n_waves) {
     const uint32_t slot = __builtin_amdgcn_readfirstlane(p.work[items.entry(w)]);
-    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w, round);
+    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w, n_waves);
     if (pend == 0u) continue;
     const uint32_t c = slot / p.cap_entries;
     const uint32_t my_j = p.entry_j[(size_t)slot * HMD_ENTRY + lane];
@@ -816,9 +793,9 @@ hmd_nn_backward(const NnPassParams p) {
 
   uint32_t cur_c = HMD_SENTINEL, n_i = 0;
   HmdNnShift sh{false, 0.0f, 0.0f, 0.0f};
-  for (uint32_t w = gw, round = 0; w < items.n; w += n_waves, ++round) {
+  for (uint32_t w = gw; w < items.n; w += n_waves) {
     const uint32_t slot = __builtin_amdgcn_readfirstlane(p.work[items.entry(w)]);
-    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w, round);
+    uint32_t pend = __builtin_amdgcn_readfirstlane(p.entry_mask[slot]) & items.mask(w, n_waves);
     if (pend == 0u) continue;
     const uint32_t c = slot / p.cap_entries;
     const uint32_t my_j = p.entry_j[(size_t)slot * HMD_ENTRY + lane];

@@ -116,6 +116,7 @@ struct ForceField {
   void autotune(uint32_t n_evals, hmd_tuning* out);
   void set_tuning(const hmd_tuning& t);
   void get_tuning(hmd_tuning* t) const;
+  bool fft_grid_tunable() const;
   double time_compute(uint32_t n_evals);
   void check_brick(const uint32_t b[3]) const;
   void alloc_bins();

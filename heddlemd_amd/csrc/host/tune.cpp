@@ -85,6 +85,13 @@ void ForceField::set_tuning(const hmd_tuning& t) {
   graph_invalid = true;
 }
 
+// Whether fft_blocks_per_cu shapes any pass: the power-of-two line passes take
+// it; the mixed-length, Stockham and slab passes have shapes of their own, and
+// timing its values on them would record noise.
+bool ForceField::fft_grid_tunable() const {
+  return !slab.on && (pass_r2c.p2 || pass_c2r.p2 || pass_a.p2 || pass_b.p2);
+}
+
 // Brick shapes: per axis the divisors of the mesh in [order, 32], combined
 // with b0 >= b1 >= b2 and 512..4096 points, that fit the LDS of the spread
 // (i64 per point) and of the gather (f32 per halo point).
@@ -140,7 +147,7 @@ void ForceField::autotune(uint32_t n_evals, hmd_tuning* out) {
   }
   if (spme_on) {
     for (uint32_t v : kFftCandidates) {
-      if (v == best.fft_blocks_per_cu) continue;
+      if (!fft_grid_tunable() || v == best.fft_blocks_per_cu) continue;
       hmd_tuning t = best;
       t.fft_blocks_per_cu = v;
       trial(t);

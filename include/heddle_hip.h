@@ -511,7 +511,9 @@ hmd_status hmd_settle_after_kick(hmd_settle* s, float dt);
  *                       entries).  The f32 per-wave force sums follow the
  *                       work split, so each value gives reproducible results
  *                       that differ from another value's in the last bits;
- *   fft_blocks_per_cu   FFT-pass workgroups per CU (forces unchanged);
+ *   fft_blocks_per_cu   FFT-pass workgroups per CU (forces unchanged) of the
+ *                       axes whose length is a power of two; others, and the
+ *                       slab path, ignore it;
  *   brick[3]            SPME spread / gather brick (forces unchanged: the
  *                       mesh sums are exact integers);
  *   spme_stream         1: SPME runs on a second stream beside the pair

@@ -105,3 +105,21 @@ def test_replayed_steps_after_retuning(gpu_ctx):
             integ.close(); field.close(); part.close()
     assert states[0][0].tobytes() == states[1][0].tobytes()
     assert states[0][1].tobytes() == states[1][1].tobytes()
+
+
+def test_fft_grid_is_tuned_only_where_it_shapes_a_pass(gpu_ctx):
+    """On 24^3 every FFT pass has a shape of its own: the candidates are the
+    one at entry, five pair grids, the other stream setting and at most eight
+    bricks, and the value at entry stays."""
+    from heddlemd_amd import systems
+    s = systems.spc_water_n(216, 3)
+    ff = systems.water_forcefield(r_cut_nm=0.8, grid=(24, 24, 24), exclusions=s["exclusions"])
+    part = api.ParticleBuffers(gpu_ctx, s["posq"], s["mass"], s["lattice"], types=s["types"])
+    field = api.ForceField(gpu_ctx, part, ff)
+    try:
+        before = field.tuning()["fft_blocks_per_cu"]
+        res = field.autotune(3)
+        print(f"24^3: {res['n_candidates']} candidates")
+        assert res["n_candidates"] <= 15 and res["fft_blocks_per_cu"] == before
+    finally:
+        field.close(); part.close()

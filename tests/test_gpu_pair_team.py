@@ -1,7 +1,8 @@
 """The pair kernel's two ways to share a list, either side of the number of
 entries where they change (1,536): a workgroup per entry for shorter lists,
 whole entries per wave for longer ones.  Forces and energies against the FP64
-oracle, and the same bytes for every launch shape.
+oracle, and the same bytes for every launch shape: 256 and 512 workgroups, which
+take several entries and clusters each, and as many as the list has work for.
 
 Force tolerance: both atoms of a pair are moved to the image nearest a cluster
 centre in f32, each by up to an ulp of L/2; at the lattice spacing a the r^-13
@@ -42,9 +43,10 @@ def jittered_argon(n, charged):
     return s, 26.0 * float(np.spacing(np.float32(0.5 * L))) / (L / side)
 
 
-@pytest.mark.parametrize("n, charged", [(1, 0), (63, 1), (130, 0), (1000, 1), (8000, 0), (8000, 1),
-                                        (12500, 0), (12500, 1), (17000, 1)])
-def test_forces_and_launch_shapes(gpu_ctx, n, charged):
+@pytest.mark.parametrize("n, charged, shared", [
+    (1, 0, True), (63, 1, True), (130, 0, True), (1000, 1, True), (8000, 0, True),
+    (8000, 1, True), (12500, 0, True), (12500, 1, True), (17000, 1, False)])
+def test_forces_and_launch_shapes(gpu_ctx, n, charged, shared):
     s, tol = jittered_argon(n, charged)
     part = api.ParticleBuffers(gpu_ctx, s["posq"], s["mass"], s["lattice"], types=s["types"])
     field = api.ForceField(gpu_ctx, part, s["ff"])
@@ -53,7 +55,7 @@ def test_forces_and_launch_shapes(gpu_ctx, n, charged):
     entries = field.stats()["n_work"]
     base = field.tuning()
     same = []
-    for blocks in (8, 16, 64):
+    for blocks in (1, 2, 32):
         field.set_tuning(dict(base, pair_blocks_per_cu=blocks))
         field.compute(1)
         same.append(part.forces().tobytes() == f.tobytes())
@@ -66,5 +68,8 @@ def test_forces_and_launch_shapes(gpu_ctx, n, charged):
     err_e = abs(e.astype(np.float64).sum() - e_ref.sum()) / max(np.abs(e_ref).sum(), 1e-30)
     print(f"{n} atoms, {entries} entries: forces {err:.2e}, energy {err_e:.2e}, "
           f"without energies {err_f0:.2e}")
+    assert (entries < 1536) == shared
+    if n >= 8000:
+        assert entries > 2 * 256          # several entries a workgroup of both small grids
     assert all(same)
     assert err <= tol and err_e <= 5e-6 and err_f0 <= 1e-6

@@ -203,10 +203,6 @@ __device__ inline float hmd_wave_sum8(const float v[8], uint32_t lane) {
   return c;
 }
 
-__device__ inline float hmd_readlane_f(float v, uint32_t lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), (int)lane));
-}
-
 // x / d for x < 2^21 from inv_d = 1.0f / d: (x + 1/2) / d is at least 1/(2d)
 // from an integer, and the two roundings move it by less than x / d 2^-22.
 __device__ inline uint32_t hmd_div_small(uint32_t x, float inv_d) {

@@ -79,11 +79,6 @@ __device__ inline float hmd_nn_cutoff(float s) {
   return 0.5f * (1.0f + __builtin_amdgcn_cosf(0.5f * s));
 }
 
-__device__ inline float hmd_nn_rbf(float u15, float k) {
-  const float t = u15 - k;
-  return __builtin_amdgcn_exp2f(-0.5f * HMD_NN_LOG2E * t * t);
-}
-
 // phi_{k0 + e}(x), e = 0..7, for x = 15 s, by the Gaussian product
 // recurrence phi_{k+1} = phi_k exp(x - k - 1/2), whose ratio itself shrinks
 // by e^-1 per step: two exponentials instead of eight.  From k0 = 0 the
@@ -609,7 +604,6 @@ __device__ inline void hmd_nn_load_shared(const NnPassParams& p, HmdNnShared& S)
 }
 
 typedef short hmd_s16x4 __attribute__((ext_vector_type(4)));
-typedef short hmd_s16x8 __attribute__((ext_vector_type(8)));
 
 // Column 16 t + l % 16 of a row-major [32][64] table as a matrix operand
 // whose k index runs over the rows: two transposing LDS reads, each giving
@@ -630,7 +624,7 @@ __device__ inline void hmd_nn_put4(uint16_t* row, uint32_t t, uint32_t g, hmd_bf
       half ? make_uint2(w[2], w[3]) : make_uint2(w[0], w[1]);
 }
 
-// SiLU value and derivative of four units; the value goes to h[at..at+3].
+// SiLU of four units: values to out, derivatives returned.
 __device__ inline hmd_f32x4 hmd_nn_silu_d(hmd_f32x4 z, float out[4]) {
   hmd_f32x4 d;
 #pragma unroll

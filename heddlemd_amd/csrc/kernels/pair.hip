@@ -13,9 +13,11 @@
 // closed form, and no reciprocal is taken unless the step has LJ.
 //
 // Mapping (wave64, VALU FP32; no MFMA -- there is no dense contraction):
-//  * one wave walks a contiguous share of the work list; an entry holds 64
-//    j-atoms of one 64-atom i-cluster's list, one j-atom per lane, gathered
-//    once (and shifted to the image nearest the cluster centre);
+//  * one wave walks a contiguous share of the work list, or, where the list
+//    is too short for that, the four waves of a workgroup share each entry by
+//    its i-sub-clusters (hmd_pair_body); an entry holds 64 j-atoms of one
+//    64-atom i-cluster's list, one j-atom per lane, gathered once (and shifted
+//    to the image nearest the cluster centre);
 //  * the i-cluster's atoms sit in a per-wave LDS table and are broadcast one
 //    per step by a wave-uniform LDS read, so each step evaluates 64 pairs
 //    with no global memory access and no shuffles;
@@ -234,7 +236,7 @@ __device__ inline uint32_t hmd_pair_part(uint32_t m8, uint32_t part) {
 // j-slots) are transposed so that each j lane holds its bits over the
 // i-atoms.  The j reaction is flushed once per entry: to memory, or, where the
 // workgroup's waves share the entry (s_j set, `part` of four), to the
-// workgroup's sums in LDS.  Returns the lane's j-atom.
+// workgroup's sums in LDS.
 template <bool FEV, bool LJ, bool COUL, bool SHIFT>
 __device__ inline void hmd_pair_entry(const PairParams& p, const float4* s_lj,
                                       const float4* s_ct, const float4* s_ip,

@@ -508,9 +508,8 @@ hmd_status hmd_settle_after_kick(hmd_settle* s, float dt);
  * No counterpart in the reference (its launch shapes are fixed).  The
  * shapes a force field launches with:
  *   pair_blocks_per_cu  pair-kernel workgroups per CU (capped by the list's
- *                       entries).  The f32 per-wave force sums follow the
- *                       work split, so each value gives reproducible results
- *                       that differ from another value's in the last bits;
+ *                       entries; forces unchanged: each entry's sums go to
+ *                       fixed point on their own);
  *   fft_blocks_per_cu   FFT-pass workgroups per CU (forces unchanged) of the
  *                       axes whose length is a power of two; others, and the
  *                       slab path, ignore it;

@@ -1,9 +1,8 @@
 """Launch-shape autotuner (hmd_forcefield_autotune / set_tuning / get_tuning)
 on a 3,888-atom SPC water box with a 32^3 mesh.  Bars: SPME brick and FFT
 grid changes leave the forces byte-identical (exact integer mesh sums; the
-same per-line transforms); a pair grid change regroups the f32 per-wave sums
-and moves the forces by at most 1e-6 relative RMS; the tuned shapes applied
-to a fresh force field (its list built from the same positions) give
+same per-line transforms), and so does a pair grid change (fixed-point sums
+entry by entry); the tuned shapes applied to a fresh force field (its list built from the same positions) give
 byte-identical forces; 5 graph-replayed steps
 after a brick / FFT change give byte-identical positions and velocities; an
 invalid brick is refused and the previous shapes kept."""

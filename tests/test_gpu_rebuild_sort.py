@@ -1,5 +1,5 @@
 """The list rebuild's cell sort at the sizes where its paths change: one
-workgroup up to 16,320 atoms (2^3 .. 32^3 cells, several atoms a thread, a
+workgroup up to 12,288 atoms (9^3 .. 32^3 cells, several atoms a thread, a
 partial last round), four launches beyond; and clustered atoms, whose cells
 hold many.  The pair set is exact; the cells fill in arbitrary order, and the
 rank that puts the atoms of each into the order of their ids shows in the bits
@@ -16,8 +16,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("n, clustered", [
     (1, False), (2, False), (64, False), (65, True), (520, False), (1025, True), (4097, False),
-    (5120, False), (5121, True), (6553, False), (6554, False), (12288, True), (12289, False),
-    (16320, False), (16321, True), (20001, True)])
+    (5120, False), (5121, True), (6553, False), (6554, False), (12288, True), (12289, False), (20001, True)])
 def test_pair_set_and_order(gpu_ctx, n, clustered):
     rng = np.random.default_rng(n)
     side = int(np.ceil(n ** (1 / 3) - 1e-9))

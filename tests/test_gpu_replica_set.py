@@ -104,8 +104,8 @@ def test_per_replica_logs_byte_reproducible(tmp_path):
 
 
 # A box of 216 molecules beside one across a bound at which the box alone takes
-# other kernels: 5,120 atoms (SPME binning), 16,320 atoms (cell sort).
-@pytest.mark.parametrize("n_mol, mesh", [(4006, 48), (5500, 60)])
+# other kernels: 5,120 atoms (SPME binning), 12,288 atoms (cell sort).
+@pytest.mark.parametrize("n_mol, mesh", [(4006, 48), (4200, 50)])
 def test_batch_of_unlike_boxes_takes_one_variant(n_mol, mesh):
     """Every stage is one launch over both boxes (the launches of the larger
     box alone), and both end as they do alone, byte by byte."""

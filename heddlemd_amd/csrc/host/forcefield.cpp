@@ -720,9 +720,8 @@ void ForceField::rebuild_sort() {
   NblKeyParams kp{p.posq.ptr, n, p.lattice, g[0], g[1], g[2], grid_bits, atom_key.ptr,
                   cell_count.ptr, cell_start.ptr, n_keys, 0u, cell_scan.tile_sums.ptr,
                   cell_list.ptr, sorted_id.ptr, slot_of.ptr, gate};
-  // One workgroup sorts a system whose cells and ids fit its LDS and whose
-  // atoms are few per thread (kNblSortSmall); beyond that the four launches
-  // win on the steps that do rebuild.
+  // one workgroup sorts a small system (kNblSortSmall) whose cells and ids fit
+  // its LDS, else four launches
   const uint32_t n_rule = std::max(n, c.batch.atoms);
   const size_t small_lds = 4 * (size_t)((n_keys + 255u) & ~255u) + 2 * (size_t)((n + 3u) & ~3u);
   if (n_rule <= kNblSortSmall && small_lds + 64 <= c.max_lds) {

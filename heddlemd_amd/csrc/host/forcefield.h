@@ -30,12 +30,15 @@ constexpr size_t kNblBuildStaticLds = 24576;
 // 415-445): grow by 1.5x, and grow ahead of any dropped entry once a build
 // fills more than 0.8 of the capacity.
 constexpr double kNblGrowth = 1.5;
-// Atoms up to which one workgroup does the cell sort of a rebuild, and up to
-// which it also computes the keys.  On a step without a rebuild a launch less
-// saves about 2 us (argon 10,000 with the other merged launches: 57 -> 46 us a
-// step); on one with a rebuild the one workgroup takes as long as the launches
-// it replaces, but for the keys of many atoms (8,997: 27 us with them, half of
-// it theirs).  Beyond, 16-bit ids and counts no longer fit the LDS.
+// Atoms up to which one workgroup does the cell sort of a rebuild.  Against the
+// four launches it wins wherever steps without a rebuild are many (us a step:
+// water 648 77.9 and 82.7, 6,144 118.7 and 121.5, 12,288 127.2 and 128.3; argon
+// 10,000 34.3 and 37.2, 16,000, the last that fits the LDS, 41.7 and 44.5) and
+// loses on the rebuild itself above 9,000 atoms (constant pressure, a rebuild
+// every step: 6,144 268 and 276, 8,997 279.8 and 279.7, 12,288 294.7 and 291.2,
+// 15,000 310 and 304): the line lies between.  And atoms up to which it also
+// computes the keys, else hmd_nbl_keys does: water 648 76.3 and 78.0, 5,118
+// 107.4 and 107.7, 9,000 116.6 and 115.4, 12,288 128.7 and 126.7.
 constexpr uint32_t kNblSortSmall = 12288;
 constexpr uint32_t kNblKeysInline = 5120;
 // List entries below which a pair-kernel workgroup shares an entry, and the

@@ -1,5 +1,5 @@
 """The list rebuild's cell sort at the sizes where its paths change: one
-workgroup up to 12,288 atoms (9^3 .. 32^3 cells, several atoms a thread, a
+workgroup up to 12,288 atoms (2^3 .. 32^3 cells, several atoms a thread, a
 partial last round), four launches beyond; and clustered atoms, whose cells
 hold many.  The pair set is exact; the cells fill in arbitrary order, and the
 rank that puts the atoms of each into the order of their ids shows in the bits

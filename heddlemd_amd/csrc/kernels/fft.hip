@@ -938,9 +938,8 @@ HMD_FFT_SLAB(64, 8, 8, 8, 8, 8, 4)
 // (f32 in LDS and memory): relative error of the potential against FP64, 24
 // boxes a mesh, 3.4e-7 on 24^3, 4.1e-7 on 48^3, 5.2e-7 on 80^3 and 5.9e-7 on
 // 120^3; all f32 4.8e-7, 8.0e-7, 6.6e-7 and 7.4e-7; the Stockham pass 4.1e-7,
-// 6.0e-7, 6.7e-7 and 9.2e-7.  It costs 648 atoms on 24^3 1 us of a step's 88
-// and 39,993 atoms on 80^3 3.4 us of 207 (FP64 in the c axis too another 1 us,
-// for 4% of the error).
+// 6.0e-7, 6.7e-7 and 9.2e-7.  39,993 atoms on 80^3 take 180.7 us a step with it
+// and 180.2 all f32 (FP64 in the c axis too another 1 us, for 4% of the error).
 template <int R, class V>
 __device__ inline void hmd_dft_fwd(V* v);
 
@@ -1085,6 +1084,7 @@ __device__ inline void hmd_mix_stage2(const HmdMixTile& L, const float2* B, floa
   }
 }
 
+// Factors up to MAXR (12 or 16).
 #define HMD_MIX_SWITCH(R, CALL)     \
   switch (R) {                      \
     case 2: CALL(2); break;         \
@@ -1096,13 +1096,16 @@ __device__ inline void hmd_mix_stage2(const HmdMixTile& L, const float2* B, floa
     case 9: CALL(9); break;         \
     case 10: CALL(10); break;       \
     case 12: CALL(12); break;       \
-    case 15: CALL(15); break;       \
-    default: CALL(16); break;       \
+    default:                        \
+      if constexpr (MAXR > 12) {    \
+        if (R == 15) CALL(15);      \
+        else CALL(16);              \
+      }                             \
   }
 
 // The W lines of A transformed in place through B, the butterflies in V;
 // starts after a barrier and ends with one.
-template <class V, int SG>
+template <class V, int SG, int MAXR>
 __device__ inline void hmd_mix_lines(const HmdMixTile& L, float2* A, float2* B,
                                      const float2* tw) {
 #define HMD_MIX_CALL(R) hmd_mix_stage1<R, V, SG>(L, A, B, tw)
@@ -1120,8 +1123,8 @@ __device__ inline void hmd_mix_lines(const HmdMixTile& L, float2* A, float2* B,
 // pass before) is fetched ahead of the forward transform, HMD_MIX_GV points a
 // thread, the rest at their use.
 #define HMD_MIX_GV 4
-__device__ __forceinline__ void hmd_fft_axis_mix_body(const FftParams& p, const uint32_t hmd_bx,
-    const uint32_t hmd_gx) {
+template <int MAXR>
+__device__ inline void hmd_mix_axis(const FftParams& p, const uint32_t hmd_bx) {
   extern __shared__ float2 s_buf[];
   __shared__ double s_w[2][HMD_FFT_THREADS / HMD_WAVE];
   const uint32_t n = p.n, W = p.lines_per_block, sh = (uint32_t)__builtin_ctz(W);
@@ -1155,8 +1158,8 @@ __device__ __forceinline__ void hmd_fft_axis_mix_body(const FftParams& p, const 
     }
   }
   __syncthreads();
-  if (p.sign < 0) hmd_mix_lines<double2, -1>(L, A, B, tw);
-  else hmd_mix_lines<float2, +1>(L, A, B, tw);
+  if (p.sign < 0) hmd_mix_lines<double2, -1, MAXR>(L, A, B, tw);
+  else hmd_mix_lines<float2, +1, MAXR>(L, A, B, tw);
   if (p.apply_influence) {
     double vir = 0.0, ene = 0.0;
     const auto solve = [&](uint32_t t, double2 G) {
@@ -1182,12 +1185,25 @@ __device__ __forceinline__ void hmd_fft_axis_mix_body(const FftParams& p, const 
       p.partials[2 * hmd_bx] = vs;
       p.partials[2 * hmd_bx + 1] = es;
     }
-    hmd_mix_lines<float2, +1>(L, A, B, tw);
+    hmd_mix_lines<float2, +1, MAXR>(L, A, B, tw);
   }
   for (uint32_t t = threadIdx.x; t < total; t += blockDim.x)
     if ((t & (W - 1u)) < Wc) data[at(t)] = A[t];
 }
+// Factors 15 and 16 take 120 registers (in FP64), the others 82, which fit
+// beside the waves of the pair kernel: 39,993 atoms on 80^3 with energies 186.1
+// us a step with one kernel for all, 180.7 with two.
+__device__ __forceinline__ void hmd_fft_axis_mix_body(const FftParams& p, const uint32_t hmd_bx,
+                                                      const uint32_t hmd_gx) {
+  hmd_mix_axis<12>(p, hmd_bx);
+}
 HMD_KERNEL(hmd_fft_axis_mix, FftParams, 256)
+__device__ __forceinline__ void hmd_fft_axis_mix16_body(const FftParams& p,
+                                                        const uint32_t hmd_bx,
+                                                        const uint32_t hmd_gx) {
+  hmd_mix_axis<16>(p, hmd_bx);
+}
+HMD_KERNEL(hmd_fft_axis_mix16, FftParams, 256)
 
 // Pass 1: W real lines of n2 = 2n points as n complex points each.
 __device__ __forceinline__ void hmd_fft_r2c_mix_body(const FftParams& p, const uint32_t hmd_bx,
@@ -1212,7 +1228,7 @@ __device__ __forceinline__ void hmd_fft_r2c_mix_body(const FftParams& p, const u
   for (uint32_t k = threadIdx.x; k < nch; k += blockDim.x)
     wr[k] = reinterpret_cast<const float2*>(p.twiddle_r2c)[k];
   __syncthreads();
-  hmd_mix_lines<float2, -1>(L, A, B, tw);
+  hmd_mix_lines<float2, -1, 16>(L, A, B, tw);
   float2* out = reinterpret_cast<float2*>(p.out) + (size_t)l0 * nch;
   HmdSplit s(threadIdx.x, blockDim.x, nch);
   for (uint32_t t = threadIdx.x; t < Wc * nch; t += blockDim.x, s.next()) {
@@ -1256,7 +1272,7 @@ __device__ __forceinline__ void hmd_fft_c2r_mix_body(const FftParams& p, const u
     }
   }
   __syncthreads();
-  hmd_mix_lines<float2, +1>(L, A, B, tw);
+  hmd_mix_lines<float2, +1, 16>(L, A, B, tw);
   float2* out = reinterpret_cast<float2*>(p.out) + (size_t)l0 * n;
   HmdSplit s(threadIdx.x, blockDim.x, n);
   for (uint32_t t = threadIdx.x; t < Wc * n; t += blockDim.x, s.next())

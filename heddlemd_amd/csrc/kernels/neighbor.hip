@@ -135,7 +135,7 @@ HMD_KERNEL(hmd_nbl_keys, NblKeyParams, 256)
 // Exclusive prefix of up to 256 scan-tile totals into s_off, by the 256
 // threads of the workgroup: the second level of the cell scan, taken by every
 // workgroup of the kernels that read the scan instead of by two launches of
-// their own (a gated launch costs a step without a rebuild about 2 us).
+// their own (a gated launch costs a step without a rebuild about 1.5 us).
 __device__ inline void hmd_nbl_tile_offsets(const NblKeyParams& p, uint32_t* s_off,
                                             uint32_t* s_wave) {
   const uint32_t t = threadIdx.x, lane = hmd_lane();
@@ -191,7 +191,7 @@ HMD_KERNEL(hmd_nbl_rank, NblKeyParams, 256)
 // and ranks through LDS (cell counts, then starts, then cursors; the
 // unordered cell lists as 16-bit ids).  The order is that of
 // the four kernels above.  What it saves is launches: on a step without a
-// rebuild each of the four (six with a two-level scan) costs about 2 us.
+// rebuild each of the four (six with a two-level scan) costs about 1.5 us.
 __device__ __forceinline__ void hmd_nbl_sort_small_body(const NblKeyParams& p,
                                                         const uint32_t hmd_bx,
                                                         const uint32_t hmd_gx) {

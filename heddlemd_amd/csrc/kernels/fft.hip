@@ -1084,36 +1084,48 @@ __device__ inline void hmd_mix_stage2(const HmdMixTile& L, const float2* B, floa
   }
 }
 
-// Factors up to MAXR (12 or 16).
-#define HMD_MIX_SWITCH(R, CALL)     \
-  switch (R) {                      \
-    case 2: CALL(2); break;         \
-    case 3: CALL(3); break;         \
-    case 4: CALL(4); break;         \
-    case 5: CALL(5); break;         \
-    case 6: CALL(6); break;         \
-    case 8: CALL(8); break;         \
-    case 9: CALL(9); break;         \
-    case 10: CALL(10); break;       \
-    case 12: CALL(12); break;       \
-    default:                        \
-      if constexpr (MAXR > 12) {    \
-        if (R == 15) CALL(15);      \
-        else CALL(16);              \
-      }                             \
+// The factors that a kernel holds code for in each stage (the host splits n
+// into n1 <= n2 as near its square root as there is): all in the row passes,
+// up to 12 in the column kernel, and in the one for n2 = 15 and 16 the n1 that
+// come with them (75, 135, 150, 160, 180, 192, 225, 240).  A code object a tenth
+// larger makes a context 0.4 ms dearer (6 ms).
+enum HmdMixSet { HMD_MIX_ROWS, HMD_MIX_COLS12, HMD_MIX_COLS16 };
+__device__ constexpr bool hmd_mix_has(HmdMixSet set, int stage, int R) {
+  if (set == HMD_MIX_COLS12) return R <= 12;
+  if (set == HMD_MIX_COLS16)
+    return stage == 2 ? R >= 15 : (R == 5 || R == 9 || R == 10 || R == 12 || R == 15);
+  return true;
+}
+#define HMD_MIX_CASE(R, STAGE, CALL)                  \
+  case R:                                             \
+    if constexpr (hmd_mix_has(SET, STAGE, R)) CALL(R);\
+    break;
+#define HMD_MIX_SWITCH(N, STAGE, CALL)                \
+  switch (N) {                                        \
+    HMD_MIX_CASE(2, STAGE, CALL)                      \
+    HMD_MIX_CASE(3, STAGE, CALL)                      \
+    HMD_MIX_CASE(4, STAGE, CALL)                      \
+    HMD_MIX_CASE(5, STAGE, CALL)                      \
+    HMD_MIX_CASE(6, STAGE, CALL)                      \
+    HMD_MIX_CASE(8, STAGE, CALL)                      \
+    HMD_MIX_CASE(9, STAGE, CALL)                      \
+    HMD_MIX_CASE(10, STAGE, CALL)                     \
+    HMD_MIX_CASE(12, STAGE, CALL)                     \
+    HMD_MIX_CASE(15, STAGE, CALL)                     \
+    HMD_MIX_CASE(16, STAGE, CALL)                     \
   }
 
 // The W lines of A transformed in place through B, the butterflies in V;
 // starts after a barrier and ends with one.
-template <class V, int SG, int MAXR>
+template <class V, int SG, HmdMixSet SET>
 __device__ inline void hmd_mix_lines(const HmdMixTile& L, float2* A, float2* B,
                                      const float2* tw) {
 #define HMD_MIX_CALL(R) hmd_mix_stage1<R, V, SG>(L, A, B, tw)
-  HMD_MIX_SWITCH(L.n1, HMD_MIX_CALL)
+  HMD_MIX_SWITCH(L.n1, 1, HMD_MIX_CALL)
 #undef HMD_MIX_CALL
   __syncthreads();
 #define HMD_MIX_CALL(R) hmd_mix_stage2<R, V, SG>(L, B, A)
-  HMD_MIX_SWITCH(L.n2, HMD_MIX_CALL)
+  HMD_MIX_SWITCH(L.n2, 2, HMD_MIX_CALL)
 #undef HMD_MIX_CALL
   __syncthreads();
 }
@@ -1123,7 +1135,7 @@ __device__ inline void hmd_mix_lines(const HmdMixTile& L, float2* A, float2* B,
 // pass before) is fetched ahead of the forward transform, HMD_MIX_GV points a
 // thread, the rest at their use.
 #define HMD_MIX_GV 4
-template <int MAXR>
+template <HmdMixSet SET>
 __device__ inline void hmd_mix_axis(const FftParams& p, const uint32_t hmd_bx) {
   extern __shared__ float2 s_buf[];
   __shared__ double s_w[2][HMD_FFT_THREADS / HMD_WAVE];
@@ -1158,8 +1170,8 @@ __device__ inline void hmd_mix_axis(const FftParams& p, const uint32_t hmd_bx) {
     }
   }
   __syncthreads();
-  if (p.sign < 0) hmd_mix_lines<double2, -1, MAXR>(L, A, B, tw);
-  else hmd_mix_lines<float2, +1, MAXR>(L, A, B, tw);
+  if (p.sign < 0) hmd_mix_lines<double2, -1, SET>(L, A, B, tw);
+  else hmd_mix_lines<float2, +1, SET>(L, A, B, tw);
   if (p.apply_influence) {
     double vir = 0.0, ene = 0.0;
     const auto solve = [&](uint32_t t, double2 G) {
@@ -1185,23 +1197,23 @@ __device__ inline void hmd_mix_axis(const FftParams& p, const uint32_t hmd_bx) {
       p.partials[2 * hmd_bx] = vs;
       p.partials[2 * hmd_bx + 1] = es;
     }
-    hmd_mix_lines<float2, +1, MAXR>(L, A, B, tw);
+    hmd_mix_lines<float2, +1, SET>(L, A, B, tw);
   }
   for (uint32_t t = threadIdx.x; t < total; t += blockDim.x)
     if ((t & (W - 1u)) < Wc) data[at(t)] = A[t];
 }
-// Factors 15 and 16 take 120 registers (in FP64), the others 82, which fit
+// Factors 15 and 16 take 123 registers (in FP64), the others 82, which fit
 // beside the waves of the pair kernel: 39,993 atoms on 80^3 with energies 186.1
 // us a step with one kernel for all, 180.7 with two.
 __device__ __forceinline__ void hmd_fft_axis_mix_body(const FftParams& p, const uint32_t hmd_bx,
                                                       const uint32_t hmd_gx) {
-  hmd_mix_axis<12>(p, hmd_bx);
+  hmd_mix_axis<HMD_MIX_COLS12>(p, hmd_bx);
 }
 HMD_KERNEL(hmd_fft_axis_mix, FftParams, 256)
 __device__ __forceinline__ void hmd_fft_axis_mix16_body(const FftParams& p,
                                                         const uint32_t hmd_bx,
                                                         const uint32_t hmd_gx) {
-  hmd_mix_axis<16>(p, hmd_bx);
+  hmd_mix_axis<HMD_MIX_COLS16>(p, hmd_bx);
 }
 HMD_KERNEL(hmd_fft_axis_mix16, FftParams, 256)
 
@@ -1228,7 +1240,7 @@ __device__ __forceinline__ void hmd_fft_r2c_mix_body(const FftParams& p, const u
   for (uint32_t k = threadIdx.x; k < nch; k += blockDim.x)
     wr[k] = reinterpret_cast<const float2*>(p.twiddle_r2c)[k];
   __syncthreads();
-  hmd_mix_lines<float2, -1, 16>(L, A, B, tw);
+  hmd_mix_lines<float2, -1, HMD_MIX_ROWS>(L, A, B, tw);
   float2* out = reinterpret_cast<float2*>(p.out) + (size_t)l0 * nch;
   HmdSplit s(threadIdx.x, blockDim.x, nch);
   for (uint32_t t = threadIdx.x; t < Wc * nch; t += blockDim.x, s.next()) {
@@ -1272,7 +1284,7 @@ __device__ __forceinline__ void hmd_fft_c2r_mix_body(const FftParams& p, const u
     }
   }
   __syncthreads();
-  hmd_mix_lines<float2, +1, 16>(L, A, B, tw);
+  hmd_mix_lines<float2, +1, HMD_MIX_ROWS>(L, A, B, tw);
   float2* out = reinterpret_cast<float2*>(p.out) + (size_t)l0 * n;
   HmdSplit s(threadIdx.x, blockDim.x, n);
   for (uint32_t t = threadIdx.x; t < Wc * n; t += blockDim.x, s.next())

@@ -27,6 +27,7 @@ FORCE_TOL, ENERGY_TOL = 1e-5, 1e-6
     (144, 150, 48),    # 12 x 12, 10 x 15; c: 4 x 6
     (160, 180, 16),    # 10 x 16, 12 x 15; c: 2 x 4
     (225, 240, 18),    # 15 x 15, 15 x 16; c: 3 x 3
+    (135, 192, 16),    # 9 x 15, 12 x 16; c: 2 x 4
     (162, 25, 20),     # Stockham, 5 x 5; c: 2 x 5
     (64, 48, 250),     # power of two, 6 x 8; c: Stockham (125)
     (24, 32, 8),       # mixed a, power-of-two b; c: 2 x 2

@@ -158,7 +158,7 @@ static ForceField::FftPass plan_mix_axis(uint32_t n, uint32_t n_outer, uint32_t 
   ForceField::FftPass ps;
   if (!mix_factors(n, ps.f)) return ps;
   ps.mix = true;
-  ps.k = ps.f[1] > 12 ? K_hmd_fft_axis_mix16 : K_hmd_fft_axis_mix;   // f[0] <= f[1]
+  ps.k = K_hmd_fft_axis_mix;
   for (ps.W = boxes > 1 ? 16u : 8u;; ps.W /= 2) {
     ps.grid = n_outer * ceil_div(cols, ps.W);
     ps.shmem =

@@ -29,8 +29,7 @@
   X(hmd_spme_spread_p6) X(hmd_spme_gather_p6)                                \
   X(hmd_spme_spread_p8) X(hmd_spme_gather_p8)                                \
   X(hmd_fft_r2c_c) X(hmd_fft_c2r_c) X(hmd_fft_axis) X(hmd_spme_reduce)       \
-  X(hmd_fft_axis_mix) X(hmd_fft_axis_mix16)                                  \
-  X(hmd_fft_r2c_mix) X(hmd_fft_c2r_mix)                                      \
+  X(hmd_fft_axis_mix) X(hmd_fft_r2c_mix) X(hmd_fft_c2r_mix)                  \
   X(hmd_fft_axis_16) X(hmd_fft_r2c_16) X(hmd_fft_c2r_16)                     \
   X(hmd_fft_axis_32) X(hmd_fft_r2c_32) X(hmd_fft_c2r_32)                     \
   X(hmd_fft_axis_64) X(hmd_fft_r2c_64) X(hmd_fft_c2r_64)                     \

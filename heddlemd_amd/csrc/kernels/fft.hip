@@ -19,66 +19,48 @@
 
 #define HMD_FFT_THREADS 256u
 
-// Complex arithmetic in float2 and, where a transform's butterflies run in
-// FP64, in double2.
-template <class V> struct HmdReal;
-template <> struct HmdReal<float2> { typedef float T; };
-template <> struct HmdReal<double2> { typedef double T; };
-template <class V>
-__device__ inline V cnum(typename HmdReal<V>::T x, typename HmdReal<V>::T y) {
-  V r;
-  r.x = x;
-  r.y = y;
-  return r;
+__device__ inline float2 cmul(float2 a, float2 b) {
+  return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
-template <class V>
-__device__ inline V cmul(V a, V b) {
-  return cnum<V>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-template <class V>
-__device__ inline V cadd(V a, V b) { return cnum<V>(a.x + b.x, a.y + b.y); }
-template <class V>
-__device__ inline V csub(V a, V b) { return cnum<V>(a.x - b.x, a.y - b.y); }
+__device__ inline float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
+__device__ inline float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
 __device__ inline float2 cconj(float2 a) { return make_float2(a.x, -a.y); }
 // multiply by sign * i
-template <class V>
-__device__ inline V cmul_si(V a, int sign) {
-  return sign < 0 ? cnum<V>(a.y, -a.x) : cnum<V>(-a.y, a.x);
+__device__ inline float2 cmul_si(float2 a, int sign) {
+  return sign < 0 ? make_float2(a.y, -a.x) : make_float2(-a.y, a.x);
 }
 
 // One radix-R butterfly: y_k = sum_r x_r e^{sign 2 pi i r k / R}.
-template <class V>
-__device__ inline void hmd_dft(V* v, uint32_t R, int sign) {
-  typedef typename HmdReal<V>::T T;
+__device__ inline void hmd_dft(float2* v, uint32_t R, int sign) {
   if (R == 2) {
-    V a = v[0], b = v[1];
+    float2 a = v[0], b = v[1];
     v[0] = cadd(a, b);
     v[1] = csub(a, b);
   } else if (R == 4) {
-    V t0 = cadd(v[0], v[2]), t1 = csub(v[0], v[2]);
-    V t2 = cadd(v[1], v[3]), t3 = cmul_si(csub(v[1], v[3]), sign);
+    float2 t0 = cadd(v[0], v[2]), t1 = csub(v[0], v[2]);
+    float2 t2 = cadd(v[1], v[3]), t3 = cmul_si(csub(v[1], v[3]), sign);
     v[0] = cadd(t0, t2);
     v[2] = csub(t0, t2);
     v[1] = cadd(t1, t3);
     v[3] = csub(t1, t3);
   } else if (R == 3) {
-    const T s3 = (T)0.86602540378443865, h = (T)0.5;
-    V t = cadd(v[1], v[2]);
-    V u = cmul_si(csub(v[1], v[2]), sign);
-    V m = cnum<V>(v[0].x - h * t.x, v[0].y - h * t.y);
+    const float s3 = 0.86602540378443865f;
+    float2 t = cadd(v[1], v[2]);
+    float2 u = cmul_si(csub(v[1], v[2]), sign);
+    float2 m = make_float2(v[0].x - 0.5f * t.x, v[0].y - 0.5f * t.y);
     v[0] = cadd(v[0], t);
-    v[1] = cnum<V>(m.x + s3 * u.x, m.y + s3 * u.y);
-    v[2] = cnum<V>(m.x - s3 * u.x, m.y - s3 * u.y);
+    v[1] = make_float2(m.x + s3 * u.x, m.y + s3 * u.y);
+    v[2] = make_float2(m.x - s3 * u.x, m.y - s3 * u.y);
   } else {  // R == 5
-    const T c1 = (T)0.30901699437494742, c2 = (T)-0.80901699437494742;
-    const T s1 = (T)0.95105651629515357, s2 = (T)0.58778525229247313;
-    V a1 = cadd(v[1], v[4]), b1 = csub(v[1], v[4]);
-    V a2 = cadd(v[2], v[3]), b2 = csub(v[2], v[3]);
-    V x0 = v[0];
-    V m1 = cnum<V>(x0.x + c1 * a1.x + c2 * a2.x, x0.y + c1 * a1.y + c2 * a2.y);
-    V m2 = cnum<V>(x0.x + c2 * a1.x + c1 * a2.x, x0.y + c2 * a1.y + c1 * a2.y);
-    V n1 = cmul_si(cnum<V>(s1 * b1.x + s2 * b2.x, s1 * b1.y + s2 * b2.y), sign);
-    V n2 = cmul_si(cnum<V>(s2 * b1.x - s1 * b2.x, s2 * b1.y - s1 * b2.y), sign);
+    const float c1 = 0.30901699437494742f, c2 = -0.80901699437494742f;
+    const float s1 = 0.95105651629515357f, s2 = 0.58778525229247313f;
+    float2 a1 = cadd(v[1], v[4]), b1 = csub(v[1], v[4]);
+    float2 a2 = cadd(v[2], v[3]), b2 = csub(v[2], v[3]);
+    float2 x0 = v[0];
+    float2 m1 = make_float2(x0.x + c1 * a1.x + c2 * a2.x, x0.y + c1 * a1.y + c2 * a2.y);
+    float2 m2 = make_float2(x0.x + c2 * a1.x + c1 * a2.x, x0.y + c2 * a1.y + c1 * a2.y);
+    float2 n1 = cmul_si(make_float2(s1 * b1.x + s2 * b2.x, s1 * b1.y + s2 * b2.y), sign);
+    float2 n2 = cmul_si(make_float2(s2 * b1.x - s1 * b2.x, s2 * b1.y - s1 * b2.y), sign);
     v[0] = cadd(x0, cadd(a1, a2));
     v[1] = cadd(m1, n1);
     v[4] = csub(m1, n1);
@@ -327,32 +309,31 @@ HMD_KERNEL(hmd_fft_axis, FftParams, 256)
 // tile[k * W + w], loaded and stored with coalesced accesses; no runtime
 // radix, no integer division in the butterflies, no scratch arrays.
 
-template <int SG, class V>
-__device__ inline V hmd_mul_si(V a) {   // a * (SG i)
-  return SG < 0 ? cnum<V>(a.y, -a.x) : cnum<V>(-a.y, a.x);
+template <int SG>
+__device__ inline float2 hmd_mul_si(float2 a) {   // a * (SG i)
+  return SG < 0 ? make_float2(a.y, -a.x) : make_float2(-a.y, a.x);
 }
 
-template <int SG, class V>
-__device__ inline void hmd_dft4(V* v) {
-  const V t0 = cadd(v[0], v[2]), t1 = csub(v[0], v[2]);
-  const V t2 = cadd(v[1], v[3]), t3 = hmd_mul_si<SG>(csub(v[1], v[3]));
+template <int SG>
+__device__ inline void hmd_dft4(float2* v) {
+  const float2 t0 = cadd(v[0], v[2]), t1 = csub(v[0], v[2]);
+  const float2 t2 = cadd(v[1], v[3]), t3 = hmd_mul_si<SG>(csub(v[1], v[3]));
   v[0] = cadd(t0, t2);
   v[2] = csub(t0, t2);
   v[1] = cadd(t1, t3);
   v[3] = csub(t1, t3);
 }
 
-template <int SG, class V>
-__device__ inline void hmd_dft8(V* v) {
-  V e[4] = {v[0], v[2], v[4], v[6]};
-  V o[4] = {v[1], v[3], v[5], v[7]};
+template <int SG>
+__device__ inline void hmd_dft8(float2* v) {
+  float2 e[4] = {v[0], v[2], v[4], v[6]};
+  float2 o[4] = {v[1], v[3], v[5], v[7]};
   hmd_dft4<SG>(e);
   hmd_dft4<SG>(o);
-  typedef typename HmdReal<V>::T T;
-  const T h = (T)0.70710678118654752;   // cos(pi/4)
-  const V o1 = cmul(o[1], cnum<V>(h, SG * h));
-  const V o2 = hmd_mul_si<SG>(o[2]);
-  const V o3 = cmul(o[3], cnum<V>(-h, SG * h));
+  const float h = 0.70710678118654752f;   // cos(pi/4)
+  const float2 o1 = cmul(o[1], make_float2(h, SG * h));
+  const float2 o2 = hmd_mul_si<SG>(o[2]);
+  const float2 o3 = cmul(o[3], make_float2(-h, SG * h));
   v[0] = cadd(e[0], o[0]);
   v[4] = csub(e[0], o[0]);
   v[1] = cadd(e[1], o1);
@@ -363,9 +344,9 @@ __device__ inline void hmd_dft8(V* v) {
   v[7] = csub(e[3], o3);
 }
 
-template <int SG, class V>
-__device__ inline void hmd_dft16(V* v) {
-  V e[8], o[8];
+template <int SG>
+__device__ inline void hmd_dft16(float2* v) {
+  float2 e[8], o[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     e[k] = v[2 * k];
@@ -374,13 +355,13 @@ __device__ inline void hmd_dft16(V* v) {
   hmd_dft8<SG>(e);
   hmd_dft8<SG>(o);
   // cos and sin of 2 pi k / 16
-  typedef typename HmdReal<V>::T T;
-  const T c1 = (T)0.92387953251128674, c2 = (T)0.70710678118654752, c3 = (T)0.38268343236508977;
-  const T C[8] = {(T)1, c1, c2, c3, (T)0, -c3, -c2, -c1};
-  const T S[8] = {(T)0, c3, c2, c1, (T)1, c1, c2, c3};
+  const float C[8] = {1.0f, 0.92387953251128674f, 0.70710678118654752f, 0.38268343236508977f,
+                      0.0f, -0.38268343236508977f, -0.70710678118654752f, -0.92387953251128674f};
+  const float S[8] = {0.0f, 0.38268343236508977f, 0.70710678118654752f, 0.92387953251128674f,
+                      1.0f, 0.92387953251128674f, 0.70710678118654752f, 0.38268343236508977f};
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    const V t = cmul(o[k], cnum<V>(C[k], SG * S[k]));
+    const float2 t = cmul(o[k], make_float2(C[k], SG * S[k]));
     v[k] = cadd(e[k], t);
     v[k + 8] = csub(e[k], t);
   }
@@ -923,7 +904,7 @@ HMD_FFT_SLAB(64, 8, 8, 8, 8, 8, 4)
 // 18 ... 150 and their halves): the two-stage transform above with the factors
 // chosen at run time.  Each stage is a switch over register DFTs of fixed
 // length, so a line is two LDS round trips and one twiddle per point, where
-// the Stockham pass above takes one round trip, a twiddle from memory and two
+// the Stockham pass below takes one round trip, a twiddle from memory and two
 // integer divisions per radix (4, 2, 3, 5) and evaluates the influence
 // function (an FP64 exp) at every point of every step; here it is a table.
 // Bound by latency: a workgroup of a small mesh runs a handful of butterflies
@@ -931,79 +912,131 @@ HMD_FFT_SLAB(64, 8, 8, 8, 8, 8, 4)
 // A step of the 648-atom box (24^3) went from 200 to 157 us, of 4,503 atoms
 // (40^3) from 315 to 242 us, of 39,993 atoms (80^3) from 314 to 230 us.
 // One direction is compiled: the inverse conjugates on the way in and out.
-//
-// The influence function amplifies the lowest modes, where a liquid has the
-// least amplitude, so the f32 sums of the forward column passes set the
-// potential's error.  Those two passes run their butterflies in FP64 registers
-// (f32 in LDS and memory): relative error of the potential against FP64, 24
-// boxes a mesh, 3.4e-7 on 24^3, 4.1e-7 on 48^3, 5.2e-7 on 80^3 and 5.9e-7 on
-// 120^3; all f32 4.8e-7, 8.0e-7, 6.6e-7 and 7.4e-7; the Stockham pass 4.1e-7,
-// 6.0e-7, 6.7e-7 and 9.2e-7.  39,993 atoms on 80^3 take 180.7 us a step with it
-// and 180.2 all f32 (FP64 in the c axis too another 1 us, for 4% of the error).
-template <int R, class V>
-__device__ inline void hmd_dft_fwd(V* v);
+// cos and sin of 2 pi k / R.
+template <int R> struct HmdRoots;
+template <> struct HmdRoots<6> {
+  static __device__ float C(int k) {
+    const float t[6] = {
+        1.0f, 0.5f, -0.5f, -1.0f, -0.5f, 0.5f};
+    return t[k];
+  }
+  static __device__ float S(int k) {
+    const float t[6] = {
+        0.0f, 0.866025403784439f, 0.866025403784439f, 0.0f, -0.866025403784438f,
+        -0.866025403784439f};
+    return t[k];
+  }
+};
+template <> struct HmdRoots<9> {
+  static __device__ float C(int k) {
+    const float t[9] = {
+        1.0f, 0.766044443118978f, 0.173648177666930f, -0.5f, -0.939692620785908f,
+        -0.939692620785908f, -0.5f, 0.173648177666930f, 0.766044443118978f};
+    return t[k];
+  }
+  static __device__ float S(int k) {
+    const float t[9] = {
+        0.0f, 0.642787609686539f, 0.984807753012208f, 0.866025403784439f, 0.342020143325669f,
+        -0.342020143325669f, -0.866025403784438f, -0.984807753012208f, -0.642787609686540f};
+    return t[k];
+  }
+};
+template <> struct HmdRoots<10> {
+  static __device__ float C(int k) {
+    const float t[10] = {
+        1.0f, 0.809016994374947f, 0.309016994374947f, -0.309016994374947f, -0.809016994374947f,
+        -1.0f, -0.809016994374948f, -0.309016994374948f, 0.309016994374947f, 0.809016994374947f};
+    return t[k];
+  }
+  static __device__ float S(int k) {
+    const float t[10] = {
+        0.0f, 0.587785252292473f, 0.951056516295154f, 0.951056516295154f, 0.587785252292473f,
+        0.0f, -0.587785252292473f, -0.951056516295154f, -0.951056516295154f, -0.587785252292473f};
+    return t[k];
+  }
+};
+template <> struct HmdRoots<12> {
+  static __device__ float C(int k) {
+    const float t[12] = {
+        1.0f, 0.866025403784439f, 0.5f, 0.0f, -0.5f, -0.866025403784439f, -1.0f,
+        -0.866025403784439f, -0.5f, 0.0f, 0.5f, 0.866025403784438f};
+    return t[k];
+  }
+  static __device__ float S(int k) {
+    const float t[12] = {
+        0.0f, 0.5f, 0.866025403784439f, 1.0f, 0.866025403784439f, 0.5f, 0.0f, -0.5f,
+        -0.866025403784438f, -1.0f, -0.866025403784439f, -0.5f};
+    return t[k];
+  }
+};
+template <> struct HmdRoots<15> {
+  static __device__ float C(int k) {
+    const float t[15] = {
+        1.0f, 0.913545457642601f, 0.669130606358858f, 0.309016994374947f, -0.104528463267653f,
+        -0.5f, -0.809016994374947f, -0.978147600733806f, -0.978147600733806f,
+        -0.809016994374948f, -0.5f, -0.104528463267654f, 0.309016994374947f, 0.669130606358858f,
+        0.913545457642601f};
+    return t[k];
+  }
+  static __device__ float S(int k) {
+    const float t[15] = {
+        0.0f, 0.406736643075800f, 0.743144825477394f, 0.951056516295154f, 0.994521895368273f,
+        0.866025403784439f, 0.587785252292473f, 0.207911690817759f, -0.207911690817759f,
+        -0.587785252292473f, -0.866025403784438f, -0.994521895368273f, -0.951056516295154f,
+        -0.743144825477394f, -0.406736643075800f};
+    return t[k];
+  }
+};
 
-// Forward DFT of R = A B points in registers, A and B coprime (Good, J. R.
-// Stat. Soc. B 20, 361, 1958): point (B a + A b) mod R, output k from outputs
-// k mod A and k mod B of the two transforms, and no twiddles between them.
-template <int A, int B, class V>
-__device__ inline void hmd_dft_coprime(V* v) {
+__device__ inline void hmd_dft2(float2* v) {
+  const float2 a = v[0], b = v[1];
+  v[0] = cadd(a, b);
+  v[1] = csub(a, b);
+}
+
+// Forward DFT of A B points in registers: B DFTs of length A, the twiddles,
+// A DFTs of length B.
+template <int R>
+__device__ inline void hmd_dft_fwd(float2* v);
+
+template <int A, int B>
+__device__ inline void hmd_dft_ab(float2* v) {
   constexpr int R = A * B;
-  V t[B][A], y[A][B];
+  float2 t[B][A];
 #pragma unroll
   for (int b = 0; b < B; ++b) {
 #pragma unroll
-    for (int a = 0; a < A; ++a) t[b][a] = v[(B * a + A * b) % R];
-    hmd_dft_fwd<A, V>(t[b]);
+    for (int a = 0; a < A; ++a) t[b][a] = v[B * a + b];
+    hmd_dft_fwd<A>(t[b]);
+#pragma unroll
+    for (int k = 1; k < A; ++k)
+      if (b > 0)
+        t[b][k] = cmul(t[b][k], make_float2(HmdRoots<R>::C((b * k) % R),
+                                            -HmdRoots<R>::S((b * k) % R)));
   }
 #pragma unroll
   for (int k = 0; k < A; ++k) {
+    float2 u[B];
 #pragma unroll
-    for (int b = 0; b < B; ++b) y[k][b] = t[b][k];
-    hmd_dft_fwd<B, V>(y[k]);
-  }
+    for (int b = 0; b < B; ++b) u[b] = t[b][k];
+    hmd_dft_fwd<B>(u);
 #pragma unroll
-  for (int k = 0; k < R; ++k) v[k] = y[k % A][k % B];
-}
-
-// Forward DFT of 9 points: three DFTs of 3, the four twiddles, three of 3.
-template <class V>
-__device__ inline void hmd_dft9(V* v) {
-  typedef typename HmdReal<V>::T T;
-  const V w1 = cnum<V>((T)0.76604444311897804, (T)-0.64278760968653933);
-  const V w2 = cnum<V>((T)0.17364817766693035, (T)-0.98480775301220806);
-  const V w4 = cnum<V>((T)-0.93969262078590838, (T)-0.34202014332566873);
-  V t[3][3];
-#pragma unroll
-  for (int b = 0; b < 3; ++b) {
-#pragma unroll
-    for (int a = 0; a < 3; ++a) t[b][a] = v[3 * a + b];
-    hmd_dft(t[b], 3u, -1);
-  }
-  t[1][1] = cmul(t[1][1], w1);
-  t[1][2] = cmul(t[1][2], w2);
-  t[2][1] = cmul(t[2][1], w2);
-  t[2][2] = cmul(t[2][2], w4);
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    V u[3] = {t[0][k], t[1][k], t[2][k]};
-    hmd_dft(u, 3u, -1);
-#pragma unroll
-    for (int q = 0; q < 3; ++q) v[k + 3 * q] = u[q];
+    for (int q = 0; q < B; ++q) v[k + A * q] = u[q];
   }
 }
 
-template <int R, class V>
-__device__ inline void hmd_dft_fwd(V* v) {
-  if constexpr (R == 2 || R == 3 || R == 5) hmd_dft(v, (uint32_t)R, -1);
+template <int R>
+__device__ inline void hmd_dft_fwd(float2* v) {
+  if constexpr (R == 2) hmd_dft2(v);
+  else if constexpr (R == 3 || R == 5) hmd_dft(v, (uint32_t)R, -1);
   else if constexpr (R == 4) hmd_dft4<-1>(v);
   else if constexpr (R == 8) hmd_dft8<-1>(v);
   else if constexpr (R == 16) hmd_dft16<-1>(v);
-  else if constexpr (R == 9) hmd_dft9(v);
-  else if constexpr (R == 6) hmd_dft_coprime<2, 3, V>(v);
-  else if constexpr (R == 10) hmd_dft_coprime<2, 5, V>(v);
-  else if constexpr (R == 12) hmd_dft_coprime<4, 3, V>(v);
-  else hmd_dft_coprime<3, 5, V>(v);
+  else if constexpr (R == 6) hmd_dft_ab<2, 3>(v);
+  else if constexpr (R == 9) hmd_dft_ab<3, 3>(v);
+  else if constexpr (R == 10) hmd_dft_ab<2, 5>(v);
+  else if constexpr (R == 12) hmd_dft_ab<4, 3>(v);
+  else hmd_dft_ab<3, 5>(v);
 }
 
 // t / d and t % d for t = t0, t0 + step, ...: one division, then carries.
@@ -1036,96 +1069,75 @@ __device__ inline HmdMixTile hmd_mix_cols(uint32_t n1, uint32_t n2, uint32_t W) 
   return HmdMixTile{n1, n2, W, W, 1u, (n1 | 1u) * W, W, 1u, false};
 }
 
-template <class V>
-__device__ inline V hmd_cast(float2 a) { return cnum<V>(a.x, a.y); }
-template <class V>
-__device__ inline float2 hmd_to_f32(V a) { return make_float2((float)a.x, (float)a.y); }
-
 // Stage 1: for every line and m < n2, the n1-point DFT over points
-// n2 j + m, times e^{-2 pi i m k / n} (SG > 0: of the conjugates).
-template <int R, class V, int SG>
+// n2 j + m, times e^{-2 pi i m k / n}.
+template <int R>
 __device__ inline void hmd_mix_stage1(const HmdMixTile& L, const float2* A, float2* B,
-                                      const float2* tw) {
+                                      const float2* tw, float conj) {
   HmdSplit s(threadIdx.x, blockDim.x, L.rows ? L.n2 : L.W);
   for (uint32_t t = threadIdx.x; t < L.W * L.n2; t += blockDim.x, s.next()) {
     const uint32_t w = L.rows ? s.q : s.r, m = L.rows ? s.r : s.q;
-    V v[R];
+    float2 v[R];
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-      const float2 x = A[(L.n2 * (uint32_t)j + m) * L.ea + w * L.la];
-      v[j] = hmd_cast<V>(SG < 0 ? x : cconj(x));
+      v[j] = A[(L.n2 * (uint32_t)j + m) * L.ea + w * L.la];
+      v[j].y *= conj;
     }
-    hmd_dft_fwd<R, V>(v);
+    hmd_dft_fwd<R>(v);
     float2* out = B + m * L.bm + w * L.lb;
-    out[0] = hmd_to_f32(v[0]);
+    out[0] = v[0];
 #pragma unroll
-    for (int k = 1; k < R; ++k)
-      out[(uint32_t)k * L.bk] = hmd_to_f32(cmul(v[k], hmd_cast<V>(tw[m * (uint32_t)k])));
+    for (int k = 1; k < R; ++k) out[(uint32_t)k * L.bk] = cmul(v[k], tw[m * (uint32_t)k]);
   }
 }
 
 // Stage 2: for every line and k1 < n1, the n2-point DFT over m, to points
-// k1 + n1 k2 (SG > 0: conjugated).
-template <int R, class V, int SG>
-__device__ inline void hmd_mix_stage2(const HmdMixTile& L, const float2* B, float2* A) {
+// k1 + n1 k2.
+template <int R>
+__device__ inline void hmd_mix_stage2(const HmdMixTile& L, const float2* B, float2* A,
+                                      float conj) {
   HmdSplit s(threadIdx.x, blockDim.x, L.rows ? L.n1 : L.W);
   for (uint32_t t = threadIdx.x; t < L.W * L.n1; t += blockDim.x, s.next()) {
     const uint32_t w = L.rows ? s.q : s.r, k1 = L.rows ? s.r : s.q;
-    V u[R];
+    float2 u[R];
     const float2* in = B + k1 * L.bk + w * L.lb;
 #pragma unroll
-    for (int m = 0; m < R; ++m) u[m] = hmd_cast<V>(in[(uint32_t)m * L.bm]);
-    hmd_dft_fwd<R, V>(u);
+    for (int m = 0; m < R; ++m) u[m] = in[(uint32_t)m * L.bm];
+    hmd_dft_fwd<R>(u);
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-      const float2 x = hmd_to_f32(u[k]);
-      A[(k1 + L.n1 * (uint32_t)k) * L.ea + w * L.la] = SG < 0 ? x : cconj(x);
+      u[k].y *= conj;
+      A[(k1 + L.n1 * (uint32_t)k) * L.ea + w * L.la] = u[k];
     }
   }
 }
 
-// The factors that a kernel holds code for in each stage (the host splits n
-// into n1 <= n2 as near its square root as there is): all in the row passes,
-// up to 12 in the column kernel, and in the one for n2 = 15 and 16 the n1 that
-// come with them (75, 135, 150, 160, 180, 192, 225, 240).  A code object a tenth
-// larger makes a context 0.4 ms dearer (6 ms).
-enum HmdMixSet { HMD_MIX_ROWS, HMD_MIX_COLS12, HMD_MIX_COLS16 };
-__device__ constexpr bool hmd_mix_has(HmdMixSet set, int stage, int R) {
-  if (set == HMD_MIX_COLS12) return R <= 12;
-  if (set == HMD_MIX_COLS16)
-    return stage == 2 ? R >= 15 : (R == 5 || R == 9 || R == 10 || R == 12 || R == 15);
-  return true;
-}
-#define HMD_MIX_CASE(R, STAGE, CALL)                  \
-  case R:                                             \
-    if constexpr (hmd_mix_has(SET, STAGE, R)) CALL(R);\
-    break;
-#define HMD_MIX_SWITCH(N, STAGE, CALL)                \
-  switch (N) {                                        \
-    HMD_MIX_CASE(2, STAGE, CALL)                      \
-    HMD_MIX_CASE(3, STAGE, CALL)                      \
-    HMD_MIX_CASE(4, STAGE, CALL)                      \
-    HMD_MIX_CASE(5, STAGE, CALL)                      \
-    HMD_MIX_CASE(6, STAGE, CALL)                      \
-    HMD_MIX_CASE(8, STAGE, CALL)                      \
-    HMD_MIX_CASE(9, STAGE, CALL)                      \
-    HMD_MIX_CASE(10, STAGE, CALL)                     \
-    HMD_MIX_CASE(12, STAGE, CALL)                     \
-    HMD_MIX_CASE(15, STAGE, CALL)                     \
-    HMD_MIX_CASE(16, STAGE, CALL)                     \
+#define HMD_MIX_SWITCH(R, CALL)     \
+  switch (R) {                      \
+    case 2: CALL(2); break;         \
+    case 3: CALL(3); break;         \
+    case 4: CALL(4); break;         \
+    case 5: CALL(5); break;         \
+    case 6: CALL(6); break;         \
+    case 8: CALL(8); break;         \
+    case 9: CALL(9); break;         \
+    case 10: CALL(10); break;       \
+    case 12: CALL(12); break;       \
+    case 15: CALL(15); break;       \
+    default: CALL(16); break;       \
   }
 
-// The W lines of A transformed in place through B, the butterflies in V;
-// starts after a barrier and ends with one.
-template <class V, int SG, HmdMixSet SET>
-__device__ inline void hmd_mix_lines(const HmdMixTile& L, float2* A, float2* B,
-                                     const float2* tw) {
-#define HMD_MIX_CALL(R) hmd_mix_stage1<R, V, SG>(L, A, B, tw)
-  HMD_MIX_SWITCH(L.n1, 1, HMD_MIX_CALL)
+// The W lines of A transformed in place through B; starts after a barrier
+// and ends with one.
+__device__ inline void hmd_mix_fft(const HmdMixTile& L, float2* A, float2* B, const float2* tw,
+                                   int sign) {
+  const float conj = sign < 0 ? 1.0f : -1.0f;
+#define HMD_MIX_CALL(R) hmd_mix_stage1<R>(L, A, B, tw, conj)
+  HMD_MIX_SWITCH(L.n1, HMD_MIX_CALL)
 #undef HMD_MIX_CALL
   __syncthreads();
-#define HMD_MIX_CALL(R) hmd_mix_stage2<R, V, SG>(L, B, A)
-  HMD_MIX_SWITCH(L.n2, 2, HMD_MIX_CALL)
+#define HMD_MIX_CALL(R) hmd_mix_stage2<R>(L, B, A, conj)
+  HMD_MIX_SWITCH(L.n2, HMD_MIX_CALL)
 #undef HMD_MIX_CALL
   __syncthreads();
 }
@@ -1135,8 +1147,8 @@ __device__ inline void hmd_mix_lines(const HmdMixTile& L, float2* A, float2* B,
 // pass before) is fetched ahead of the forward transform, HMD_MIX_GV points a
 // thread, the rest at their use.
 #define HMD_MIX_GV 4
-template <HmdMixSet SET>
-__device__ inline void hmd_mix_axis(const FftParams& p, const uint32_t hmd_bx) {
+__device__ __forceinline__ void hmd_fft_axis_mix_body(const FftParams& p, const uint32_t hmd_bx,
+    const uint32_t hmd_gx) {
   extern __shared__ float2 s_buf[];
   __shared__ double s_w[2][HMD_FFT_THREADS / HMD_WAVE];
   const uint32_t n = p.n, W = p.lines_per_block, sh = (uint32_t)__builtin_ctz(W);
@@ -1170,8 +1182,7 @@ __device__ inline void hmd_mix_axis(const FftParams& p, const uint32_t hmd_bx) {
     }
   }
   __syncthreads();
-  if (p.sign < 0) hmd_mix_lines<double2, -1, SET>(L, A, B, tw);
-  else hmd_mix_lines<float2, +1, SET>(L, A, B, tw);
+  hmd_mix_fft(L, A, B, tw, p.sign);
   if (p.apply_influence) {
     double vir = 0.0, ene = 0.0;
     const auto solve = [&](uint32_t t, double2 G) {
@@ -1197,25 +1208,12 @@ __device__ inline void hmd_mix_axis(const FftParams& p, const uint32_t hmd_bx) {
       p.partials[2 * hmd_bx] = vs;
       p.partials[2 * hmd_bx + 1] = es;
     }
-    hmd_mix_lines<float2, +1, SET>(L, A, B, tw);
+    hmd_mix_fft(L, A, B, tw, +1);
   }
   for (uint32_t t = threadIdx.x; t < total; t += blockDim.x)
     if ((t & (W - 1u)) < Wc) data[at(t)] = A[t];
 }
-// Factors 15 and 16 take 123 registers (in FP64), the others 82, which fit
-// beside the waves of the pair kernel: 39,993 atoms on 80^3 with energies 186.1
-// us a step with one kernel for all, 180.7 with two.
-__device__ __forceinline__ void hmd_fft_axis_mix_body(const FftParams& p, const uint32_t hmd_bx,
-                                                      const uint32_t hmd_gx) {
-  hmd_mix_axis<HMD_MIX_COLS12>(p, hmd_bx);
-}
 HMD_KERNEL(hmd_fft_axis_mix, FftParams, 256)
-__device__ __forceinline__ void hmd_fft_axis_mix16_body(const FftParams& p,
-                                                        const uint32_t hmd_bx,
-                                                        const uint32_t hmd_gx) {
-  hmd_mix_axis<HMD_MIX_COLS16>(p, hmd_bx);
-}
-HMD_KERNEL(hmd_fft_axis_mix16, FftParams, 256)
 
 // Pass 1: W real lines of n2 = 2n points as n complex points each.
 __device__ __forceinline__ void hmd_fft_r2c_mix_body(const FftParams& p, const uint32_t hmd_bx,
@@ -1240,7 +1238,7 @@ __device__ __forceinline__ void hmd_fft_r2c_mix_body(const FftParams& p, const u
   for (uint32_t k = threadIdx.x; k < nch; k += blockDim.x)
     wr[k] = reinterpret_cast<const float2*>(p.twiddle_r2c)[k];
   __syncthreads();
-  hmd_mix_lines<float2, -1, HMD_MIX_ROWS>(L, A, B, tw);
+  hmd_mix_fft(L, A, B, tw, -1);
   float2* out = reinterpret_cast<float2*>(p.out) + (size_t)l0 * nch;
   HmdSplit s(threadIdx.x, blockDim.x, nch);
   for (uint32_t t = threadIdx.x; t < Wc * nch; t += blockDim.x, s.next()) {
@@ -1284,7 +1282,7 @@ __device__ __forceinline__ void hmd_fft_c2r_mix_body(const FftParams& p, const u
     }
   }
   __syncthreads();
-  hmd_mix_lines<float2, +1, HMD_MIX_ROWS>(L, A, B, tw);
+  hmd_mix_fft(L, A, B, tw, +1);
   float2* out = reinterpret_cast<float2*>(p.out) + (size_t)l0 * n;
   HmdSplit s(threadIdx.x, blockDim.x, n);
   for (uint32_t t = threadIdx.x; t < Wc * n; t += blockDim.x, s.next())

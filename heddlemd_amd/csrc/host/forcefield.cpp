@@ -148,11 +148,12 @@ static bool mix_factors(uint32_t n, uint32_t f[2]) {
 // Launch shapes of the mixed two-stage passes of a mesh, one of `boxes` that
 // share the launch.  Columns: 8 adjacent lines a workgroup (whole 64-byte
 // segments of the mesh) while that gives every CU a workgroup, else 4; 16 in a
-// batch whose boxes do so together (64 boxes of 24^3 to 48^3: 159 us a step
-// with widths picked for each box alone, 107 with 8, 80 with 16; four boxes
-// 124 us a step with any).  The energy partials follow the grid.  Rows: 8
-// lines or more, up to 32 once every CU has two workgroups (the same 64 boxes:
-// 56 us a step with 8, 36 with 16, 25 with 32).
+// batch whose boxes do so together (64 boxes of 24^3 to 48^3: 170 us a step
+// with widths picked for each box alone, 86 with these; 8 columns take a third
+// longer than 16, 32 as long; four boxes 124 us a step with any).  The energy
+// partials follow the grid.  Rows: 8 lines or more, up to 32 once every CU has
+// two workgroups (the same 64 boxes: 56 us a step with 8, 36 with 16, 25 with
+// 32).
 static ForceField::FftPass plan_mix_axis(uint32_t n, uint32_t n_outer, uint32_t cols,
                                          uint32_t num_cus, uint32_t boxes) {
   ForceField::FftPass ps;

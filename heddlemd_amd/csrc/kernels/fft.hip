@@ -904,13 +904,16 @@ HMD_FFT_SLAB(64, 8, 8, 8, 8, 8, 4)
 // 18 ... 150 and their halves): the two-stage transform above with the factors
 // chosen at run time.  Each stage is a switch over register DFTs of fixed
 // length, so a line is two LDS round trips and one twiddle per point, where
-// the Stockham pass below takes one round trip, a twiddle from memory and two
+// the Stockham pass above takes one round trip, a twiddle from memory and two
 // integer divisions per radix (4, 2, 3, 5) and evaluates the influence
 // function (an FP64 exp) at every point of every step; here it is a table.
 // Bound by latency: a workgroup of a small mesh runs a handful of butterflies
 // a thread, so what counts is the number of dependent LDS and L2 round trips.
 // A step of the 648-atom box (24^3) went from 200 to 157 us, of 4,503 atoms
 // (40^3) from 315 to 242 us, of 39,993 atoms (80^3) from 314 to 230 us.
+// Relative error of the potential against FP64 over 24 boxes a mesh (the
+// Stockham pass): 4.8e-7 (4.1e-7) on 24^3, 7.8e-7 (5.7e-7) on 40^3, 6.6e-7
+// (6.7e-7) on 80^3, 7.4e-7 (9.2e-7) on 120^3.
 // One direction is compiled: the inverse conjugates on the way in and out.
 // cos and sin of 2 pi k / R.
 template <int R> struct HmdRoots;

@@ -108,8 +108,10 @@ def test_replayed_steps_after_retuning(gpu_ctx):
 
 def test_fft_grid_is_tuned_only_where_it_shapes_a_pass(gpu_ctx):
     """On 24^3 every FFT pass has a shape of its own: the candidates are the
-    one at entry, five pair grids, the other stream setting and at most eight
-    bricks, and the value at entry stays."""
+    shapes at entry, five or six pair grids (the one at entry again, once
+    another has beaten it), the other stream setting and at most eight bricks;
+    five or six FFT grids more would make it 19 at least.  The value at entry
+    stays."""
     from heddlemd_amd import systems
     s = systems.spc_water_n(216, 3)
     ff = systems.water_forcefield(r_cut_nm=0.8, grid=(24, 24, 24), exclusions=s["exclusions"])
@@ -119,6 +121,6 @@ def test_fft_grid_is_tuned_only_where_it_shapes_a_pass(gpu_ctx):
         before = field.tuning()["fft_blocks_per_cu"]
         res = field.autotune(3)
         print(f"24^3: {res['n_candidates']} candidates")
-        assert res["n_candidates"] <= 15 and res["fft_blocks_per_cu"] == before
+        assert res["n_candidates"] <= 16 and res["fft_blocks_per_cu"] == before
     finally:
         field.close(); part.close()
